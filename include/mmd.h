@@ -173,11 +173,15 @@ int mmd_boys(mmd_ctx *ctx, int n, const double *m, const double *T, int table, d
  * for the context's basis and nuclei (mmd_set_atoms); P the half density
  * C_occ C_occ^T and W = P F P (N x N, host), bf_atom the atom of each basis
  * function (the reference's atom.mask, mmd/molecule.py:74-80).  The nuclear
- * repulsion term (forces.py:52-60) is the caller's.  grad: natom x 3, host.
+ * repulsion term (forces.py:52-60) is the caller's; mmd_rhf_total_gradient
+ * adds it for the nuclei given (natom x 4: charge, x, y, z).  grad: natom x 3,
+ * host.
  * One molecule per context; up to 4096 atoms.  mmd_last_gradient_ms: device
  * time of the last call (HIP events around its kernels).
  */
 int mmd_rhf_gradient(mmd_ctx *ctx, const double *P, const double *W, const int32_t *bf_atom, double *grad);
+int mmd_rhf_total_gradient(mmd_ctx *ctx, const double *P, const double *W, const int32_t *bf_atom,
+                           const double *nuclei, double *grad);
 int mmd_last_gradient_ms(mmd_ctx *ctx, double *ms);
 
 /*

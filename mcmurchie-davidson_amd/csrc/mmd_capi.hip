@@ -20,6 +20,7 @@
 #include "mmd_batch.h"
 #include "mmd_device.h"
 #include "mmd_gemm.h"
+#include "mmd_grad.h"
 #include "mmd_kernels.h"
 #include "mmd_scf.h"
 #include "mmd_types.h"
@@ -198,6 +199,16 @@ struct mmd_ctx {
     DevBuf<double> g_PW;                // gradient: P, W and the natom x 3 result
     DevBuf<int> g_atom;                 // gradient: atom of each basis function
     double last_grad_ms = 0.0;
+    // gradient by shell class: exponent of the first function of every
+    // primitive pair, the classes' bra slices (of grad_pslice primitive pairs,
+    // and of one for the wavefront kernels) and flat primitive-pair lists,
+    // made from the pair table on first use
+    std::vector<double> ppa;
+    DevBuf<double> d_ppa, g_rep;
+    DevBuf<int4> g_slices;
+    DevBuf<int2> g_flat;
+    int g_slice_off[NPAIRCLASS + 1] = {0}, g_one_off[NPAIRCLASS + 1] = {0}, g_flat_off[NPAIRCLASS + 1] = {0};
+    bool grad_plan_ok = false;
 
     // Molecules of a block-diagonal basis (mmd_set_molecules; one molecule
     // unless set): molecule m owns functions [mol_f0[m], mol_f0[m] + mol_n[m])
@@ -529,6 +540,8 @@ int build_pairs(mmd_ctx* c, const DiagView* diag)
             }
     std::vector<std::vector<ShellPair>> byclass(NPAIRCLASS);
     std::vector<PrimPair> pp;
+    c->ppa.clear();
+    c->grad_plan_ok = false;
     for (int m = 0; m < c->nmol; ++m)
         for (int I = c->mol_s0[m]; I < c->mol_s0[m + 1]; ++I)
             for (int J = c->mol_s0[m]; J <= I; ++J) {
@@ -582,6 +595,7 @@ int build_pairs(mmd_ctx* c, const DiagView* diag)
                         pq.inv2p = 0.5 / pq.p;
                         pq.invp = 1.0 / pq.p;
                         pp.push_back(pq);
+                        c->ppa.push_back(ea);
                     }
                 sp.npp = (int)pp.size() - sp.pp0;
                 if (sp.npp == 0) sp.q = 0.0;   // no primitive pair survives: never screened in
@@ -1289,7 +1303,141 @@ int mmd_set_molecules(mmd_ctx* ctx, int nmol, const int32_t* nbf_per_mol, const 
     return MMD_OK;
 }
 
-int mmd_rhf_gradient(mmd_ctx* ctx, const double* P, const double* W, const int32_t* bf_atom, double* grad)
+namespace {
+// Bra slices and flat ket lists of the gradient's class kernels, from the
+// pair table.
+int build_grad_plan(mmd_ctx* c)
+{
+    if (c->grad_plan_ok) return MMD_OK;
+    std::vector<int4> sl, one;
+    std::vector<int2> flat;
+    for (int pc = 0; pc < NPAIRCLASS; ++pc) {
+        c->g_slice_off[pc] = (int)sl.size();
+        c->g_one_off[pc] = (int)one.size();
+        c->g_flat_off[pc] = (int)flat.size();
+        // bra slices of grad_pslice primitive pairs, shorter where the whole
+        // molecule would not give the class some 1000 work units: a slice is
+        // a serial chain in every lane, and a small molecule leaves most of
+        // the GPU idle ((H2O) cc-pVDZ, (pp|pp): 133 us in 10 workgroups of 16)
+        int64_t prims = 0, kets = 0;
+        for (int P = 0; P < c->pc_off[pc + 1]; ++P) {
+            kets += c->pairs[P].npp;
+            if (P >= c->pc_off[pc]) prims += c->pairs[P].npp;
+        }
+        int step = grad_pslice(pc);
+        while (step > 1 && (prims / step) * (kets / 256 + 1) < 1024) step /= 2;
+        for (int P = c->pc_off[pc]; P < c->pc_off[pc + 1]; ++P) {
+            const int npp = c->pairs[P].npp;
+            for (int i = 0; i < npp; ++i) flat.push_back(make_int2(P, i));
+            const int end = (int)flat.size() - c->g_flat_off[pc];
+            for (int i = 0; i < npp; i += step) sl.push_back(make_int4(P, i, std::min(npp, i + step), end));
+            if (pc >= 4)   // (dp) and (dd): the bras of the wavefront classes
+                for (int i = 0; i < npp; ++i) one.push_back(make_int4(P, i, i + 1, end));
+        }
+    }
+    c->g_slice_off[NPAIRCLASS] = (int)sl.size();
+    c->g_one_off[NPAIRCLASS] = (int)one.size();
+    c->g_flat_off[NPAIRCLASS] = (int)flat.size();
+    for (int pc = 0; pc <= NPAIRCLASS; ++pc) c->g_one_off[pc] += (int)sl.size();
+    sl.insert(sl.end(), one.begin(), one.end());
+    HIP_TRY(c->g_slices.reserve(std::max<size_t>(1, sl.size())));
+    HIP_TRY(c->g_flat.reserve(std::max<size_t>(1, flat.size())));
+    HIP_TRY(c->d_ppa.reserve(std::max<size_t>(1, c->ppa.size())));
+    HIP_TRY(hipMemcpyAsync(c->g_slices.p, sl.data(), sizeof(int4) * sl.size(), hipMemcpyHostToDevice, c->st));
+    HIP_TRY(hipMemcpyAsync(c->g_flat.p, flat.data(), sizeof(int2) * flat.size(), hipMemcpyHostToDevice, c->st));
+    HIP_TRY(hipMemcpyAsync(c->d_ppa.p, c->ppa.data(), sizeof(double) * c->ppa.size(), hipMemcpyHostToDevice, c->st));
+    HIP_TRY(hipStreamSynchronize(c->st));
+    c->grad_plan_ok = true;
+    return MMD_OK;
+}
+
+// The gradient by shell class: the one-electron pair classes and the 21
+// quartet classes, spread over the context's streams by their work.
+int gradient_shells(mmd_ctx* c, const double* dP, const double* dW, const double* nuc, double* dg)
+{
+    int rc;
+    if (!c->pairs_ok && (rc = build_pairs(c, nullptr))) return rc;
+    if ((rc = onee_pair_list(c))) return rc;
+    if ((rc = build_grad_plan(c))) return rc;
+    const size_t nrep = (size_t)GRAD_REPLICAS * 3 * c->natom;
+    HIP_TRY(c->g_rep.reserve(nrep));
+    HIP_TRY(launch_fill(nrep, c->g_rep.p, 0.0, c->st));
+    GradArgs A;
+    A.pairs = c->d_pairs.p;
+    A.pp = c->d_pp.p;
+    A.ppa = c->d_ppa.p;
+    A.boys = c->d_boys.p;
+    A.gcomp = c->d_gcomp.p;
+    A.P = dP;
+    A.bf_atom = c->g_atom.p;
+    A.grad = c->g_rep.p;
+    A.N = c->nbf;
+    A.natom = c->natom;
+    A.lds_atoms = c->natom <= 256 ? 1 : 0;   // 6 KB of LDS at most beside the class's own
+    struct Task {
+        double cost;
+        int kind, id;   // kind 0: quartet class id; 1: one-electron pair class id
+    };
+    std::vector<Task> tasks;
+    GradClass cls[NQCLASS];
+    for (int qc = 0; qc < NQCLASS; ++qc) {
+        int pcb, pck, la, lb, lc, ld;
+        class_of(qc, &pcb, &pck);
+        qclass_decode(qc, &la, &lb, &lc, &ld);
+        const bool wave = fock_class_is_mfma(la, lb, lc, ld);
+        const int* off = wave ? c->g_one_off : c->g_slice_off;
+        GradClass& C = cls[qc];
+        C.slices = c->g_slices.p + off[pcb];
+        C.nslice = off[pcb + 1] - off[pcb];
+        C.flat = c->g_flat.p + c->g_flat_off[pck];
+        C.nflat = c->g_flat_off[pck + 1] - c->g_flat_off[pck];
+        C.nkc = (C.nflat + 255) / 256;
+        C.tri = pcb == pck ? 1 : 0;
+        if (C.nslice == 0 || C.nflat == 0) continue;
+        const double prims = (double)(c->g_flat_off[pcb + 1] - c->g_flat_off[pcb]) * C.nflat * (C.tri ? 0.5 : 1.0);
+        const double work = 100.0 + nherm(la + lb + lc + ld + 1) * 6.0
+                          + 3.0 * ncart(la) * ncart(lb) * nherm(la + lb) * nherm(lc + ld);
+        tasks.push_back({prims * work + 1e6, 0, qc});   // 1e6: a launch's fixed latency
+    }
+    OneeArgs O = onee_args(c);
+    for (int pc = 0; pc < NPAIRCLASS; ++pc)
+        if (c->onee_off[pc + 1] > c->onee_off[pc])
+            tasks.push_back({1e6 + 1e4 * (c->onee_off[pc + 1] - c->onee_off[pc]), 1, pc});
+    std::sort(tasks.begin(), tasks.end(), [](const Task& x, const Task& y) { return x.cost > y.cost; });
+    hipStream_t streams[1 + mmd_ctx::NSIDE] = {c->st};
+    for (int i = 0; i < mmd_ctx::NSIDE; ++i) streams[1 + i] = c->side[i];
+    double load[1 + mmd_ctx::NSIDE] = {0};
+    bool used[1 + mmd_ctx::NSIDE] = {true};
+    HIP_TRY(hipEventRecord(c->evfork, c->st));
+    for (const Task& t : tasks) {
+        int si = 0;
+        for (int i = 1; i < c->nstreams; ++i)
+            if (load[i] < load[si]) si = i;
+        load[si] += t.cost;
+        hipStream_t sq = streams[si];
+        if (!used[si]) {
+            HIP_TRY(hipStreamWaitEvent(sq, c->evfork, 0));
+            used[si] = true;
+        }
+        if (t.kind == 0)
+            HIP_TRY(launch_grad_class(t.id, A, cls[t.id], sq));
+        else
+            HIP_TRY(launch_grad_onee(t.id, O, c->d_onee_list.p + c->onee_off[t.id],
+                                     c->onee_off[t.id + 1] - c->onee_off[t.id], c->g_atom.p, dP, dW, c->g_rep.p, sq));
+    }
+    for (int i = 1; i < c->nstreams; ++i) {
+        if (!used[i]) continue;
+        HIP_TRY(hipEventRecord(c->evjoin[i - 1], streams[i]));
+        HIP_TRY(hipStreamWaitEvent(c->st, c->evjoin[i - 1], 0));
+    }
+    HIP_TRY(launch_grad_sum(c->natom, GRAD_REPLICAS, c->g_rep.p, nuc, dg, c->st));
+    return MMD_OK;
+}
+}  // namespace
+
+namespace {
+int rhf_gradient(mmd_ctx* ctx, const double* P, const double* W, const int32_t* bf_atom, const double* nuc,
+                 double* grad)
 {
     int rc = check_ctx(ctx);
     if (rc) return rc;
@@ -1302,18 +1450,31 @@ int mmd_rhf_gradient(mmd_ctx* ctx, const double* P, const double* W, const int32
     for (int i = 0; i < N; ++i)
         if (bf_atom[i] < 0 || bf_atom[i] >= natom) return fail(MMD_ERR_ARG, "basis function %d: atom out of range", i);
     const size_t nn = (size_t)N * N;
-    HIP_TRY(ctx->g_PW.reserve(2 * nn + 3 * (size_t)natom));
+    HIP_TRY(ctx->g_PW.reserve(2 * nn + 7 * (size_t)natom));
     HIP_TRY(ctx->g_atom.reserve(N));
     double* dP = ctx->g_PW.p;
     double* dW = dP + nn;
     double* dg = dW + nn;
+    double* dn = nuc ? dg + 3 * (size_t)natom : nullptr;
     HIP_TRY(hipMemcpyAsync(dP, P, sizeof(double) * nn, hipMemcpyHostToDevice, ctx->st));
     HIP_TRY(hipMemcpyAsync(dW, W, sizeof(double) * nn, hipMemcpyHostToDevice, ctx->st));
     HIP_TRY(hipMemcpyAsync(ctx->g_atom.p, bf_atom, sizeof(int32_t) * N, hipMemcpyHostToDevice, ctx->st));
-    HIP_TRY(launch_fill(3 * (size_t)natom, dg, 0.0, ctx->st));
+    if (nuc) HIP_TRY(hipMemcpyAsync(dn, nuc, sizeof(double) * 4 * natom, hipMemcpyHostToDevice, ctx->st));
+    // whole shells, each on one atom: the shell-class kernels; else the
+    // per-function kernels
+    bool shells = ctx->shells_ok;
+    for (size_t k = 0; k < ctx->shells.size() && shells; ++k)
+        for (int i = 1; i < ncart(ctx->shells[k].l); ++i)
+            shells = shells && bf_atom[ctx->shells[k].bf0 + i] == bf_atom[ctx->shells[k].bf0];
     HIP_TRY(hipEventRecord(ctx->ev0, ctx->st));
-    HIP_TRY(launch_rhf_gradient(N, ctx->d_bf.p, ctx->d_bf_exp.p, ctx->d_bf_w.p, natom, ctx->d_atoms.p, ctx->d_boys.p,
-                                ctx->g_atom.p, dP, dW, dg, ctx->st));
+    if (shells) {
+        if ((rc = gradient_shells(ctx, dP, dW, dn, dg))) return rc;
+    } else {
+        HIP_TRY(launch_fill(3 * (size_t)natom, dg, 0.0, ctx->st));
+        HIP_TRY(launch_rhf_gradient(N, ctx->d_bf.p, ctx->d_bf_exp.p, ctx->d_bf_w.p, natom, ctx->d_atoms.p,
+                                    ctx->d_boys.p, ctx->g_atom.p, dP, dW, dg, ctx->st));
+        if (dn) HIP_TRY(launch_grad_sum(natom, 1, dg, dn, dg, ctx->st));
+    }
     HIP_TRY(hipEventRecord(ctx->ev1, ctx->st));
     HIP_TRY(hipMemcpyAsync(grad, dg, sizeof(double) * 3 * natom, hipMemcpyDeviceToHost, ctx->st));
     HIP_TRY(hipStreamSynchronize(ctx->st));
@@ -1321,6 +1482,20 @@ int mmd_rhf_gradient(mmd_ctx* ctx, const double* P, const double* W, const int32
     HIP_TRY(hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
     ctx->last_grad_ms = ms;
     return MMD_OK;
+}
+
+}  // namespace
+
+int mmd_rhf_gradient(mmd_ctx* ctx, const double* P, const double* W, const int32_t* bf_atom, double* grad)
+{
+    return rhf_gradient(ctx, P, W, bf_atom, nullptr, grad);
+}
+
+int mmd_rhf_total_gradient(mmd_ctx* ctx, const double* P, const double* W, const int32_t* bf_atom,
+                           const double* nuclei, double* grad)
+{
+    if (!nuclei) return fail(MMD_ERR_ARG, "null pointer");
+    return rhf_gradient(ctx, P, W, bf_atom, nuclei, grad);
 }
 
 int mmd_last_gradient_ms(mmd_ctx* ctx, double* ms)

@@ -14,9 +14,14 @@
 // or 2b E^{i,j+1}_t - j E^{i,j-1}_t (second centre), cython/grad.pyx:97-103.
 // The fourth centre of an ERI follows from translational invariance,
 // d/dD = -(d/dA + d/dB + d/dC).
+//
+// Bases of whole shells take the kernels by shell class (the pair kernels
+// below and mmd_grad_class.h); the per-function kernels with runtime angular
+// momenta, whose tables lie in scratch, serve the other bases.
 #include <hip/hip_runtime.h>
 #include <algorithm>
 #include "mmd_device.h"
+#include "mmd_grad.h"
 #include "mmd_kernels.h"
 
 namespace mmd {
@@ -324,7 +329,271 @@ __global__ void __launch_bounds__(256) grad_one_electron_kernel(int nbf, const B
     }
 }
 
+// ---------------------------------------------------------------------------
+// One-electron part by shell pair, compile-time pair classes: one wavefront
+// per pair (a, b), l_a >= l_b; a lane item is a primitive pair with every
+// G-th nucleus.  With w_ab = 2 P_ab times the pair's degeneracy, the pair's
+// weights enter the Hermite space first, D_k = sum_ab w_ab E^{ab}_k and
+// DR_x,k = sum_ab w_ab dE^{ab}_k/dR_x (R = A - B), so that a nucleus costs
+// one R_tuv table of order l_a + l_b + 1 and 6 H(l_a + l_b) products:
+//   d/dP = sum_k D_k R_{k+x},  A: (a/p) d/dP + d/dR,  B: (b/p) d/dP - d/dR,
+//   the nucleus: -d/dP.
+// Overlap and kinetic energy need 1-D overlaps only, and d/dB = -d/dA.
+// Bound by FP64 latency; the per-function kernel, its tables in scratch,
+// took 1182 us at (H2O)4 6-31G.
+// ---------------------------------------------------------------------------
+template <int LA, int LB>
+__global__ void __launch_bounds__(256) grad_onee_pair_kernel(OneeArgs A, const int2* __restrict__ list, int npairs,
+                                                             const int* __restrict__ bf_atom,
+                                                             const double* __restrict__ P,
+                                                             const double* __restrict__ W, double* grad)
+{
+    constexpr int NA = ncart(LA), NB = ncart(LB), NAB = NA * NB, L = LA + LB, H = nherm(L), NT = L + 2;
+    const int wid = (int)(((size_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6);
+    const int lane = threadIdx.x & 63;
+    if (wid >= npairs) return;   // uniform across the wavefront
+    double* g = grad + (size_t)(wid % GRAD_REPLICAS) * 3 * A.natom;
+    const int2 pr = list[wid];
+    const OneeShell a = A.shells[pr.x], b = A.shells[pr.y];
+    const double Ac[3] = {a.x, a.y, a.z}, Bc[3] = {b.x, b.y, b.z};
+    const double AB2 = (a.x - b.x) * (a.x - b.x) + (a.y - b.y) * (a.y - b.y) + (a.z - b.z) * (a.z - b.z);
+    const double deg = pr.x == pr.y ? 1.0 : 2.0;
+    const size_t n = (size_t)A.nbf;
+    const int npp = a.np * b.np;
+    int G = npp >= 64 ? 1 : 64 / npp;
+    if (G > A.natom) G = A.natom;
+    // weight of component pair (ca, cb) in M (the lower triangle counts)
+    auto wgt = [&](const double* __restrict__ M, int ca, int cb) {
+        const size_t i = (size_t)a.bf0 + ca, j = (size_t)b.bf0 + cb;
+        return 2.0 * deg * A.gcomp[i] * A.gcomp[j] * M[(i > j ? i : j) * n + (i > j ? j : i)];
+    };
+    double gA[3] = {0, 0, 0}, gB[3] = {0, 0, 0};
+    for (int it = lane; it < npp * G; it += 64) {
+        const int ipp = it % npp, grp = it / npp;
+        const int ia = ipp / b.np, ib = ipp - ia * b.np;
+        const double ea = A.exps[a.p0 + ia], eb = A.exps[b.p0 + ib];
+        const double p = ea + eb, ip = 1.0 / p;
+        const double w = A.wts[a.p0 + ia] * A.wts[b.p0 + ib] * exp(-ea * eb * ip * AB2);
+        const double Pc[3] = {(ea * a.x + eb * b.x) * ip, (ea * a.y + eb * b.y) * ip, (ea * a.z + eb * b.z) * ip};
+        if (grp == 0) {
+            // overlap and kinetic energy (cython/grad.pyx:352-507) from the 1-D
+            // overlaps s_ij = E^{ij}_0: s_{i+1,j} = PA s_ij + (i s_{i-1,j} + j s_{i,j-1}) / 2p
+            constexpr int SJ = LB + 3;
+            double s[3][(LA + 2) * SJ];
+            const double h = 0.5 * ip;
+            sfor<3>([&](auto xx) {
+                constexpr int x = decltype(xx)::value;
+                const double pa = Pc[x] - Ac[x], pb = Pc[x] - Bc[x];
+                s[x][0] = 1.0;
+                sfor<SJ - 1>([&](auto jj) {
+                    constexpr int j = decltype(jj)::value;
+                    double v = pb * s[x][j];
+                    if constexpr (j > 0) v = fma((double)j * h, s[x][j - 1], v);
+                    s[x][j + 1] = v;
+                });
+                sfor<LA + 1>([&](auto ii) {
+                    sfor<SJ>([&](auto jj) {
+                        constexpr int i = decltype(ii)::value, j = decltype(jj)::value;
+                        double v = pa * s[x][i * SJ + j];
+                        if constexpr (i > 0) v = fma((double)i * h, s[x][(i - 1) * SJ + j], v);
+                        if constexpr (j > 0) v = fma((double)j * h, s[x][i * SJ + j - 1], v);
+                        s[x][(i + 1) * SJ + j] = v;
+                    });
+                });
+            });
+            const double pre = 3.141592653589793238462643383279 * ip * sqrt(3.141592653589793238462643383279 * ip) * w;
+            sfor<NAB>([&](auto kk) {
+                constexpr int k = decltype(kk)::value, ca = k / NB, cb = k % NB;
+                constexpr int li[3] = {comp_lx(LA, ca), comp_ly(LA, ca), comp_lz(LA, ca)};
+                constexpr int lj[3] = {comp_lx(LB, cb), comp_ly(LB, cb), comp_lz(LB, cb)};
+                const double wp = wgt(P, ca, cb) * pre, ws = wgt(W, ca, cb) * pre;
+                double S0[3], S1[3], T0[3], T1[3];   // plain and d/dA
+                sfor<3>([&](auto xx) {
+                    constexpr int x = decltype(xx)::value, i = li[x], j = lj[x];
+                    auto kin = [&](auto i_) {   // (2j+1) b s_ij - 2 b^2 s_{i,j+2} - j (j-1)/2 s_{i,j-2}
+                        constexpr int q = decltype(i_)::value;
+                        double v = (2.0 * j + 1.0) * eb * s[x][q * SJ + j] - 2.0 * eb * eb * s[x][q * SJ + j + 2];
+                        if constexpr (j >= 2) v -= 0.5 * j * (j - 1.0) * s[x][q * SJ + j - 2];
+                        return v;
+                    };
+                    S0[x] = s[x][i * SJ + j];
+                    T0[x] = kin(std::integral_constant<int, i>{});
+                    S1[x] = 2.0 * ea * s[x][(i + 1) * SJ + j];
+                    T1[x] = 2.0 * ea * kin(std::integral_constant<int, i + 1>{});
+                    if constexpr (i > 0) {
+                        S1[x] -= (double)i * s[x][(i - 1) * SJ + j];
+                        T1[x] -= (double)i * kin(std::integral_constant<int, i - 1>{});
+                    }
+                });
+                sfor<3>([&](auto xx) {
+                    constexpr int x = decltype(xx)::value, y = (x + 1) % 3, z = (x + 2) % 3;
+                    const double dt = T1[x] * S0[y] * S0[z] + S1[x] * (T0[y] * S0[z] + S0[y] * T0[z]);
+                    const double v = wp * dt - ws * S1[x] * S0[y] * S0[z];
+                    gA[x] += v;
+                    gB[x] -= v;
+                });
+            });
+        }
+        // nuclear attraction (cython/grad.pyx:509-)
+        double D[H], DR[3][H];
+        {
+            double e0[3][(LA + 1) * (LB + 1) * (L + 1)], e1[3][(LA + 1) * (LB + 1) * (L + 1)];
+            sfor<3>([&](auto xx) {
+                constexpr int x = decltype(xx)::value;
+                double E[(LA + 2) * (LB + 1) * NT];
+                hermite_E<LA + 1, LB, 1>(0.5 * ip, Pc[x] - Ac[x], Pc[x] - Bc[x], E);
+                sfor<LA + 1>([&](auto ii) {
+                    sfor<LB + 1>([&](auto jj) {
+                        constexpr int i = decltype(ii)::value, j = decltype(jj)::value;
+                        sfor<i + j + 1>([&](auto tt) {
+                            constexpr int t = decltype(tt)::value;
+                            auto e = [&](int i_, int k) { return E[(i_ * (LB + 1) + j) * NT + k]; };
+                            double dv = 2.0 * ea * e(i + 1, t);
+                            if constexpr (i > 0) dv -= (double)i * e(i - 1, t);
+                            if constexpr (t > 0) dv -= ea * ip * e(i, t - 1);
+                            e0[x][(i * (LB + 1) + j) * (L + 1) + t] = e(i, t);
+                            e1[x][(i * (LB + 1) + j) * (L + 1) + t] = dv;
+                        });
+                    });
+                });
+            });
+            sfor<H>([&](auto k) { D[k] = DR[0][k] = DR[1][k] = DR[2][k] = 0.0; });
+            sfor<NAB>([&](auto kk) {
+                constexpr int k = decltype(kk)::value, ca = k / NB, cb = k % NB;
+                constexpr int ix = comp_lx(LA, ca), iy = comp_ly(LA, ca), iz = comp_lz(LA, ca);
+                constexpr int jx = comp_lx(LB, cb), jy = comp_ly(LB, cb), jz = comp_lz(LB, cb);
+                constexpr int ox = (ix * (LB + 1) + jx) * (L + 1), oy = (iy * (LB + 1) + jy) * (L + 1),
+                              oz = (iz * (LB + 1) + jz) * (L + 1);
+                const double wp = wgt(P, ca, cb);
+                sfor<ix + jx + 1>([&](auto t_) {
+                    constexpr int t = decltype(t_)::value;
+                    sfor<iy + jy + 1>([&](auto u_) {
+                        constexpr int u = decltype(u_)::value;
+                        sfor<iz + jz + 1>([&](auto v_) {
+                            constexpr int v = decltype(v_)::value, m = hidx(t, u, v);
+                            const double x0 = wp * e0[0][ox + t], yz = e0[1][oy + u] * e0[2][oz + v];
+                            D[m] = fma(x0, yz, D[m]);
+                            DR[0][m] = fma(wp * e1[0][ox + t], yz, DR[0][m]);
+                            DR[1][m] = fma(x0 * e1[1][oy + u], e0[2][oz + v], DR[1][m]);
+                            DR[2][m] = fma(x0 * e0[1][oy + u], e1[2][oz + v], DR[2][m]);
+                        });
+                    });
+                });
+            });
+        }
+        const double vpre = -2.0 * 3.141592653589793238462643383279 * ip * w;
+        for (int at = grp; at < A.natom; at += G) {
+            const double* nuc = A.atoms + 4 * (size_t)at;
+            const double X = Pc[0] - nuc[1], Y = Pc[1] - nuc[2], Z = Pc[2] - nuc[3];
+            double F[L + 2];
+            boys_seeds<L + 1, double>(p * (X * X + Y * Y + Z * Z), p, nuc[0] * vpre, A.boys + (size_t)(L + 1) * BOYS_NT,
+                                      F);
+            double R[nherm(L + 1)];
+            hermite_R<L + 1, double>(X, Y, Z, F, R);
+            double gP[3] = {0, 0, 0}, gR[3] = {0, 0, 0};
+            sfor<H>([&](auto kk) {
+                constexpr int k = decltype(kk)::value;
+                constexpr Herm3 h = hdecode(k);
+                gP[0] = fma(D[k], R[hidx(h.t + 1, h.u, h.v)], gP[0]);
+                gP[1] = fma(D[k], R[hidx(h.t, h.u + 1, h.v)], gP[1]);
+                gP[2] = fma(D[k], R[hidx(h.t, h.u, h.v + 1)], gP[2]);
+                sfor<3>([&](auto x) { gR[x] = fma(DR[x][k], R[k], gR[x]); });
+            });
+            sfor<3>([&](auto x) {
+                gA[x] += fma(ea * ip, gP[x], gR[x]);
+                gB[x] += fma(eb * ip, gP[x], -gR[x]);
+                atomicAdd(&g[3 * at + x], -gP[x]);
+            });
+        }
+    }
+    for (int off = 32; off > 0; off >>= 1)
+        sfor<3>([&](auto x) {
+            gA[x] += __shfl_xor(gA[x], off);
+            gB[x] += __shfl_xor(gB[x], off);
+        });
+    if (lane != 0) return;
+    const int ta = bf_atom[a.bf0], tb = bf_atom[b.bf0];
+    sfor<3>([&](auto x) {
+        atomicAdd(&g[3 * ta + x], gA[x]);
+        atomicAdd(&g[3 * tb + x], gB[x]);
+    });
+}
+
+// out[3a + x] = sum of the replicas, plus the nuclear repulsion term
+// -sum_b Z_a Z_b (r_a - r_b)_x / R^3 (mmd/forces.py:52-60; coinciding nuclei
+// are left out as there) when nuc is given
+__global__ void grad_sum_kernel(int natom, int nrep, const double* __restrict__ rep, const double* __restrict__ nuc,
+                                double* __restrict__ out)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x, n = 3 * natom;
+    if (i >= n) return;
+    double s = 0.0;
+    for (int r = 0; r < nrep; ++r) s += rep[(size_t)r * n + i];
+    if (nuc) {
+        const int a = i / 3, x = i - 3 * a;
+        double v = 0.0;
+        for (int b = 0; b < natom; ++b) {
+            const double dx = nuc[4 * a + 1] - nuc[4 * b + 1], dy = nuc[4 * a + 2] - nuc[4 * b + 2],
+                         dz = nuc[4 * a + 3] - nuc[4 * b + 3];
+            const double r2 = dx * dx + dy * dy + dz * dz, r = sqrt(r2);
+            if (r <= 1e-8) continue;
+            v -= (x == 0 ? dx : (x == 1 ? dy : dz)) * nuc[4 * a] * nuc[4 * b] / (r2 * r);
+        }
+        s += v;
+    }
+    out[i] = s;
+}
+
+template <int LA, int LB>
+hipError_t launch_grad_onee_pc(const OneeArgs& A, const int2* list, int n, const int* bf_atom, const double* P,
+                               const double* W, double* grad, hipStream_t st)
+{
+    if (n <= 0) return hipSuccess;
+    hipLaunchKernelGGL((grad_onee_pair_kernel<LA, LB>), dim3((unsigned)((n + 3) / 4)), dim3(256), 0, st, A, list, n,
+                       bf_atom, P, W, grad);
+    return hipGetLastError();
+}
+
 }  // namespace
+
+#define MMD_GRAD_CLASSES(X)                                                                              \
+    X(0, 0, 0, 0) X(1, 0, 0, 0) X(1, 0, 1, 0) X(1, 1, 0, 0) X(1, 1, 1, 0) X(1, 1, 1, 1) X(2, 0, 0, 0)   \
+    X(2, 0, 1, 0) X(2, 0, 1, 1) X(2, 0, 2, 0) X(2, 1, 0, 0) X(2, 1, 1, 0) X(2, 1, 1, 1) X(2, 1, 2, 0)   \
+    X(2, 1, 2, 1) X(2, 2, 0, 0) X(2, 2, 1, 0) X(2, 2, 1, 1) X(2, 2, 2, 0) X(2, 2, 2, 1) X(2, 2, 2, 2)
+#define DECL(a, b, c, d) \
+    hipError_t grad_class_launch_##a##b##c##d(const GradArgs& A, const GradClass& C, hipStream_t st);
+MMD_GRAD_CLASSES(DECL)
+#undef DECL
+
+hipError_t launch_grad_class(int qc, const GradArgs& A, const GradClass& C, hipStream_t st)
+{
+    int la, lb, lc, ld;
+    qclass_decode(qc, &la, &lb, &lc, &ld);
+#define CASE(a, b, c, d) \
+    if (la == a && lb == b && lc == c && ld == d) return grad_class_launch_##a##b##c##d(A, C, st);
+    MMD_GRAD_CLASSES(CASE)
+#undef CASE
+    return hipErrorInvalidValue;
+}
+
+hipError_t launch_grad_onee(int pc, const OneeArgs& A, const int2* list, int n, const int* bf_atom, const double* P,
+                            const double* W, double* grad, hipStream_t st)
+{
+    switch (pc) {
+    case 0: return launch_grad_onee_pc<0, 0>(A, list, n, bf_atom, P, W, grad, st);
+    case 1: return launch_grad_onee_pc<1, 0>(A, list, n, bf_atom, P, W, grad, st);
+    case 2: return launch_grad_onee_pc<1, 1>(A, list, n, bf_atom, P, W, grad, st);
+    case 3: return launch_grad_onee_pc<2, 0>(A, list, n, bf_atom, P, W, grad, st);
+    case 4: return launch_grad_onee_pc<2, 1>(A, list, n, bf_atom, P, W, grad, st);
+    default: return launch_grad_onee_pc<2, 2>(A, list, n, bf_atom, P, W, grad, st);
+    }
+}
+
+hipError_t launch_grad_sum(int natom, int nrep, const double* rep, const double* nuc, double* grad, hipStream_t st)
+{
+    hipLaunchKernelGGL(grad_sum_kernel, dim3((3 * natom + 63) / 64), dim3(64), 0, st, natom, nrep, rep, nuc, grad);
+    return hipGetLastError();
+}
 
 hipError_t launch_rhf_gradient(int nbf, const BFDesc* bfs, const double* pexp, const double* pw, int natom,
                                const double* atoms, const double* boys, const int* bf_atom, const double* P,

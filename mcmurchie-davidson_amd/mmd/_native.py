@@ -90,6 +90,8 @@ lib.mmd_set_ket_slices.restype = _c_int
 lib.mmd_set_ket_slices.argtypes = [_ctx_p, _vp, _vp]
 lib.mmd_rhf_gradient.restype = _c_int
 lib.mmd_rhf_gradient.argtypes = [_ctx_p, _vp, _vp, _vp, _vp]
+lib.mmd_rhf_total_gradient.restype = _c_int
+lib.mmd_rhf_total_gradient.argtypes = [_ctx_p, _vp, _vp, _vp, _vp, _vp]
 lib.mmd_last_gradient_ms.restype = _c_int
 lib.mmd_last_gradient_ms.argtypes = [_ctx_p, _vp]
 lib.mmd_fock_profile_sums.restype = _c_int
@@ -135,7 +137,8 @@ EXPORTED = [
     "mmd_last_error", "mmd_version", "mmd_device_count", "mmd_ctx_create", "mmd_ctx_destroy",
     "mmd_set_basis", "mmd_set_atoms", "mmd_one_electron", "mmd_schwarz", "mmd_set_schwarz",
     "mmd_eri_tensor", "mmd_eri_list", "mmd_fock_delta", "mmd_fock_delta_noalloc", "mmd_jk_tensor", "mmd_boys",
-    "mmd_last_fock_ms", "mmd_set_profiling", "mmd_fock_stats", "mmd_fock_profile_sums", "mmd_rhf_gradient", "mmd_set_class_impl", "mmd_set_ket_slices",
+    "mmd_last_fock_ms", "mmd_set_profiling", "mmd_fock_stats", "mmd_fock_profile_sums", "mmd_rhf_gradient", "mmd_rhf_total_gradient",
+    "mmd_set_class_impl", "mmd_set_ket_slices",
     "mmd_last_gradient_ms", "mmd_set_precision", "mmd_fock_tiers",
     "mmd_set_streams", "mmd_set_lds_limit", "mmd_overlap_powers", "mmd_dgemm", "mmd_set_molecules",
     "mmd_batch_rhf", "mmd_scf_begin", "mmd_scf_step", "mmd_scf_density", "mmd_scf_get", "mmd_ao2mo",
@@ -381,9 +384,10 @@ class Context:
         check(lib.mmd_set_ket_slices(self._h, None if src is None else _ptr(src), _ptr(cur)))
         return cur
 
-    def rhf_gradient(self, P, W, bf_atom):
+    def rhf_gradient(self, P, W, bf_atom, nuclei=None):
         """Electronic part of the RHF nuclear gradient (natom, 3) for the
-        half density P, W = P F P and the atom of each basis function."""
+        half density P, W = P F P and the atom of each basis function; with
+        nuclei (natom rows of charge, x, y, z), the nuclear repulsion's too."""
         N = self.nbf
         P = np.ascontiguousarray(np.real(P), dtype=np.float64)
         W = np.ascontiguousarray(np.real(W), dtype=np.float64)
@@ -391,7 +395,13 @@ class Context:
         if P.shape != (N, N) or W.shape != (N, N) or at.shape != (N,):
             raise ValueError("P and W must be N x N and bf_atom of length N")
         g = np.zeros(3 * self.natom)
-        check(lib.mmd_rhf_gradient(self._h, _ptr(P), _ptr(W), _ptr(at), _ptr(g)))
+        if nuclei is None:
+            check(lib.mmd_rhf_gradient(self._h, _ptr(P), _ptr(W), _ptr(at), _ptr(g)))
+        else:
+            nuc = _f64(nuclei)
+            if nuc.shape != (self.natom, 4):
+                raise ValueError("nuclei must be natom x 4")
+            check(lib.mmd_rhf_total_gradient(self._h, _ptr(P), _ptr(W), _ptr(at), _ptr(nuc), _ptr(g)))
         return g.reshape(-1, 3)
 
     def last_gradient_ms(self):

@@ -8,9 +8,8 @@ them.  The electronic part
     sum_pq P_pq 2 dH_pq/dX + sum_pqrs Gamma_pqrs d(pq|rs)/dX - 2 sum_pq W_pq dS_pq/dX
 
 (P = C_occ C_occ^T, W = P F P, Gamma the density products of
-forces.py:62-84) comes from libmmd's mmd_rhf_gradient in one pass over all
-atoms and directions; the nuclear repulsion term is added here
-(forces.py:52-60).
+forces.py:62-84) and the nuclear repulsion term (forces.py:52-60) come from
+libmmd's mmd_rhf_total_gradient in one pass over all atoms and directions.
 """
 import numpy as np
 
@@ -45,7 +44,8 @@ class Forces(object):
         P = np.real(self.P)
         W = P @ np.real(self.F) @ P
         ctx = self.native
-        g = ctx.rhf_gradient(P, W, basis_atoms(self)) + nuclear_repulsion_gradient(self.atoms)
+        nuclei = [[atom.charge, *atom.origin] for atom in self.atoms]
+        g = ctx.rhf_gradient(P, W, basis_atoms(self), nuclei)
         self.gradient_ms = ctx.last_gradient_ms()
         for a, atom in enumerate(self.atoms):
             atom.forces = -g[a]
