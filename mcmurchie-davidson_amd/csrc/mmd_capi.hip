@@ -210,6 +210,12 @@ struct mmd_ctx {
     int g_slice_off[NPAIRCLASS + 1] = {0}, g_one_off[NPAIRCLASS + 1] = {0}, g_flat_off[NPAIRCLASS + 1] = {0};
     bool grad_plan_ok = false;
 
+    // integral-block kernels: staged bra data per pair class (made from the
+    // pair table on first use), copies of the raw G
+    DevBuf<double> d_btab, d_graw;
+    size_t btab_off[NPAIRCLASS] = {0};
+    bool btab_ok = false;
+
     // Molecules of a block-diagonal basis (mmd_set_molecules; one molecule
     // unless set): molecule m owns functions [mol_f0[m], mol_f0[m] + mol_n[m])
     // and shells [mol_s0[m], mol_s0[m + 1]); pairs and quartets never mix
@@ -542,6 +548,7 @@ int build_pairs(mmd_ctx* c, const DiagView* diag)
     std::vector<PrimPair> pp;
     c->ppa.clear();
     c->grad_plan_ok = false;
+    c->btab_ok = false;
     for (int m = 0; m < c->nmol; ++m)
         for (int I = c->mol_s0[m]; I < c->mol_s0[m + 1]; ++I)
             for (int J = c->mol_s0[m]; J <= I; ++J) {
@@ -610,6 +617,15 @@ int build_pairs(mmd_ctx* c, const DiagView* diag)
                 if (x.npp != y.npp) return x.npp > y.npp;
                 return x.q > y.q;
             });
+        else   // no Schwarz factors yet: by contraction length, for the lanes' balance
+            std::stable_sort(v.begin(), v.end(), [](const ShellPair& x, const ShellPair& y) {
+                return x.mol != y.mol ? x.mol < y.mol : x.npp > y.npp;
+            });
+        int pos = 0;
+        for (ShellPair& sp : v) {
+            sp.pad = pos;
+            pos += sp.npp;
+        }
         c->pc_off[pc] = (int)c->pairs.size();
         c->kr_first[pc].assign(c->nmol, (int)v.size());
         c->kr_end[pc].assign(c->nmol, 0);
@@ -748,6 +764,40 @@ int grid_for(int64_t items)
     if (g < 1) g = 1;
     if (g > 2048) g = 2048;
     return (int)g;
+}
+
+// Independent launches spread over the context's streams, largest first and
+// each to the least loaded stream, between a fork from and a join to c->st.
+struct StreamTask {
+    double cost;
+    int id;
+};
+template <class F>
+int spread_tasks(mmd_ctx* c, std::vector<StreamTask>& tasks, F&& launch)
+{
+    std::sort(tasks.begin(), tasks.end(), [](const StreamTask& x, const StreamTask& y) { return x.cost > y.cost; });
+    hipStream_t streams[1 + mmd_ctx::NSIDE] = {c->st};
+    for (int i = 0; i < mmd_ctx::NSIDE; ++i) streams[1 + i] = c->side[i];
+    double load[1 + mmd_ctx::NSIDE] = {0};
+    bool used[1 + mmd_ctx::NSIDE] = {true};
+    HIP_TRY(hipEventRecord(c->evfork, c->st));
+    for (const StreamTask& t : tasks) {
+        int si = 0;
+        for (int i = 1; i < c->nstreams; ++i)
+            if (load[i] < load[si]) si = i;
+        load[si] += t.cost;
+        if (!used[si]) {
+            HIP_TRY(hipStreamWaitEvent(streams[si], c->evfork, 0));
+            used[si] = true;
+        }
+        HIP_TRY(launch(t.id, streams[si]));
+    }
+    for (int i = 1; i < c->nstreams; ++i) {
+        if (!used[i]) continue;
+        HIP_TRY(hipEventRecord(c->evjoin[i - 1], streams[i]));
+        HIP_TRY(hipStreamWaitEvent(c->st, c->evjoin[i - 1], 0));
+    }
+    return MMD_OK;
 }
 
 ClassArgs base_args(mmd_ctx* c)
@@ -1374,11 +1424,7 @@ int gradient_shells(mmd_ctx* c, const double* dP, const double* dW, const double
     A.N = c->nbf;
     A.natom = c->natom;
     A.lds_atoms = c->natom <= 256 ? 1 : 0;   // 6 KB of LDS at most beside the class's own
-    struct Task {
-        double cost;
-        int kind, id;   // kind 0: quartet class id; 1: one-electron pair class id
-    };
-    std::vector<Task> tasks;
+    std::vector<StreamTask> tasks;   // quartet classes, then (from NQCLASS) one-electron pair classes
     GradClass cls[NQCLASS];
     for (int qc = 0; qc < NQCLASS; ++qc) {
         int pcb, pck, la, lb, lc, ld;
@@ -1397,39 +1443,19 @@ int gradient_shells(mmd_ctx* c, const double* dP, const double* dW, const double
         const double prims = (double)(c->g_flat_off[pcb + 1] - c->g_flat_off[pcb]) * C.nflat * (C.tri ? 0.5 : 1.0);
         const double work = 100.0 + nherm(la + lb + lc + ld + 1) * 6.0
                           + 3.0 * ncart(la) * ncart(lb) * nherm(la + lb) * nherm(lc + ld);
-        tasks.push_back({prims * work + 1e6, 0, qc});   // 1e6: a launch's fixed latency
+        tasks.push_back({prims * work + 1e6, qc});   // 1e6: a launch's fixed latency
     }
     OneeArgs O = onee_args(c);
     for (int pc = 0; pc < NPAIRCLASS; ++pc)
         if (c->onee_off[pc + 1] > c->onee_off[pc])
-            tasks.push_back({1e6 + 1e4 * (c->onee_off[pc + 1] - c->onee_off[pc]), 1, pc});
-    std::sort(tasks.begin(), tasks.end(), [](const Task& x, const Task& y) { return x.cost > y.cost; });
-    hipStream_t streams[1 + mmd_ctx::NSIDE] = {c->st};
-    for (int i = 0; i < mmd_ctx::NSIDE; ++i) streams[1 + i] = c->side[i];
-    double load[1 + mmd_ctx::NSIDE] = {0};
-    bool used[1 + mmd_ctx::NSIDE] = {true};
-    HIP_TRY(hipEventRecord(c->evfork, c->st));
-    for (const Task& t : tasks) {
-        int si = 0;
-        for (int i = 1; i < c->nstreams; ++i)
-            if (load[i] < load[si]) si = i;
-        load[si] += t.cost;
-        hipStream_t sq = streams[si];
-        if (!used[si]) {
-            HIP_TRY(hipStreamWaitEvent(sq, c->evfork, 0));
-            used[si] = true;
-        }
-        if (t.kind == 0)
-            HIP_TRY(launch_grad_class(t.id, A, cls[t.id], sq));
-        else
-            HIP_TRY(launch_grad_onee(t.id, O, c->d_onee_list.p + c->onee_off[t.id],
-                                     c->onee_off[t.id + 1] - c->onee_off[t.id], c->g_atom.p, dP, dW, c->g_rep.p, sq));
-    }
-    for (int i = 1; i < c->nstreams; ++i) {
-        if (!used[i]) continue;
-        HIP_TRY(hipEventRecord(c->evjoin[i - 1], streams[i]));
-        HIP_TRY(hipStreamWaitEvent(c->st, c->evjoin[i - 1], 0));
-    }
+            tasks.push_back({1e6 + 1e4 * (c->onee_off[pc + 1] - c->onee_off[pc]), NQCLASS + pc});
+    rc = spread_tasks(c, tasks, [&](int id, hipStream_t sq) {
+        if (id < NQCLASS) return launch_grad_class(id, A, cls[id], sq);
+        const int pc = id - NQCLASS;
+        return launch_grad_onee(pc, O, c->d_onee_list.p + c->onee_off[pc], c->onee_off[pc + 1] - c->onee_off[pc],
+                                c->g_atom.p, dP, dW, c->g_rep.p, sq);
+    });
+    if (rc) return rc;
     HIP_TRY(launch_grad_sum(c->natom, GRAD_REPLICAS, c->g_rep.p, nuc, dg, c->st));
     return MMD_OK;
 }
@@ -1561,49 +1587,101 @@ int mmd_set_schwarz(mmd_ctx* ctx, const double* diag)
 }
 
 namespace {
-// The full (ij|kl) tensor from the shell-pair tables: every quartet class
-// with bra pair class >= ket pair class, all canonical shell quartets of it
-// (bra pair >= ket pair inside one pair class), every integral stored at its
-// eight index permutations.  Every element of dst is written.
-hipError_t eri_tensor_shells(mmd_ctx* c, double* dst)
+// Staged bra data of every pair class, from the pair table.
+int build_bra_tables(mmd_ctx* c)
 {
-    ClassArgs A = base_args(c);
-    A.G = dst;
-    size_t bps = 0;
-    for (int qc = 0; qc < NQCLASS; ++qc) bps = std::max(bps, (size_t)tensor_class_bps(qc));
-    DevBuf<double> table;
-    hipError_t e = table.reserve(std::max<size_t>(1, (size_t)c->npp_total * bps));
-    if (e != hipSuccess) return e;
+    if (c->btab_ok) return MMD_OK;
+    size_t total = 0;
+    for (int pc = 0; pc < NPAIRCLASS; ++pc) {
+        c->btab_off[pc] = total;
+        for (int P = c->pc_off[pc]; P < c->pc_off[pc + 1]; ++P)
+            total += (size_t)c->pairs[P].npp * bra_table_stride(pc);
+    }
+    HIP_TRY(c->d_btab.reserve(std::max<size_t>(1, total)));
+    for (int pc = 0; pc < NPAIRCLASS; ++pc)
+        HIP_TRY(launch_bra_table(pc, c->d_pairs.p, c->d_pp.p, c->pc_off[pc], c->pc_off[pc + 1] - c->pc_off[pc],
+                                 c->d_btab.p + c->btab_off[pc], c->st));
+    c->btab_ok = true;
+    return MMD_OK;
+}
+
+// Every quartet class on the integral-block kernels (the stored tensor, or a
+// raw build with the fields of `raw`), side by side on the context's streams.
+int run_block_classes(mmd_ctx* c, const ClassArgs& A, const BlockArgs& raw)
+{
+    if (int rc = build_bra_tables(c)) return rc;
+    std::vector<StreamTask> tasks;
+    BlockArgs cls[NQCLASS];
+    int64_t npp[NPAIRCLASS] = {0};
+    for (int pc = 0; pc < NPAIRCLASS; ++pc)
+        for (int P = c->pc_off[pc]; P < c->pc_off[pc + 1]; ++P) npp[pc] += c->pairs[P].npp;
     for (int qc = 0; qc < NQCLASS; ++qc) {
         int pcb, pck, la, lb, lc, ld;
         class_of(qc, &pcb, &pck);
         qclass_decode(qc, &la, &lb, &lc, &ld);
-        const int boff = c->pc_off[pcb], nb = c->pc_off[pcb + 1] - boff;
-        const int koff = c->pc_off[pck], nk = c->pc_off[pck + 1] - koff;
-        if (nb == 0 || nk == 0) continue;
-        const int tri = pcb == pck;
-        if (la == 2 && lb == 2 && lc == 2 && ld == 2) {   // (dd|dd): the wavefront tensor kernel
-            std::vector<int2> q;
-            q.reserve((size_t)nb * (nb + 1) / 2);
-            for (int P = 0; P < nb; ++P)
-                for (int Q = 0; Q <= P; ++Q) q.push_back(make_int2(boff + P, koff + Q));
-            const int n = (int)q.size();
-            e = c->d_surv.reserve(q.size());
-            if (e == hipSuccess) e = hipMemcpyAsync(c->d_surv.p, q.data(), sizeof(int2) * q.size(),
-                                                    hipMemcpyHostToDevice, c->st);
-            if (e == hipSuccess) e = hipMemcpyAsync(c->d_count.p + qc, &n, sizeof(int), hipMemcpyHostToDevice, c->st);
-            if (e == hipSuccess) e = hipStreamSynchronize(c->st);   // q and n leave scope
-            if (e != hipSuccess) return e;
-            ClassArgs W = A;
-            W.quart = c->d_surv.p;
-            W.count = c->d_count.p + qc;
-            e = launch_tensor_wave_class(W, n, c->st);
-        } else {
-            e = launch_tensor_class(qc, A, boff, nb, koff, nk, tri, table.p, dst, c->st);
-        }
-        if (e != hipSuccess) return e;
+        BlockArgs& B = cls[qc];
+        B = raw;
+        B.boff = c->pc_off[pcb];
+        B.nb = c->pc_off[pcb + 1] - B.boff;
+        B.koff = c->pc_off[pck];
+        B.nk = c->pc_off[pck + 1] - B.koff;
+        B.tri = pcb == pck ? 1 : 0;
+        B.table = c->d_btab.p + c->btab_off[pcb];
+        if (B.nb == 0 || B.nk == 0) continue;
+        // lanes per quartet from the classes' mean contraction lengths, at
+        // least four (the LDS blocks of a wavefront hold sixteen groups)
+        auto lg = [](int64_t n, int64_t pairs) { return n >= 3 * pairs ? 2 : (2 * n >= 3 * pairs ? 1 : 0); };
+        B.lgb = lg(npp[pcb], B.nb);
+        B.lgk = lg(npp[pck], B.nk);
+        if (B.lgb + B.lgk < 2) B.lgk = 2 - B.lgb;
+        const double prims = (double)npp[pcb] * npp[pck] * (B.tri ? 0.5 : 1.0);
+        tasks.push_back({1e6 + prims * (40.0 + 4.0 * nherm(la + lb + lc + ld)
+                                        + (double)ncart(la) * ncart(lb) * ncart(lc) * ncart(ld)), qc});
     }
-    return hipStreamSynchronize(c->st);   // before the table is freed
+    return spread_tasks(c, tasks, [&](int qc, hipStream_t sq) { return launch_block_class(qc, A, cls[qc], sq); });
+}
+
+// The full (ij|kl) tensor from the shell-pair tables: every quartet class
+// with bra pair class >= ket pair class, all canonical shell quartets of it
+// (bra pair >= ket pair inside one pair class), every integral stored at its
+// eight index permutations.  Every element of dst is written.
+int eri_tensor_shells(mmd_ctx* c, double* dst)
+{
+    ClassArgs A = base_args(c);
+    A.G = dst;
+    BlockArgs B;
+    memset(&B, 0, sizeof(B));
+    return run_block_classes(c, A, B);
+}
+
+// formPT's unsymmetrised G of the density difference in d_D (and d_Dim) with
+// |dP| in d_absD, into d_graw: the real matrix, then the imaginary one.
+int raw_fock_shells(mmd_ctx* c, bool complex_dP, double tol)
+{
+    const size_t nn = (size_t)c->nbf * c->nbf;
+    HIP_TRY(launch_shell_block_max_raw((int)c->shells.size(), c->d_sh_bf0.p, c->d_sh_nbf.p, c->nbf, c->d_absD.p,
+                                       c->d_Dsh.p, c->st));
+    // copies of G, so that the updates of a small matrix do not queue at the
+    // same addresses; 128 MB of them at most
+    const int nrep = (int)std::max<size_t>(1, std::min<size_t>(16, (size_t(8) << 20) / nn));
+    HIP_TRY(c->d_graw.reserve(nrep * 2 * nn));
+    HIP_TRY(launch_fill(nrep * 2 * nn, c->d_graw.p, 0.0, c->st));
+    ClassArgs A = base_args(c);
+    A.D = c->d_D.p;
+    A.absD = c->d_absD.p;
+    A.sqS = c->d_sqS.p;
+    A.tol = tol;
+    A.G = c->d_graw.p;
+    BlockArgs B;
+    memset(&B, 0, sizeof(B));
+    B.raw = 1;
+    B.nrep = nrep;
+    B.Dim = complex_dP ? c->d_Dim.p : nullptr;
+    B.Dsh = c->d_Dsh.p;
+    B.nshell = (int)c->shells.size();
+    if (int rc = run_block_classes(c, A, B)) return rc;
+    HIP_TRY(launch_sum_copies((complex_dP ? 2 : 1) * nn, nrep, 2 * nn, c->d_graw.p, c->d_graw.p, c->st));
+    return MMD_OK;
 }
 }  // namespace
 
@@ -1625,7 +1703,7 @@ int mmd_eri_tensor(mmd_ctx* ctx, double* out, int out_on_device)
             rc = build_pairs(ctx, nullptr);
             if (rc) return rc;
         }
-        HIP_TRY(eri_tensor_shells(ctx, dst));
+        if ((rc = eri_tensor_shells(ctx, dst))) return rc;
     } else {
         HIP_TRY(launch_canonical_quartets(0, ctx->nbf, ctx->d_bf.p, ctx->d_bf_exp.p, ctx->d_bf_w.p, ctx->d_boys.p,
                                           nullptr, nullptr, nullptr, 0.0, dst, ctx->st));
@@ -1693,7 +1771,11 @@ int mmd_fock_delta(mmd_ctx* ctx, const double* dP_re, const double* dP_im, doubl
         if (rc) return rc;
         HIP_TRY(launch_symmetrize(N, ctx->d_G.p, ctx->d_Gout.p, ctx->st));
         HIP_TRY(hipMemcpyAsync(G_re, ctx->d_Gout.p, sizeof(double) * nn, k_out, ctx->st));
-    } else {
+    } else if (ctx->pairs_ok && ctx->nmol == 1) {
+        if ((rc = raw_fock_shells(ctx, dP_im != nullptr, tol))) return rc;
+        HIP_TRY(hipMemcpyAsync(G_re, ctx->d_graw.p, sizeof(double) * nn, k_out, ctx->st));
+        if (dP_im) HIP_TRY(hipMemcpyAsync(G_im, ctx->d_graw.p + nn, sizeof(double) * nn, k_out, ctx->st));
+    } else {   // functions that do not form whole shells, or several molecules
         for (int part = 0; part < (dP_im ? 2 : 1); ++part) {
             HIP_TRY(launch_fill(nn, ctx->d_G.p, 0.0, ctx->st));
             HIP_TRY(launch_canonical_quartets(1, N, ctx->d_bf.p, ctx->d_bf_exp.p, ctx->d_bf_w.p, ctx->d_boys.p,

@@ -1,6 +1,7 @@
 // Dispatch table over the shell-quartet classes of the Fock-build kernel
 // (each compiled in its own objects from mmd_eri_class.hip, in FP64 and in
 // the FP32 tier).
+#include "mmd_eri_core.h"
 #include "mmd_kernels.h"
 
 namespace mmd {
@@ -18,35 +19,70 @@ namespace mmd {
 MMD_CLASSES(DECL)
 #undef DECL
 
-#define DECLT(a, b, c, d)                                                                                    \
-    hipError_t tensor_class_launch_##a##b##c##d##_d(const ClassArgs& A, int boff, int nb, int koff, int nk,  \
-                                                    int tri, double* table, double* out, hipStream_t st);    \
-    int tensor_class_bps_##a##b##c##d##_d();
-MMD_CLASSES(DECLT)
-#undef DECLT
-
-hipError_t launch_tensor_class(int qc, const ClassArgs& A, int boff, int nb, int koff, int nk, int tri,
-                               double* table, double* out, hipStream_t st)
+// Staged bra data of stage_bra for every primitive pair of a pair class, in
+// class order: table + (pair's position) * BPS.
+namespace {
+template <int LA, int LB>
+__global__ void __launch_bounds__(64) bra_table_kernel(const ShellPair* __restrict__ pairs,
+                                                       const PrimPair* __restrict__ pp, int boff, double* table)
 {
-    int la, lb, lc, ld;
-    qclass_decode(qc, &la, &lb, &lc, &ld);
-#define CASE(a, b, c, d)                          \
-    if (la == a && lb == b && lc == c && ld == d) \
-        return tensor_class_launch_##a##b##c##d##_d(A, boff, nb, koff, nk, tri, table, out, st);
-    MMD_CLASSES(CASE)
-#undef CASE
-    return hipErrorInvalidValue;
+    using S = ClassShape<LA, LB, 0, 0>;
+    const ShellPair bra = pairs[boff + blockIdx.x];
+    for (int idx = threadIdx.x; idx < 3 * bra.npp; idx += blockDim.x) {
+        const int ip = idx / 3, x = idx - 3 * ip;
+        const PrimPair* P = pp + bra.pp0 + ip;
+        double* b = table + (size_t)(bra.pad + ip) * S::BPS;
+        if (x == 0) {
+            b[0] = P->p;
+            b[1] = TWO_PI_2_5 * P->K * P->invp;
+            b[2] = P->Px;
+            b[3] = P->Py;
+            b[4] = P->Pz;
+        }
+        double E[S::EB];
+        hermite_E<LA, LB, 1>(P->inv2p, x == 0 ? P->PAx : (x == 1 ? P->PAy : P->PAz),
+                             x == 0 ? P->PBx : (x == 1 ? P->PBy : P->PBz), E);
+        sfor<S::EB>([&](auto k) { b[8 + x * S::EB + k] = E[k]; });
+    }
+}
+}  // namespace
+
+int bra_table_stride(int pc)
+{
+    constexpr int bps[NPAIRCLASS] = {ClassShape<0, 0, 0, 0>::BPS, ClassShape<1, 0, 0, 0>::BPS,
+                                     ClassShape<1, 1, 0, 0>::BPS, ClassShape<2, 0, 0, 0>::BPS,
+                                     ClassShape<2, 1, 0, 0>::BPS, ClassShape<2, 2, 0, 0>::BPS};
+    return bps[pc];
 }
 
-int tensor_class_bps(int qc)
+hipError_t launch_bra_table(int pc, const ShellPair* pairs, const PrimPair* pp, int boff, int nb, double* table,
+                            hipStream_t st)
+{
+    if (nb <= 0) return hipSuccess;
+#define CASE(i, a, b) \
+    case i: hipLaunchKernelGGL((bra_table_kernel<a, b>), dim3(nb), dim3(64), 0, st, pairs, pp, boff, table); break;
+    switch (pc) {
+        CASE(0, 0, 0) CASE(1, 1, 0) CASE(2, 1, 1) CASE(3, 2, 0) CASE(4, 2, 1) CASE(5, 2, 2)
+    default: return hipErrorInvalidValue;
+    }
+#undef CASE
+    return hipGetLastError();
+}
+
+#define DECLB(a, b, c, d) \
+    hipError_t block_class_launch_##a##b##c##d(const ClassArgs& A, const BlockArgs& B, hipStream_t st);
+MMD_CLASSES(DECLB)
+#undef DECLB
+
+hipError_t launch_block_class(int qc, const ClassArgs& A, const BlockArgs& B, hipStream_t st)
 {
     int la, lb, lc, ld;
     qclass_decode(qc, &la, &lb, &lc, &ld);
 #define CASE(a, b, c, d) \
-    if (la == a && lb == b && lc == c && ld == d) return tensor_class_bps_##a##b##c##d##_d();
+    if (la == a && lb == b && lc == c && ld == d) return block_class_launch_##a##b##c##d(A, B, st);
     MMD_CLASSES(CASE)
 #undef CASE
-    return 0;
+    return launch_block_dddd(A, B, st);
 }
 
 hipError_t launch_fock_class(int qc, int fp32, const ClassArgs& A, const RowArgs& R, int grid, hipStream_t st)

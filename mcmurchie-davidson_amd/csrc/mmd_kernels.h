@@ -40,13 +40,22 @@ hipError_t launch_fock_wave_class(int la, int lb, int lc, int ld, int fp32, cons
                                   hipStream_t st);
 hipError_t launch_fock_mfma_class(int la, int lb, int lc, int ld, int fp32, const ClassArgs& A, int64_t max_quartets,
                                   hipStream_t st);
-// Stored ERI tensor from shell quartets: class kernels (every class but
-// (dd|dd)) and the wavefront kernel for (dd|dd).  table: staged bra data,
-// tensor_class_bps(qc) doubles per primitive pair.
-hipError_t launch_tensor_class(int qc, const ClassArgs& A, int boff, int nb, int koff, int nk, int tri,
-                               double* table, double* out, hipStream_t st);
-int tensor_class_bps(int qc);
-hipError_t launch_tensor_wave_class(const ClassArgs& A, int64_t nquartets, hipStream_t st);
+// Integral blocks of one quartet class (stored tensor, or formPT's raw
+// build): mmd_eri_block.h, and the wavefront kernel for (dd|dd).
+hipError_t launch_block_class(int qc, const ClassArgs& A, const BlockArgs& B, hipStream_t st);
+hipError_t launch_block_dddd(const ClassArgs& A, const BlockArgs& B, hipStream_t st);
+// Staged bra data of a pair class: bra_table_stride(pc) doubles per primitive
+// pair, read by launch_block_class.
+int bra_table_stride(int pc);
+hipError_t launch_bra_table(int pc, const ShellPair* pairs, const PrimPair* pp, int boff, int nb, double* table,
+                            hipStream_t st);
+// Dsh of a raw build: the largest |dP| of a shell block in either order of
+// the two shells (dP need not be symmetric); infinity where a value is NaN, so
+// that the screen keeps what meets it.
+hipError_t launch_shell_block_max_raw(int nshell, const int* sh_bf0, const int* sh_nbf, int N, const double* absD,
+                                      double* Dsh, hipStream_t st);
+// out (n elements; may be the first copy) = the sum of nrep copies `stride` apart
+hipError_t launch_sum_copies(size_t n, int nrep, size_t stride, const double* rep, double* out, hipStream_t st);
 // High angular-momentum classes whose two Hermite contractions run on the
 // matrix cores (fock_mfma_class_kernel), one wavefront per shell quartet.
 inline bool fock_class_is_mfma(int la, int lb, int lc, int ld)

@@ -15,7 +15,7 @@ struct ShellPair {
     int32_t same;        // sa == sb
     int32_t mol;         // molecule of the pair (a basis can hold several, block-diagonally)
     int32_t c0;          // first basis function of that molecule
-    int32_t pad;
+    int32_t pad;         // its first primitive pair's position among those of its pair class
     double q;            // max over the pair's functions of sqrt((ab|ab))
 };
 
@@ -95,5 +95,19 @@ struct RowArgs {
     unsigned long long* stat_nprim;
 };
 
+// Work of one quartet class of the integral-block kernels: the stored tensor
+// (raw = 0, A.G the N^4 output) or formPT's unsymmetrised build (raw = 1,
+// A.G nrep copies of the real and imaginary N x N matrices).
+constexpr int BLOCK_GROUPS = 16;     // quartets of a wavefront at most (groups of at least 4 lanes)
+struct BlockArgs {
+    int boff, nb, koff, nk;     // bra and ket pairs of the class
+    int tri;                    // same pair class: ket <= bra
+    int lgb, lgk;               // a group is 2^lgb x 2^lgk lanes: bra x ket primitive pairs
+    const double* table;        // staged bra data of the bra's pair class
+    int raw, nrep;
+    const double* Dim;          // raw: imaginary part of dP, or null
+    const double* Dsh;          // raw: shell-block maxima of |dP|
+    int nshell;
+};
 
 }  // namespace mmd

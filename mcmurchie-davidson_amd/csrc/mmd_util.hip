@@ -4,6 +4,7 @@
 // one-electron integrals and the stored-tensor J/K contraction.
 #include <hip/hip_runtime.h>
 #include "mmd_device.h"
+#include "mmd_eri_block.h"
 #include "mmd_kernels.h"
 #include "mmd_scf.h"
 
@@ -630,15 +631,13 @@ __global__ void __launch_bounds__(64 * GW_WAVES) fock_wave_class_kernel(ClassArg
     }
 }
 
-// Compile-time variant for one class (used for (dd|dd)): lane m evaluates
-// F_m, the R_tuv levels are computed in parallel across the wavefront
-// through two LDS buffers, the E tables by six lanes; the ket contraction
-// W_tuv(cd) is spread over the lanes into LDS, then every lane applies the
-// bra expansion to its component quartets.  TENSOR: the integrals are
-// stored at their eight index permutations in A.G (an N^4 tensor) instead
-// of being digested into a Fock matrix.
-template <int LA, int LB, int LC, int LD, bool TENSOR = false>
-__global__ void __launch_bounds__(64 * GW_WAVES) fock_wave_class_kernel_t(ClassArgs A)
+// Integral blocks of (dd|dd) (mmd_eri_block.h's entry points), one wavefront
+// per shell quartet: lane m evaluates F_m, the R_tuv levels are computed in
+// parallel across the wavefront through two LDS buffers, the E tables by six
+// lanes; the ket contraction W_tuv(cd) is spread over the lanes into LDS,
+// then every lane applies the bra expansion to its component quartets.
+template <int LA, int LB, int LC, int LD>
+__global__ void __launch_bounds__(64 * GW_WAVES) eri_block_wave_kernel(ClassArgs A, BlockArgs B)
 {
     constexpr int L = LA + LB + LC + LD;
     constexpr int NA = ncart(LA), NB = ncart(LB), NC = ncart(LC), ND = ncart(LD);
@@ -653,12 +652,14 @@ __global__ void __launch_bounds__(64 * GW_WAVES) fock_wave_class_kernel_t(ClassA
     __shared__ double Es[GW_WAVES][3 * EB + 3 * EK];
     __shared__ double Fs[GW_WAVES][L + 1];
     const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int nq = *A.count;
-    const int N = A.N;
+    const int64_t nq = B.tri ? (int64_t)B.nb * (B.nb + 1) / 2 : (int64_t)B.nb * B.nk;
+    double* Grep = A.G + (B.raw ? (size_t)(blockIdx.x % B.nrep) * 2 * A.N * A.N : 0);
     for (int64_t q = (int64_t)blockIdx.x * GW_WAVES + wv; q < nq; q += (int64_t)gridDim.x * GW_WAVES) {
-        const int2 qd = A.quart[q];
+        int2 qd;
+        block_quartet(B, q, qd.x, qd.y);
         const ShellPair bra = A.pairs[qd.x];
         const ShellPair ket = A.pairs[qd.y];
+        if (B.raw && !raw_keeps(A, B, bra, ket)) continue;   // uniform across the wavefront
         double acc[NCPL];
         for (int i = 0; i < NCPL; ++i) acc[i] = 0.0;
         for (int ip = 0; ip < bra.npp; ++ip) {
@@ -764,52 +765,17 @@ __global__ void __launch_bounds__(64 * GW_WAVES) fock_wave_class_kernel_t(ClassA
                 wave_sync();
             }
         }
-        const int bfa = bra.bfa, bfb = bra.bfb, bfc = ket.bfa, bfd = ket.bfb;
-        if constexpr (TENSOR) {
-            const size_t n = (size_t)N;
-#pragma unroll
-            for (int i = 0; i < NCPL; ++i) {
-                const int k = lane + 64 * i;
-                if (k >= NTOT) continue;
-                const int ab = k / NCD, cd = k % NCD;
-                const size_t p = bfa + ab / NB, qq = bfb + ab % NB, r = bfc + cd / ND, s = bfd + cd % ND;
-                const size_t pq = p * n + qq, qp = qq * n + p, rs = r * n + s, sr = s * n + r;
-                // one producer per orbit of the eight permutations
-                if ((bra.same && p < qq) || (ket.same && r < s) || (qd.x == qd.y && pq < rs)) continue;
-                const double v = acc[i] * A.gcomp[p] * A.gcomp[qq] * A.gcomp[r] * A.gcomp[s];
-                A.G[pq * n * n + rs] = v;
-                A.G[qp * n * n + rs] = v;
-                A.G[pq * n * n + sr] = v;
-                A.G[qp * n * n + sr] = v;
-                A.G[rs * n * n + pq] = v;
-                A.G[sr * n * n + pq] = v;
-                A.G[rs * n * n + qp] = v;
-                A.G[sr * n * n + qp] = v;
-            }
-            continue;
-        }
-        const double deg = (bra.same ? 1.0 : 2.0) * (ket.same ? 1.0 : 2.0) * (qd.x == qd.y ? 1.0 : 2.0);
 #pragma unroll
         for (int i = 0; i < NCPL; ++i) {
             const int k = lane + 64 * i;
             if (k >= NTOT) continue;
             const int ab = k / NCD, cd = k % NCD;
-            const int p = bfa + ab / NB, qq = bfb + ab % NB, r = bfc + cd / ND, s = bfd + cd % ND;
-            const double* aD = A.absD;
-            const double bound = A.sqS[(size_t)p * N + qq] * A.sqS[(size_t)r * N + s]
-                * fmax(fmax(fmax(4.0 * aD[(size_t)p * N + qq], 4.0 * aD[(size_t)r * N + s]),
-                            fmax(aD[(size_t)p * N + r], aD[(size_t)p * N + s])),
-                       fmax(aD[(size_t)qq * N + r], aD[(size_t)qq * N + s]));
-            if (bound < A.tol) continue;
-            const double v = acc[i] * deg * A.gcomp[p] * A.gcomp[qq] * A.gcomp[r] * A.gcomp[s];
-            const double* D = A.D;
-            double* G = A.G;
-            atomicAdd(&G[(size_t)p * N + qq], v * D[(size_t)r * N + s]);
-            atomicAdd(&G[(size_t)r * N + s], v * D[(size_t)p * N + qq]);
-            atomicAdd(&G[(size_t)qq * N + s], -0.25 * v * D[(size_t)p * N + r]);
-            atomicAdd(&G[(size_t)qq * N + r], -0.25 * v * D[(size_t)p * N + s]);
-            atomicAdd(&G[(size_t)p * N + r], -0.25 * v * D[(size_t)qq * N + s]);
-            atomicAdd(&G[(size_t)p * N + s], -0.25 * v * D[(size_t)qq * N + r]);
+            const int a = ab / NB, b = ab % NB, c = cd / ND, d = cd % ND;
+            if (!unique_component(bra, ket, qd.x == qd.y, a, b, c, d)) continue;
+            const int p = bra.bfa + a, qq = bra.bfb + b, r = ket.bfa + c, s = ket.bfb + d;
+            const double v = acc[i] * A.gcomp[p] * A.gcomp[qq] * A.gcomp[r] * A.gcomp[s];
+            if (B.raw) raw_digest(A, B, Grep, v, p, qq, r, s);
+            else tensor_store(A.G, (size_t)A.N, v, p, qq, r, s);
         }
     }
 }
@@ -821,22 +787,16 @@ hipError_t launch_fock_wave_class(int la, int lb, int lc, int ld, int fp32, cons
     int64_t grid = (max_quartets + GW_WAVES - 1) / GW_WAVES;
     if (grid < 1) grid = 1;
     if (grid > 4096) grid = 4096;
-    if (la == 2 && lb == 2 && lc == 2 && ld == 2)
-        hipLaunchKernelGGL((fock_wave_class_kernel_t<2, 2, 2, 2>), dim3((unsigned)grid), dim3(64 * GW_WAVES), 0, st, A);
-    else
-        hipLaunchKernelGGL(fock_wave_class_kernel, dim3((unsigned)grid), dim3(64 * GW_WAVES), 0, st, A, la, lb, lc, ld);
+    hipLaunchKernelGGL(fock_wave_class_kernel, dim3((unsigned)grid), dim3(64 * GW_WAVES), 0, st, A, la, lb, lc, ld);
     return hipGetLastError();
 }
 
-// Stored-tensor mode of the (dd|dd) class: A.quart lists the canonical shell
-// quartets (*A.count of them) and A.G is the N^4 output tensor.
-hipError_t launch_tensor_wave_class(const ClassArgs& A, int64_t nquartets, hipStream_t st)
+hipError_t launch_block_dddd(const ClassArgs& A, const BlockArgs& B, hipStream_t st)
 {
-    if (nquartets <= 0) return hipSuccess;
-    int64_t grid = (nquartets + GW_WAVES - 1) / GW_WAVES;
-    if (grid > 4096) grid = 4096;
-    hipLaunchKernelGGL((fock_wave_class_kernel_t<2, 2, 2, 2, true>), dim3((unsigned)grid), dim3(64 * GW_WAVES), 0, st,
-                       A);
+    const int64_t nq = B.tri ? (int64_t)B.nb * (B.nb + 1) / 2 : (int64_t)B.nb * B.nk;
+    if (nq <= 0) return hipSuccess;
+    const int64_t grid = nq < 4 * 4096 ? (nq + GW_WAVES - 1) / GW_WAVES : 4096;
+    hipLaunchKernelGGL((eri_block_wave_kernel<2, 2, 2, 2>), dim3((unsigned)grid), dim3(64 * GW_WAVES), 0, st, A, B);
     return hipGetLastError();
 }
 
@@ -877,6 +837,51 @@ hipError_t launch_shell_block_max(int nshell, const int* sh_bf0, const int* sh_n
     if (n <= 0) return hipSuccess;
     hipLaunchKernelGGL(shell_block_max_kernel, dim3((n + 255) / 256), dim3(256), 0, st, nshell, sh_bf0, sh_nbf, N,
                        absD, Dsh);
+    return hipGetLastError();
+}
+
+__global__ void shell_block_max_raw_kernel(int nshell, const int* __restrict__ bf0, const int* __restrict__ nbf, int N,
+                                           const double* __restrict__ absD, double* __restrict__ Dsh)
+{
+    const int idx = blockIdx.x * blockDim.x + threadIdx.x;
+    if (idx >= nshell * nshell) return;
+    const int s1 = idx / nshell, s2 = idx % nshell;
+    double m = 0.0;
+    bool nan = false;
+    for (int i = 0; i < nbf[s1]; ++i)
+        for (int j = 0; j < nbf[s2]; ++j) {
+            const double u = absD[(size_t)(bf0[s1] + i) * N + bf0[s2] + j];
+            const double v = absD[(size_t)(bf0[s2] + j) * N + bf0[s1] + i];
+            nan = nan || u != u || v != v;
+            m = fmax(m, fmax(u, v));
+        }
+    Dsh[idx] = nan ? HUGE_VAL : m;
+}
+
+hipError_t launch_shell_block_max_raw(int nshell, const int* sh_bf0, const int* sh_nbf, int N, const double* absD,
+                                      double* Dsh, hipStream_t st)
+{
+    const int n = nshell * nshell;
+    if (n <= 0) return hipSuccess;
+    hipLaunchKernelGGL(shell_block_max_raw_kernel, dim3((n + 255) / 256), dim3(256), 0, st, nshell, sh_bf0, sh_nbf, N,
+                       absD, Dsh);
+    return hipGetLastError();
+}
+
+__global__ void sum_copies_kernel(size_t n, int nrep, size_t stride, const double* rep, double* out)
+{
+    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    double s = 0.0;
+    for (int r = 0; r < nrep; ++r) s += rep[r * stride + i];
+    out[i] = s;
+}
+
+hipError_t launch_sum_copies(size_t n, int nrep, size_t stride, const double* rep, double* out, hipStream_t st)
+{
+    if (n == 0) return hipSuccess;
+    hipLaunchKernelGGL(sum_copies_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, n, nrep, stride, rep,
+                       out);
     return hipGetLastError();
 }
 
