@@ -52,7 +52,7 @@ struct ClassShape {
     // ones) add the primitive-slice partials of a batch into an LDS buffer
     // and digest each quartet once; QB is their batch size (buffer <= 16 KB).
     static constexpr int NABCD = NAB * NCD;
-    static constexpr bool IBUF = NABCD <= 32;
+    static constexpr bool IBUF = NABCD <= 36;
     // Items are (quartet, ket primitive slice) pairs, not whole quartets,
     // for the buffered classes and for the classes whose ket pairs are the
     // heavily contracted (ss) and (ps) pairs (up to 81 primitive pairs per
