@@ -22,6 +22,7 @@
 #include "mmd_gemm.h"
 #include "mmd_grad.h"
 #include "mmd_kernels.h"
+#include "mmd_pairs.h"
 #include "mmd_scf.h"
 #include "mmd_types.h"
 
@@ -174,14 +175,16 @@ struct mmd_ctx {
 
     // shell pairs (grouped by pair class, sorted inside each class)
     bool pairs_ok = false;
-    double prim_qmax = 0.0;
-    std::vector<ShellPair> pairs;
     int pc_off[NPAIRCLASS + 1] = {0};
+    int pc_npp[NPAIRCLASS] = {0}, pc_maxpp[NPAIRCLASS] = {0};   // primitive pairs of a class, largest count of a pair
+    DevBuf<int2> d_ranges;              // per class and molecule: its pairs {first, end} in the class
+    DevBuf<int> w_count, w_scan, w_ints;   // work of the table build (PairWork; stats, unit counters)
+    DevBuf<double> w_q;
+    DevBuf<unsigned long long> w_qmax;
     DevBuf<ShellPair> d_pairs;
     DevBuf<PrimPair> d_pp;
     DevBuf<double> d_onee;   // S, T, V, M (3), L (3) of mmd_one_electron
     DevBuf<double> d_ns;     // overlap powers: S, X, U and the Newton-Schulz work (8 N^2 + 2)
-    int64_t npp_total = 0;
 
     // Schwarz
     bool schwarz_ok = false;
@@ -203,7 +206,6 @@ struct mmd_ctx {
     // primitive pair, the classes' bra slices (of grad_pslice primitive pairs,
     // and of one for the wavefront kernels) and flat primitive-pair lists,
     // made from the pair table on first use
-    std::vector<double> ppa;
     DevBuf<double> d_ppa, g_rep;
     DevBuf<int4> g_slices;
     DevBuf<int2> g_flat;
@@ -230,8 +232,6 @@ struct mmd_ctx {
     DevBuf<double> d_mol_dmax;          // per molecule: max |dP| of the build
     int64_t npl = 0;
     int rw = 0;
-    // per pair class, per molecule: the class-local range [first, end) of its pairs
-    std::vector<int> kr_first[NPAIRCLASS], kr_end[NPAIRCLASS];
 
     // density / Fock scratch
     DevBuf<double> d_D, d_Dim, d_absD, d_Dsh, d_G, d_Gout;
@@ -389,20 +389,6 @@ int upload_shells(mmd_ctx* c)
     return MMD_OK;
 }
 
-// Schwarz-type bound of a primitive pair's product function (any component):
-// sqrt([ab|ab]) of an s-type pair, 2 pi^{5/2} / (p^2 sqrt(2p)) K^2, times
-// (1 + |AB| + 1/sqrt(p))^{la+lb} 4^{la+lb} to cover the Hermite expansion of
-// higher angular momenta.
-double prim_bound(double p, double K, double AB2, int lab)
-{
-    const double s = sqrt(34.98683665524972497 / (p * p * sqrt(2.0 * p))) * fabs(K);
-    const double f = 4.0 * (1.0 + sqrt(AB2) + 1.0 / sqrt(p));
-    double m = 1.0;
-    for (int i = 0; i < lab; ++i) m *= f;
-    return s * m;
-}
-constexpr double PRIM_DROP = 1e-20;
-
 // Shells [mol_s0[m], mol_s0[m+1]) of each molecule (shells never span two),
 // and, for a batch, the molecules' blocks {f0, n, s0, s1} on the device.
 int molecule_shell_ranges(mmd_ctx* c)
@@ -430,13 +416,19 @@ int onee_pair_list(mmd_ctx* c)
     if (c->onee_list_ok) return MMD_OK;
     if (int rc = molecule_shell_ranges(c)) return rc;
     std::vector<std::vector<int2>> byclass(NPAIRCLASS);
-    for (int m = 0; m < c->nmol; ++m)
+    std::vector<int2> ranges((size_t)NPAIRCLASS * c->nmol);
+    for (int m = 0; m < c->nmol; ++m) {
+        for (int pc = 0; pc < NPAIRCLASS; ++pc) ranges[(size_t)pc * c->nmol + m].x = (int)byclass[pc].size();
         for (int I = c->mol_s0[m]; I < c->mol_s0[m + 1]; ++I)
             for (int J = c->mol_s0[m]; J <= I; ++J) {
                 int a = I, b = J;
                 if (c->shells[I].l < c->shells[J].l) std::swap(a, b);
                 byclass[pair_class(c->shells[a].l, c->shells[b].l)].push_back(make_int2(a, b));
             }
+        for (int pc = 0; pc < NPAIRCLASS; ++pc) ranges[(size_t)pc * c->nmol + m].y = (int)byclass[pc].size();
+    }
+    HIP_TRY(c->d_ranges.reserve(ranges.size()));
+    HIP_TRY(hipMemcpyAsync(c->d_ranges.p, ranges.data(), sizeof(int2) * ranges.size(), hipMemcpyHostToDevice, c->st));
     std::vector<int2> all;
     for (int pc = 0; pc < NPAIRCLASS; ++pc) {
         c->onee_off[pc] = (int)all.size();
@@ -508,245 +500,106 @@ int schwarz_diagonal(mmd_ctx* c, double* out)
     return MMD_OK;
 }
 
-// Host view of the Schwarz diagonal (pq|pq): element (i, j) = p[row[i] + j].
-// The full N x N matrix, or the molecules' diagonal blocks packed one after
-// another (pairs never mix molecules).
-struct DiagView {
-    const double* p = nullptr;
-    std::vector<int64_t> row;
-    double at(int i, int j) const { return p[row[i] + j]; }
-};
+void class_of(int qc, int* pcb, int* pck);
 
 // Shell pairs of each molecule, grouped by pair class and sorted in each
 // class by (molecule, primitive pairs descending, Schwarz factor
-// descending), with their primitive-pair tables.  diag: the full N x N
-// Schwarz diagonal (pq|pq), or null before it is known (factors 1).
-// Shell pairs I >= J in canonical orientation, with primitive-pair data.
-// `diag` (optional): the Schwarz diagonal for the factors q; pairs are then
-// sorted inside each pair class by (npp desc, q desc).
-int build_pairs(mmd_ctx* c, const DiagView* diag)
+// descending), with their primitive-pair tables, on the device.  diag: the
+// N x N Schwarz diagonal (pq|pq) on the device, or null before it is known
+// (factors 1).  With a diagonal also the Fock build's work units: they belong
+// to the pair table, and a build (mmd_fock_delta_noalloc) allocates nothing.
+int build_pairs(mmd_ctx* c, const double* diag)
 {
-    const int N = c->nbf;
-    if (int rc = molecule_shell_ranges(c)) return rc;
-    // largest primitive-pair bound, for the primitive-pair screen
-    c->prim_qmax = 0.0;
-    for (int m = 0; m < c->nmol; ++m)
-        for (int I = c->mol_s0[m]; I < c->mol_s0[m + 1]; ++I)
-            for (int J = c->mol_s0[m]; J <= I; ++J) {
-                const Shell& A = c->shells[I];
-                const Shell& B = c->shells[J];
-                const double AB2 = (A.x - B.x) * (A.x - B.x) + (A.y - B.y) * (A.y - B.y) + (A.z - B.z) * (A.z - B.z);
-                for (int i = 0; i < A.np; ++i)
-                    for (int j = 0; j < B.np; ++j) {
-                        const double ea = c->sh_exp[A.p0 + i], eb = c->sh_exp[B.p0 + j];
-                        const double p = ea + eb;
-                        const double K = c->sh_w[A.p0 + i] * c->sh_w[B.p0 + j] * exp(-ea * eb / p * AB2);
-                        c->prim_qmax = std::max(c->prim_qmax, prim_bound(p, K, AB2, A.l + B.l));
-                    }
-            }
-    std::vector<std::vector<ShellPair>> byclass(NPAIRCLASS);
-    std::vector<PrimPair> pp;
-    c->ppa.clear();
+    if (int rc = onee_pair_list(c)) return rc;
     c->grad_plan_ok = false;
     c->btab_ok = false;
-    for (int m = 0; m < c->nmol; ++m)
-        for (int I = c->mol_s0[m]; I < c->mol_s0[m + 1]; ++I)
-            for (int J = c->mol_s0[m]; J <= I; ++J) {
-                int a = I, b = J;
-                if (c->shells[I].l < c->shells[J].l) std::swap(a, b);
-                const Shell& A = c->shells[a];
-                const Shell& B = c->shells[b];
-                ShellPair sp;
-                sp.sa = a;
-                sp.sb = b;
-                sp.bfa = A.bf0;
-                sp.bfb = B.bf0;
-                sp.pp0 = (int)pp.size();
-                sp.same = (a == b) ? 1 : 0;
-                sp.mol = m;
-                sp.c0 = c->mol_f0[m];
-                sp.pad = 0;
-                // pair factor q = max sqrt((ab|ab)) over the pair's functions
-                double q = 1.0;
-                if (diag) {
-                    q = 0.0;
-                    for (int x = 0; x < ncart(A.l); ++x)
-                        for (int y = 0; y < ncart(B.l); ++y) {
-                            const double v = diag->at(A.bf0 + x, B.bf0 + y);
-                            const double r = v > 0.0 ? sqrt(v) : 0.0;
-                            if (r > q) q = r;
-                        }
-                }
-                sp.q = q;
-                const double AB2 = (A.x - B.x) * (A.x - B.x) + (A.y - B.y) * (A.y - B.y) + (A.z - B.z) * (A.z - B.z);
-                for (int i = 0; i < A.np; ++i)
-                    for (int j = 0; j < B.np; ++j) {
-                        const double ea = c->sh_exp[A.p0 + i], eb = c->sh_exp[B.p0 + j];
-                        PrimPair pq;
-                        pq.p = ea + eb;
-                        pq.K = c->sh_w[A.p0 + i] * c->sh_w[B.p0 + j] * exp(-ea * eb / pq.p * AB2);
-                        // Primitive-pair screening (Fock-build tables only): a pair
-                        // whose Schwarz-type bound, times the largest bound of any
-                        // pair, is below PRIM_DROP contributes less than that to
-                        // every primitive quartet and is left out.
-                        if (prim_bound(pq.p, pq.K, AB2, A.l + B.l) * c->prim_qmax < PRIM_DROP) continue;
-                        pq.Px = (ea * A.x + eb * B.x) / pq.p;
-                        pq.Py = (ea * A.y + eb * B.y) / pq.p;
-                        pq.Pz = (ea * A.z + eb * B.z) / pq.p;
-                        pq.PAx = pq.Px - A.x;
-                        pq.PAy = pq.Py - A.y;
-                        pq.PAz = pq.Pz - A.z;
-                        pq.PBx = pq.Px - B.x;
-                        pq.PBy = pq.Py - B.y;
-                        pq.PBz = pq.Pz - B.z;
-                        pq.inv2p = 0.5 / pq.p;
-                        pq.invp = 1.0 / pq.p;
-                        pp.push_back(pq);
-                        c->ppa.push_back(ea);
-                    }
-                sp.npp = (int)pp.size() - sp.pp0;
-                if (sp.npp == 0) sp.q = 0.0;   // no primitive pair survives: never screened in
-                byclass[pair_class(A.l, B.l)].push_back(sp);
-            }
-    c->pairs.clear();
-    for (int pc = 0; pc < NPAIRCLASS; ++pc) {
-        auto& v = byclass[pc];
-        if (diag)
-            std::stable_sort(v.begin(), v.end(), [](const ShellPair& x, const ShellPair& y) {
-                if (x.mol != y.mol) return x.mol < y.mol;
-                if (x.npp != y.npp) return x.npp > y.npp;
-                return x.q > y.q;
-            });
-        else   // no Schwarz factors yet: by contraction length, for the lanes' balance
-            std::stable_sort(v.begin(), v.end(), [](const ShellPair& x, const ShellPair& y) {
-                return x.mol != y.mol ? x.mol < y.mol : x.npp > y.npp;
-            });
-        int pos = 0;
-        for (ShellPair& sp : v) {
-            sp.pad = pos;
-            pos += sp.npp;
-        }
-        c->pc_off[pc] = (int)c->pairs.size();
-        c->kr_first[pc].assign(c->nmol, (int)v.size());
-        c->kr_end[pc].assign(c->nmol, 0);
-        for (int k = 0; k < (int)v.size(); ++k) {
-            const int m = v[k].mol;
-            c->kr_first[pc][m] = std::min(c->kr_first[pc][m], k);
-            c->kr_end[pc][m] = std::max(c->kr_end[pc][m], k + 1);
-        }
-        for (int m = 0; m < c->nmol; ++m)
-            if (c->kr_first[pc][m] > c->kr_end[pc][m]) c->kr_first[pc][m] = c->kr_end[pc][m] = 0;
-        c->pairs.insert(c->pairs.end(), v.begin(), v.end());
-    }
-    c->pc_off[NPAIRCLASS] = (int)c->pairs.size();
-    c->npp_total = (int64_t)pp.size();
-    HIP_TRY(c->d_pairs.reserve(c->pairs.size()));
-    HIP_TRY(c->d_pp.reserve(pp.size()));
-    HIP_TRY(hipMemcpyAsync(c->d_pairs.p, c->pairs.data(), sizeof(ShellPair) * c->pairs.size(), hipMemcpyHostToDevice,
-                           c->st));
-    HIP_TRY(hipMemcpyAsync(c->d_pp.p, pp.data(), sizeof(PrimPair) * pp.size(), hipMemcpyHostToDevice, c->st));
-    HIP_TRY(hipStreamSynchronize(c->st));
+    c->pairs_ok = c->units_ok = false;
+    for (int pc = 0; pc <= NPAIRCLASS; ++pc) c->pc_off[pc] = c->onee_off[pc];
+    const size_t n = (size_t)c->pc_off[NPAIRCLASS];
+    HIP_TRY(c->d_pairs.reserve(n));
+    HIP_TRY(c->w_count.reserve(n));
+    HIP_TRY(c->w_q.reserve(n));
+    HIP_TRY(c->w_scan.reserve(n + n / 1024 + 2));
+    HIP_TRY(c->w_qmax.reserve(1));
+    constexpr int STATS = (int)(sizeof(PairStats) / sizeof(int)), HIST = NQCLASS * UNIT_BUCKETS;
+    HIP_TRY(c->w_ints.reserve(STATS + NQCLASS + HIST));
+    int* d_counts = c->w_ints.p + STATS;
+    int* d_hist = d_counts + NQCLASS;
+    PairInput I;
+    I.shells = c->d_oshell.p;
+    I.exps = c->d_sh_exp.p;
+    I.wts = c->d_sh_w.p;
+    I.list = c->d_onee_list.p;
+    I.ranges = c->d_ranges.p;
+    I.mol_blocks = c->nmol > 1 ? c->d_mol_blocks.p : nullptr;
+    I.diag = diag;
+    I.nmol = c->nmol;
+    I.N = c->nbf;
+    PairWork W;
+    W.count = c->w_count.p;
+    W.q = c->w_q.p;
+    W.scan = c->w_scan.p;
+    W.qmax = c->w_qmax.p;
+    UnitInput U;
+    U.pairs = c->d_pairs.p;
+    U.ranges = c->d_ranges.p;
+    U.nmol = c->nmol;
+    for (int pc = 0; pc <= NPAIRCLASS; ++pc) I.off[pc] = U.off[pc] = c->pc_off[pc];
     // quartet-class sizes (implicit enumeration; for several molecules an
     // upper bound, the screen keeps the quartets of one molecule)
     c->qc_off[0] = 0;
     for (int qc = 0; qc < NQCLASS; ++qc) {
-        int pcb = 0;
-        while ((pcb + 1) * (pcb + 2) / 2 <= qc) ++pcb;
-        const int pck = qc - pcb * (pcb + 1) / 2;
+        int pcb, pck;
+        class_of(qc, &pcb, &pck);
         const int64_t nb = c->pc_off[pcb + 1] - c->pc_off[pcb];
         const int64_t nk = c->pc_off[pck + 1] - c->pc_off[pck];
         c->qc_total[qc] = (pcb == pck) ? nb * (nb + 1) / 2 : nb * nk;
         c->qc_off[qc + 1] = c->qc_off[qc] + c->qc_total[qc];
+        // ket segment of a work unit: long (survivors are batched inside a
+        // unit), but short enough for a few thousand segments per class.
+        // (Shorter segments make a class that runs alone faster, but cost
+        // more than they gain when classes or molecules share the GPU.)
+        int seg = 4096;
+        while (seg > 256 && c->qc_total[qc] / std::max(1, c->nmol) / seg < 4096) seg /= 2;
+        c->unit_seg[qc] = U.seg[qc] = seg;
     }
+    HIP_TRY(launch_pair_sort(I, W, c->d_pairs.p, reinterpret_cast<PairStats*>(c->w_ints.p), c->st));
+    if (diag) HIP_TRY(launch_unit_count(U, d_hist, d_counts, c->w_q.p, c->st));   // the factors are in the pairs now
+    int h[STATS + NQCLASS] = {0};
+    HIP_TRY(hipMemcpyAsync(h, c->w_ints.p, sizeof(int) * (STATS + (diag ? NQCLASS : 0)), hipMemcpyDeviceToHost, c->st));
+    HIP_TRY(hipStreamSynchronize(c->st));
+    PairStats stats;
+    memcpy(&stats, h, sizeof(stats));
+    size_t npp = 0;
+    for (int pc = 0; pc < NPAIRCLASS; ++pc) {
+        c->pc_npp[pc] = stats.total[pc];
+        c->pc_maxpp[pc] = std::max(1, stats.maxpp[pc]);
+        npp += (size_t)stats.total[pc];
+    }
+    HIP_TRY(c->d_pp.reserve(std::max<size_t>(1, npp)));
+    HIP_TRY(c->d_ppa.reserve(std::max<size_t>(1, npp)));
+    HIP_TRY(launch_pair_fill(I, W, c->d_pairs.p, c->d_pp.p, c->d_ppa.p, c->st));
+    if (diag) {
+        int64_t units = 0;
+        for (int qc = 0; qc < NQCLASS; ++qc) {
+            c->unit_off[qc] = units;
+            units += h[STATS + qc];
+        }
+        c->unit_off[NQCLASS] = units;
+        HIP_TRY(c->d_units.reserve(std::max<size_t>(1, (size_t)units)));
+        HIP_TRY(c->d_ubound.reserve(std::max<size_t>(1, (size_t)units)));
+        HIP_TRY(launch_unit_scatter(U, d_hist, c->w_q.p, c->d_units.p, c->d_ubound.p, c->st));
+        c->units_ok = true;
+    }
+    HIP_TRY(hipStreamSynchronize(c->st));
     HIP_TRY(c->d_count.reserve(2 * NQCLASS));
     c->pairs_ok = true;
-    c->units_ok = false;
     for (int qc = 0; qc < NQCLASS; ++qc) {
         c->plan_ms[qc] = 0.0;
         c->impl_choice[qc] = -1;
     }
     c->plan_countdown = 0;
     c->tune_phase = 0;
-    return MMD_OK;
-}
-
-// Work units of every class: one per (bra pair, slice of at most PSLICE of
-// its primitive pairs, segment of seg ket pairs), in decreasing order of
-// estimated cost (bra primitive pairs x ket primitive pairs of the
-// segment), so that the heaviest units start first.  Slicing the bra
-// primitives spreads the heavily contracted pairs over several workgroups.
-void class_of(int qc, int* pcb, int* pck);
-
-int build_units(mmd_ctx* c)
-{
-    std::vector<int4> all;
-    std::vector<UnitBound> allb;
-    std::vector<std::pair<double, int4>> v;
-    std::vector<double> kpre, kqmax;
-    for (int qc = 0; qc < NQCLASS; ++qc) {
-        c->unit_off[qc] = (int64_t)all.size();
-        int pcb, pck;
-        class_of(qc, &pcb, &pck);
-        const int boff = c->pc_off[pcb], nb = c->pc_off[pcb + 1] - boff;
-        const int koff = c->pc_off[pck], nk = c->pc_off[pck + 1] - koff;
-        const bool tri = pcb == pck;
-        const int64_t quartets = tri ? (int64_t)nb * (nb + 1) / 2 : (int64_t)nb * nk;
-        // ket segment: long (survivors are batched inside a unit), but short
-        // enough for a few thousand segments per class.  (Shorter segments
-        // make a class that runs alone faster, but cost more than they gain
-        // when classes or molecules share the GPU.)
-        int seg = 4096;
-        while (seg > 256 && quartets / std::max(1, c->nmol) / seg < 4096) seg /= 2;
-        c->unit_seg[qc] = seg;
-        if (nb == 0 || nk == 0) continue;
-        kpre.assign(nk + 1, 0.0);
-        for (int k = 0; k < nk; ++k) kpre[k + 1] = kpre[k] + c->pairs[koff + k].npp;
-        // largest ket pair factor of a segment [k0, k1): kets are sorted by
-        // molecule, so a running maximum restarted at each segment start
-        auto seg_qmax = [&](int k0, int k1) {
-            double m = 0.0;
-            for (int k = k0; k < k1; ++k) m = std::max(m, c->pairs[koff + k].q);
-            return m;
-        };
-        v.clear();
-        for (int P = 0; P < nb; ++P) {
-            const ShellPair& bp = c->pairs[boff + P];
-            const int npp = bp.npp;
-            // the kets of the bra pair's molecule (up to the bra pair itself
-            // in the triangular classes)
-            const int kfirst = c->kr_first[pck][bp.mol];
-            const int kend = tri ? P + 1 : c->kr_end[pck][bp.mol];
-            for (int k0 = kfirst; k0 < kend; k0 += seg) {
-                const int k1 = std::min(kend, k0 + seg);
-                const double kc = kpre[k1] - kpre[k0];
-                for (int ip = 0; ip < npp; ip += PSLICE) {
-                    const int ip1 = std::min(npp, ip + PSLICE);
-                    v.push_back({(ip1 - ip) * kc, make_int4(P, ip | (ip1 << 16), k0, k1)});
-                }
-            }
-        }
-        std::stable_sort(v.begin(), v.end(), [](const std::pair<double, int4>& x, const std::pair<double, int4>& y) {
-            return x.first > y.first;
-        });
-        for (auto& e : v) {
-            all.push_back(e.second);
-            const ShellPair& bp = c->pairs[boff + e.second.x];
-            const double qb = bp.q * seg_qmax(e.second.z, e.second.w);
-            float qf = (float)qb;
-            if ((double)qf < qb) qf = nextafterf(qf, HUGE_VALF);
-            allb.push_back(UnitBound{qf, bp.mol});
-        }
-    }
-    c->unit_off[NQCLASS] = (int64_t)all.size();
-    HIP_TRY(c->d_units.reserve(std::max<size_t>(1, all.size())));
-    HIP_TRY(c->d_ubound.reserve(std::max<size_t>(1, allb.size())));
-    if (!all.empty()) {
-        HIP_TRY(hipMemcpyAsync(c->d_units.p, all.data(), sizeof(int4) * all.size(), hipMemcpyHostToDevice, c->st));
-        HIP_TRY(hipMemcpyAsync(c->d_ubound.p, allb.data(), sizeof(UnitBound) * allb.size(), hipMemcpyHostToDevice,
-                               c->st));
-    }
-    HIP_TRY(hipStreamSynchronize(c->st));
-    c->units_ok = true;
     return MMD_OK;
 }
 
@@ -839,11 +692,7 @@ struct FockScratch {
 int run_fock_classes(mmd_ctx* c, ClassArgs A, double tol, FockScratch& W0)
 {
     const bool tier32 = c->fp32_below > tol;
-    if (!c->units_ok) {
-        if (!W0.allow_measure) return fail(MMD_ERR_STATE, "work units are built by mmd_schwarz / mmd_set_schwarz");
-        const int rc = build_units(c);
-        if (rc) return rc;
-    }
+    if (!c->units_ok) return fail(MMD_ERR_STATE, "work units are built by mmd_schwarz / mmd_set_schwarz");
     bool row_kernel[NQCLASS], kj_lds[NQCLASS];
     int maxpp[NQCLASS];
     // a build that times the row or the matrix-core variant of the classes
@@ -859,8 +708,7 @@ int run_fock_classes(mmd_ctx* c, ClassArgs A, double tol, FockScratch& W0)
         int la, lb, lc, ld, pcb, pck;
         qclass_decode(qc, &la, &lb, &lc, &ld);
         class_of(qc, &pcb, &pck);
-        maxpp[qc] = 1;
-        for (int P = c->pc_off[pcb]; P < c->pc_off[pcb + 1]; ++P) maxpp[qc] = std::max(maxpp[qc], c->pairs[P].npp);
+        maxpp[qc] = c->pc_maxpp[pcb];
         bool mfma = fock_class_is_wave(la, lb, lc, ld);
         if (mfma && fock_class_has_both(la, lb, lc, ld)) {
             if (c->impl_mode == 0) mfma = false;
@@ -900,9 +748,6 @@ int run_fock_classes(mmd_ctx* c, ClassArgs A, double tol, FockScratch& W0)
     // events on its own stream (times include sharing the GPU with the other
     // classes); mode 2 runs the classes one after the other on the main
     // stream, so that each class's events time it alone.
-    double pc_npp[NPAIRCLASS] = {0};
-    for (int pc = 0; pc < NPAIRCLASS; ++pc)
-        for (int P = c->pc_off[pc]; P < c->pc_off[pc + 1]; ++P) pc_npp[pc] += c->pairs[P].npp;
     int order[NQCLASS], nord = 0;
     double cost[NQCLASS] = {0};
     for (int qc = 0; qc < NQCLASS; ++qc) {
@@ -910,7 +755,7 @@ int run_fock_classes(mmd_ctx* c, ClassArgs A, double tol, FockScratch& W0)
         int pcb, pck, la, lb, lc, ld;
         class_of(qc, &pcb, &pck);
         qclass_decode(qc, &la, &lb, &lc, &ld);
-        const double prim = pc_npp[pcb] * pc_npp[pck] * (pcb == pck ? 0.5 : 1.0);
+        const double prim = (double)c->pc_npp[pcb] * c->pc_npp[pck] * (pcb == pck ? 0.5 : 1.0);
         const int L = la + lb + lc + ld;
         cost[qc] = prim * (40.0 + 4.0 * nherm(L) + (double)ncart(la) * ncart(lb) * ncart(lc) * ncart(ld));
         order[nord++] = qc;
@@ -1075,32 +920,18 @@ int collect_profile(mmd_ctx* c)
 namespace {
 // The Schwarz matrix (pq|pq) is in d_schwarz: its square roots for the
 // screen, and the sorted shell-pair tables with their factors
-// q = max sqrt((ab|ab)) from the host view diag.
-int finish_schwarz(mmd_ctx* ctx, const DiagView& diag)
+// q = max sqrt((ab|ab)) and the work units.
+int finish_schwarz(mmd_ctx* ctx)
 {
     const size_t nn = (size_t)ctx->nbf * ctx->nbf;
     HIP_TRY(launch_sqrt_clamped(nn, ctx->d_schwarz.p, ctx->d_sqS.p, ctx->st));
-    HIP_TRY(hipStreamSynchronize(ctx->st));
+    if (ctx->shells_ok) {   // else only the per-function paths are available
+        if (int rc = build_pairs(ctx, ctx->d_schwarz.p)) return rc;
+    } else {
+        HIP_TRY(hipStreamSynchronize(ctx->st));
+    }
     ctx->schwarz_ok = true;
-    if (!ctx->shells_ok) return MMD_OK;   // only the per-function paths are available
-    const int rc = build_pairs(ctx, &diag);   // pair factors q from the diagonal
-    if (rc) return rc;
-    // the Fock build's work units belong to the pair table: built here, at
-    // set-up, so that a build (mmd_fock_delta_noalloc) allocates nothing
-    return build_units(ctx);
-}
-
-// Install a Schwarz diagonal (N*N, (pq|pq), host) and rebuild the pair tables.
-int set_schwarz(mmd_ctx* ctx, const std::vector<double>& h)
-{
-    const int N = ctx->nbf;
-    const size_t nn = (size_t)N * N;
-    HIP_TRY(hipMemcpyAsync(ctx->d_schwarz.p, h.data(), sizeof(double) * nn, hipMemcpyHostToDevice, ctx->st));
-    DiagView v;
-    v.p = h.data();
-    v.row.resize(N);
-    for (int i = 0; i < N; ++i) v.row[i] = (int64_t)i * N;
-    return finish_schwarz(ctx, v);
+    return MMD_OK;
 }
 
 }  // namespace
@@ -1361,6 +1192,9 @@ namespace {
 int build_grad_plan(mmd_ctx* c)
 {
     if (c->grad_plan_ok) return MMD_OK;
+    std::vector<ShellPair> pairs((size_t)c->pc_off[NPAIRCLASS]);
+    HIP_TRY(hipMemcpyAsync(pairs.data(), c->d_pairs.p, sizeof(ShellPair) * pairs.size(), hipMemcpyDeviceToHost, c->st));
+    HIP_TRY(hipStreamSynchronize(c->st));
     std::vector<int4> sl, one;
     std::vector<int2> flat;
     for (int pc = 0; pc < NPAIRCLASS; ++pc) {
@@ -1371,15 +1205,13 @@ int build_grad_plan(mmd_ctx* c)
         // molecule would not give the class some 1000 work units: a slice is
         // a serial chain in every lane, and a small molecule leaves most of
         // the GPU idle ((H2O) cc-pVDZ, (pp|pp): 133 us in 10 workgroups of 16)
-        int64_t prims = 0, kets = 0;
-        for (int P = 0; P < c->pc_off[pc + 1]; ++P) {
-            kets += c->pairs[P].npp;
-            if (P >= c->pc_off[pc]) prims += c->pairs[P].npp;
-        }
+        int64_t kets = 0;
+        for (int k = 0; k <= pc; ++k) kets += c->pc_npp[k];
+        const int64_t prims = c->pc_npp[pc];
         int step = grad_pslice(pc);
         while (step > 1 && (prims / step) * (kets / 256 + 1) < 1024) step /= 2;
         for (int P = c->pc_off[pc]; P < c->pc_off[pc + 1]; ++P) {
-            const int npp = c->pairs[P].npp;
+            const int npp = pairs[P].npp;
             for (int i = 0; i < npp; ++i) flat.push_back(make_int2(P, i));
             const int end = (int)flat.size() - c->g_flat_off[pc];
             for (int i = 0; i < npp; i += step) sl.push_back(make_int4(P, i, std::min(npp, i + step), end));
@@ -1394,10 +1226,8 @@ int build_grad_plan(mmd_ctx* c)
     sl.insert(sl.end(), one.begin(), one.end());
     HIP_TRY(c->g_slices.reserve(std::max<size_t>(1, sl.size())));
     HIP_TRY(c->g_flat.reserve(std::max<size_t>(1, flat.size())));
-    HIP_TRY(c->d_ppa.reserve(std::max<size_t>(1, c->ppa.size())));
     HIP_TRY(hipMemcpyAsync(c->g_slices.p, sl.data(), sizeof(int4) * sl.size(), hipMemcpyHostToDevice, c->st));
     HIP_TRY(hipMemcpyAsync(c->g_flat.p, flat.data(), sizeof(int2) * flat.size(), hipMemcpyHostToDevice, c->st));
-    HIP_TRY(hipMemcpyAsync(c->d_ppa.p, c->ppa.data(), sizeof(double) * c->ppa.size(), hipMemcpyHostToDevice, c->st));
     HIP_TRY(hipStreamSynchronize(c->st));
     c->grad_plan_ok = true;
     return MMD_OK;
@@ -1569,13 +1399,10 @@ int mmd_schwarz(mmd_ctx* ctx, double* diag)
     if (ctx->nbf == 0) return fail(MMD_ERR_STATE, "no basis set");
     const int N = ctx->nbf;
     const size_t nn = (size_t)N * N;
-    std::vector<double> h(nn);
     HIP_TRY(ctx->d_schwarz.reserve(nn));
     if ((rc = schwarz_diagonal(ctx, ctx->d_schwarz.p))) return rc;
-    HIP_TRY(hipMemcpyAsync(h.data(), ctx->d_schwarz.p, sizeof(double) * nn, hipMemcpyDeviceToHost, ctx->st));
-    HIP_TRY(hipStreamSynchronize(ctx->st));
-    if (diag) memcpy(diag, h.data(), sizeof(double) * nn);
-    return set_schwarz(ctx, h);
+    if (diag) HIP_TRY(hipMemcpyAsync(diag, ctx->d_schwarz.p, sizeof(double) * nn, hipMemcpyDeviceToHost, ctx->st));
+    return finish_schwarz(ctx);
 }
 
 int mmd_set_schwarz(mmd_ctx* ctx, const double* diag)
@@ -1584,8 +1411,10 @@ int mmd_set_schwarz(mmd_ctx* ctx, const double* diag)
     if (rc) return rc;
     if (ctx->nbf == 0) return fail(MMD_ERR_STATE, "no basis set");
     if (!diag) return fail(MMD_ERR_ARG, "null pointer");
-    std::vector<double> h(diag, diag + (size_t)ctx->nbf * ctx->nbf);
-    return set_schwarz(ctx, h);
+    const size_t nn = (size_t)ctx->nbf * ctx->nbf;
+    HIP_TRY(ctx->d_schwarz.reserve(nn));
+    HIP_TRY(hipMemcpyAsync(ctx->d_schwarz.p, diag, sizeof(double) * nn, hipMemcpyHostToDevice, ctx->st));
+    return finish_schwarz(ctx);
 }
 
 namespace {
@@ -1596,8 +1425,7 @@ int build_bra_tables(mmd_ctx* c)
     size_t total = 0;
     for (int pc = 0; pc < NPAIRCLASS; ++pc) {
         c->btab_off[pc] = total;
-        for (int P = c->pc_off[pc]; P < c->pc_off[pc + 1]; ++P)
-            total += (size_t)c->pairs[P].npp * bra_table_stride(pc);
+        total += (size_t)c->pc_npp[pc] * bra_table_stride(pc);
     }
     HIP_TRY(c->d_btab.reserve(std::max<size_t>(1, total)));
     for (int pc = 0; pc < NPAIRCLASS; ++pc)
@@ -1614,9 +1442,7 @@ int run_block_classes(mmd_ctx* c, const ClassArgs& A, const BlockArgs& raw)
     if (int rc = build_bra_tables(c)) return rc;
     std::vector<StreamTask> tasks;
     BlockArgs cls[NQCLASS];
-    int64_t npp[NPAIRCLASS] = {0};
-    for (int pc = 0; pc < NPAIRCLASS; ++pc)
-        for (int P = c->pc_off[pc]; P < c->pc_off[pc + 1]; ++P) npp[pc] += c->pairs[P].npp;
+    const int* npp = c->pc_npp;
     for (int qc = 0; qc < NQCLASS; ++qc) {
         int pcb, pck, la, lb, lc, ld;
         class_of(qc, &pcb, &pck);
@@ -2249,20 +2075,7 @@ int mmd_batch_rhf(mmd_ctx* ctx, const int32_t* nocc, const double* enuc, const d
     B.lds_bytes = c->lds_per_block;
     B.mol = c->b_mol.p;
     HIP_TRY(c->b_work.reserve(std::max<size_t>(1, wtot)));   // 3 n^2 per molecule: staging for packed blocks
-    {
-        // the molecules' diagonal blocks of (pq|pq), packed, for the pair factors
-        HIP_TRY(launch_batch_pack(B, c->d_schwarz.p, c->b_work.p, st));
-        std::vector<double> h(std::max<size_t>(1, ptot));
-        HIP_TRY(hipMemcpyAsync(h.data(), c->b_work.p, sizeof(double) * ptot, hipMemcpyDeviceToHost, st));
-        HIP_TRY(hipStreamSynchronize(st));
-        DiagView v;
-        v.p = h.data();
-        v.row.resize(N);
-        for (int m = 0; m < M; ++m)
-            for (int i = 0; i < mols[m].n; ++i)
-                v.row[mols[m].f0 + i] = (int64_t)mols[m].po + (int64_t)i * mols[m].n - mols[m].f0;
-        if ((rc = finish_schwarz(c, v))) return rc;
-    }
+    if ((rc = finish_schwarz(c))) return rc;
     // buffers of the Fock build, reserved before any capture
     HIP_TRY(c->d_rowctr.reserve(2 * NQCLASS));
     HIP_TRY(c->d_nprim.reserve(NPRIM_SLOTS));

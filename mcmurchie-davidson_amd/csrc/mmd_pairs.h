@@ -1,0 +1,69 @@
+// Shell-pair tables and Fock work units, built on the device (mmd_pairs.hip).
+#pragma once
+#include <hip/hip_runtime.h>
+#include "mmd_device.h"
+#include "mmd_kernels.h"
+#include "mmd_types.h"
+
+namespace mmd {
+
+constexpr int UNIT_BUCKETS = 128;    // cost classes of the work units (quarter octaves)
+constexpr int QMAX_BLOCK = 32;       // kets per running maximum of the pair factors
+
+// What the build reads: the shells, the shell pairs of every molecule grouped
+// by pair class (list[off[pc] .. off[pc+1]), by molecule inside a class), the
+// class-local range {first, end} of each molecule's pairs (ranges[pc * nmol +
+// m]), and the Schwarz diagonal (N x N, or null: factors 1).
+struct PairInput {
+    const OneeShell* shells;
+    const double* exps;
+    const double* wts;
+    const int2* list;
+    const int2* ranges;
+    const int4* mol_blocks;          // {first function, ...} per molecule, or null for one molecule
+    const double* diag;
+    int off[NPAIRCLASS + 1];
+    int nmol, N;
+};
+
+// Work buffers, npairs entries each but for the last two.
+struct PairWork {
+    int* count;                      // surviving primitive pairs, list order
+    double* q;                       // pair factors, list order
+    int* scan;                       // npairs + npairs / 1024 + 2
+    unsigned long long* qmax;        // largest primitive-pair bound
+};
+
+// Results on the host: largest and total primitive-pair count per class.
+struct PairStats {
+    int maxpp[NPAIRCLASS];
+    int total[NPAIRCLASS];
+};
+
+// Primitive pairs counted and screened, the pairs sorted inside each class by
+// (molecule, primitive pairs descending, factor descending, list order) into
+// `pairs` with their ranges in the primitive-pair table, class by class.
+hipError_t launch_pair_sort(const PairInput& I, const PairWork& W, ShellPair* pairs, PairStats* stats, hipStream_t st);
+// The primitive-pair table of the sorted pairs, and each entry's first
+// exponent (ppa).
+hipError_t launch_pair_fill(const PairInput& I, const PairWork& W, const ShellPair* pairs, PrimPair* pp, double* ppa,
+                            hipStream_t st);
+
+// Work units of the row kernels.  One per (bra pair, slice of at most PSLICE
+// of its primitive pairs, segment of seg[qc] kets of its molecule), in
+// decreasing order of cost (bra x ket primitive pairs, by quarter octaves).
+struct UnitInput {
+    const ShellPair* pairs;
+    const int2* ranges;
+    int off[NPAIRCLASS + 1];
+    int seg[NQCLASS];
+    int nmol;
+};
+// hist: NQCLASS x UNIT_BUCKETS counters; counts[qc]: units of class qc;
+// qrun: npairs running maxima.  The scatter takes the cursors that the count
+// left in hist, and writes class qc at units + (sum of the counts before it).
+hipError_t launch_unit_count(const UnitInput& I, int* hist, int* counts, double* qrun, hipStream_t st);
+hipError_t launch_unit_scatter(const UnitInput& I, int* hist, const double* qrun, int4* units, UnitBound* bounds,
+                               hipStream_t st);
+
+}  // namespace mmd
