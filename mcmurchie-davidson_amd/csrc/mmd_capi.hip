@@ -619,6 +619,19 @@ int grid_for(int64_t items)
     return (int)g;
 }
 
+// The side streams that nstreams asks for, created when a basis is set: HIP
+// deals streams to its few hardware queues in order of creation, so contexts
+// that each made all seven at once had their main streams on one queue, and
+// batch groups on different contexts ran one after the other.
+int ensure_streams(mmd_ctx* c)
+{
+    for (int i = 0; i + 1 < c->nstreams; ++i) {
+        if (!c->side[i]) HIP_TRY(hipStreamCreateWithFlags(&c->side[i], hipStreamNonBlocking));
+        if (!c->evjoin[i]) HIP_TRY(hipEventCreateWithFlags(&c->evjoin[i], hipEventDisableTiming));
+    }
+    return MMD_OK;
+}
+
 // Independent launches spread over the context's streams, largest first and
 // each to the least loaded stream, between a fork from and a join to c->st.
 struct StreamTask {
@@ -997,10 +1010,6 @@ int mmd_ctx_create(mmd_ctx** out, int device_id)
     if (e == hipSuccess) e = hipEventCreate(&c->ev0);
     if (e == hipSuccess) e = hipEventCreate(&c->ev1);
     if (e == hipSuccess) e = hipEventCreateWithFlags(&c->evfork, hipEventDisableTiming);
-    for (int i = 0; i < mmd_ctx::NSIDE && e == hipSuccess; ++i) {
-        e = hipStreamCreateWithFlags(&c->side[i], hipStreamNonBlocking);
-        if (e == hipSuccess) e = hipEventCreateWithFlags(&c->evjoin[i], hipEventDisableTiming);
-    }
     std::vector<double> tab;
     boys_build_table(tab);
     if (e == hipSuccess) e = c->d_boys.reserve(tab.size());
@@ -1102,6 +1111,7 @@ int mmd_set_basis(mmd_ctx* ctx, int nbf, const double* origin, const int32_t* lm
         rc = upload_shells(ctx);
         if (rc) return rc;
     }
+    if ((rc = ensure_streams(ctx))) return rc;
     const size_t nn = (size_t)nbf * nbf;
     HIP_TRY(ctx->d_D.reserve(nn));
     HIP_TRY(ctx->d_Dim.reserve(nn));
@@ -1887,7 +1897,9 @@ int mmd_set_streams(mmd_ctx* ctx, int n)
     if (!ctx) return fail(MMD_ERR_ARG, "null context");
     if (n < 1 || n > 1 + mmd_ctx::NSIDE) return fail(MMD_ERR_ARG, "streams must be in [1, %d]", 1 + mmd_ctx::NSIDE);
     ctx->nstreams = n;
-    return MMD_OK;
+    if (ctx->nbf == 0) return MMD_OK;
+    HIP_TRY(hipSetDevice(ctx->device));
+    return ensure_streams(ctx);
 }
 
 int mmd_set_lds_limit(mmd_ctx* ctx, int64_t bytes)
