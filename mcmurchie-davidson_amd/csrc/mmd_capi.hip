@@ -183,6 +183,10 @@ struct mmd_ctx {
     DevBuf<unsigned long long> w_qmax;
     DevBuf<ShellPair> d_pairs;
     DevBuf<PrimPair> d_pp;
+    DevBuf<KetScreen> d_kscr;    // ket tables of the row kernels
+    DevBuf<KetRef> d_kref;
+    DevBuf<double> d_kpp;
+    int64_t kpp_stride = 0;
     DevBuf<double> d_onee;   // S, T, V, M (3), L (3) of mmd_one_electron
     DevBuf<double> d_ns;     // overlap powers: S, X, U and the Newton-Schulz work (8 N^2 + 2)
 
@@ -578,7 +582,12 @@ int build_pairs(mmd_ctx* c, const double* diag)
     }
     HIP_TRY(c->d_pp.reserve(std::max<size_t>(1, npp)));
     HIP_TRY(c->d_ppa.reserve(std::max<size_t>(1, npp)));
-    HIP_TRY(launch_pair_fill(I, W, c->d_pairs.p, c->d_pp.p, c->d_ppa.p, c->st));
+    c->kpp_stride = (int64_t)((std::max<size_t>(1, npp) + 15) & ~(size_t)15);   // fields start on cache lines
+    HIP_TRY(c->d_kscr.reserve(n));
+    HIP_TRY(c->d_kref.reserve(n));
+    HIP_TRY(c->d_kpp.reserve((size_t)(KET_FIELDS * c->kpp_stride)));
+    const KetTables K = {c->d_kscr.p, c->d_kref.p, c->d_kpp.p, c->kpp_stride};
+    HIP_TRY(launch_pair_fill(I, W, c->d_pairs.p, c->d_pp.p, c->d_ppa.p, K, c->st));
     if (diag) {
         int64_t units = 0;
         for (int qc = 0; qc < NQCLASS; ++qc) {
@@ -826,6 +835,11 @@ int run_fock_classes(mmd_ctx* c, ClassArgs A, double tol, FockScratch& W0)
             R.kslice = c->ket_slice[qc];
             R.seg = c->unit_seg[qc];
             R.rw = c->rw;
+            R.kscr = c->d_kscr.p;
+            R.kref = c->d_kref.p;
+            R.kpp = c->d_kpp.p;
+            R.kstride = c->kpp_stride;
+            R.ket_npp = (int)(c->pc_npp[pck] / std::max(1, nk));
             R.units = c->d_units.p + c->unit_off[qc];
             R.ubound = c->d_ubound.p + c->unit_off[qc];
             const int64_t units = c->unit_off[qc + 1] - c->unit_off[qc];

@@ -84,7 +84,7 @@ __device__ __forceinline__ double wave_sum63(double v)
 // block goes to G.
 template <int LA, int LB, int LC, int LD, int A0, int A1>
 __device__ __forceinline__ void quartet_digest(const ClassArgs& A, int2 qd, const ShellPair& bra,
-                                               const ShellPair& ket, double* acc, double* rowA, double* rowB,
+                                               const KetRef& ket, double* acc, double* rowA, double* rowB,
                                                int RW, bool on, double* kj = nullptr)
 {
     using S = ClassShape<LA, LB, LC, LD>;
@@ -105,7 +105,7 @@ __device__ __forceinline__ void quartet_digest(const ClassArgs& A, int2 qd, cons
     sfor<S::NB>([&](auto i) { gb[i] = A.gcomp[bfb + i]; });
     sfor<S::NC>([&](auto i) { gc[i] = A.gcomp[bfc + i]; });
     sfor<S::ND>([&](auto i) { gd[i] = A.gcomp[bfd + i]; });
-    const double deg = (bra.same ? 1.0 : 2.0) * (ket.same ? 1.0 : 2.0) * (qd.x == qd.y ? 1.0 : 2.0);
+    const double deg = (bra.same ? 1.0 : 2.0) * (ket.bfa == ket.bfb ? 1.0 : 2.0) * (qd.x == qd.y ? 1.0 : 2.0);
     const double* D = A.D;
     double* G = A.G;
     const double* sq = A.sqS;
@@ -269,10 +269,40 @@ struct ClassList {
     static constexpr int QLIST = QB + CLASS_BLOCK;   // batch + one screening step
 };
 
+// Classes built in two forms: one ket primitive pair at a time, and two at a
+// time (KU) where kets are heavily contracted.  Only (ss) kets gain: at
+// (H2O)16 cc-pVDZ two at a time took (ss|ss) 0.77 -> 0.74, (ps|ss) 1.69 ->
+// 1.57, (pp|ss) 0.96 -> 0.82, (ds|ss) 0.70 -> 0.60 ms, while for the shorter
+// 6-31G kets of a batch (ps|ss) lost 10% and (pp|ss) 4% to the weightless
+// chains.  The launch takes two for an average of at least KU_MIN_NPP
+// primitive pairs per (ss) pair (6-31G water about 6, cc-pVDZ 12).
+constexpr int KU_MIN_NPP = 9;
+template <int LA, int LB, int LC, int LD>
+constexpr bool row_has_ku2()
+{
+    return LC + LD == 0 && LA + LB <= 2;
+}
+
+// Least wavefronts per SIMD that the compiler plans the registers for.  The
+// row kernels wait more than they compute (at (H2O)16 cc-pVDZ the vector
+// units are busy 30% of the time), so a second or third wavefront pays where
+// it costs few spills: (pp|pp) 0.385 -> 0.284, (ds|pp) 0.451 -> 0.321, (ds|ds)
+// 0.332 -> 0.281 ms for two instead of one (2-15 registers spilled), (ps|ps)
+// 1.21 -> 1.10 ms for three instead of two (none).  (pp|ps), (dp|ss), (dp|ps)
+// and (dd|ss) were slower with more.
+template <int LA, int LB, int LC, int LD, typename T>
+constexpr int row_min_waves()
+{
+    constexpr int c = LA * 1000 + LB * 100 + LC * 10 + LD;
+    if (!std::is_same<T, double>::value) return 1;
+    if (c == 1111 || c == 2011 || c == 2020) return 2;
+    return c == 1010 ? 3 : 1;
+}
+
 // T is the arithmetic type of the integrals (double, or float for the
 // FP32 tier); screening, digestion and all accumulation into G are FP64.
-template <int LA, int LB, int LC, int LD, typename T>
-__global__ void __launch_bounds__(CLASS_BLOCK) eri_fock_class_kernel(ClassArgs A, RowArgs R)
+template <int LA, int LB, int LC, int LD, int KU, typename T>
+__global__ void __launch_bounds__(CLASS_BLOCK, (row_min_waves<LA, LB, LC, LD, T>())) eri_fock_class_kernel(ClassArgs A, RowArgs R)
 {
     using S = ClassShape<LA, LB, LC, LD>;
     constexpr int QB = S::QB;
@@ -351,7 +381,7 @@ __global__ void __launch_bounds__(CLASS_BLOCK) eri_fock_class_kernel(ClassArgs A
                 const int t = t0 + threadIdx.x;
                 bool keep = false;
                 if (t < segn) {
-                    const ShellPair ket = A.pairs[R.koff + k0 + t];
+                    const KetScreen ket = R.kscr[R.koff + k0 + t];
                     const double* Dsh = R.Dsh;
                     const double dm = fmax(fmax(fmax(4.0 * Dsh[bra.sa * ns + bra.sb], 4.0 * Dsh[ket.sa * ns + ket.sb]),
                                                 fmax(Dsh[bra.sa * ns + ket.sa], Dsh[bra.sa * ns + ket.sb])),
@@ -384,7 +414,7 @@ __global__ void __launch_bounds__(CLASS_BLOCK) eri_fock_class_kernel(ClassArgs A
                 if constexpr (S::KSL) {
                     const int j = threadIdx.x;   // cnt <= QB <= CLASS_BLOCK
                     int x = 0;
-                    if (j < cnt) x = (A.pairs[R.koff + qlist[b0 + j]].npp + R.kslice - 1) / R.kslice;
+                    if (j < cnt) x = (R.kref[R.koff + qlist[b0 + j]].npp + R.kslice - 1) / R.kslice;
                     for (int off = 1; off < 64; off <<= 1) {
                         const int y = __shfl_up(x, off);
                         if (lane >= off) x += y;
@@ -418,7 +448,7 @@ __global__ void __launch_bounds__(CLASS_BLOCK) eri_fock_class_kernel(ClassArgs A
                     }
                     const int Q = qlist[b0 + idx];
                     const int2 qd = make_int2(R.boff + P, R.koff + Q);
-                    const ShellPair ket = A.pairs[qd.y];
+                    const KetRef ket = R.kref[qd.y];
                     const int jq0 = ks * R.kslice;
                     const int jq1 = on ? (S::KSL ? min(ket.npp, jq0 + R.kslice) : ket.npp) : jq0;
                     const int ip0 = 0, ip1 = bnp;
@@ -427,7 +457,8 @@ __global__ void __launch_bounds__(CLASS_BLOCK) eri_fock_class_kernel(ClassArgs A
                         constexpr int C = decltype(ic)::value;
                         constexpr int A0 = C * S::CH, A1 = (C + 1) * S::CH;
                         T acc[(A1 - A0) * S::NCD];
-                        quartet_compute<LA, LB, LC, LD, A0, A1, T>(A, boys_tab, bp, ket, ip0, ip1, jq0, jq1, acc);
+                        quartet_compute<LA, LB, LC, LD, A0, A1, KU, T>(KetArrays{R.kpp, R.kstride}, boys_tab, bp, ip0, ip1,
+                                                                   ket.pp0 + jq0, ket.pp0 + jq1, acc);
                         if constexpr (S::IBUF) {
                             double* dst = ibuf + (size_t)idx * S::NABCD + A0 * S::NCD;
                             if (on) sfor<(A1 - A0) * S::NCD>(
@@ -449,7 +480,7 @@ __global__ void __launch_bounds__(CLASS_BLOCK) eri_fock_class_kernel(ClassArgs A
                         if (v == 0.0) continue;
                         ibuf[i] = 0.0;
                         const int idx = i / S::NCD, cd = i - idx * S::NCD;
-                        const ShellPair ket = A.pairs[R.koff + qlist[b0 + idx]];
+                        const KetRef ket = R.kref[R.koff + qlist[b0 + idx]];
                         atomicAdd(&A.G[(size_t)(ket.bfa + cd / S::ND) * N + ket.bfb + cd % S::ND], v);
                     }
                 }
@@ -464,7 +495,7 @@ __global__ void __launch_bounds__(CLASS_BLOCK) eri_fock_class_kernel(ClassArgs A
                         const int idx = on ? item : cnt - 1;
                         const int Q = qlist[b0 + idx];
                         const int2 qd = make_int2(R.boff + P, R.koff + Q);
-                        const ShellPair ket = A.pairs[qd.y];
+                        const KetRef ket = R.kref[qd.y];
                         static_switch<0, S::NCHUNK>(chunk, [&](auto ic) {
                             constexpr int C = decltype(ic)::value;
                             constexpr int A0 = C * S::CH, A1 = (C + 1) * S::CH;

@@ -45,9 +45,15 @@ struct PairStats {
 // `pairs` with their ranges in the primitive-pair table, class by class.
 hipError_t launch_pair_sort(const PairInput& I, const PairWork& W, ShellPair* pairs, PairStats* stats, hipStream_t st);
 // The primitive-pair table of the sorted pairs, and each entry's first
-// exponent (ppa).
+// exponent (ppa), and the row kernels' ket tables of both.
+struct KetTables {
+    KetScreen* scr;
+    KetRef* ref;
+    double* pp;
+    int64_t stride;
+};
 hipError_t launch_pair_fill(const PairInput& I, const PairWork& W, const ShellPair* pairs, PrimPair* pp, double* ppa,
-                            hipStream_t st);
+                            const KetTables& K, hipStream_t st);
 
 // Work units of the row kernels.  One per (bra pair, slice of at most PSLICE
 // of its primitive pairs, segment of seg[qc] kets of its molecule), in

@@ -200,7 +200,8 @@ __global__ void __launch_bounds__(256) pair_place_kernel(PairInput I, const int*
 
 __global__ void __launch_bounds__(256) pair_fill_kernel(PairInput I, const unsigned long long* __restrict__ qmax_bits,
                                                         const ShellPair* __restrict__ pairs,
-                                                        PrimPair* __restrict__ pp, double* __restrict__ ppa)
+                                                        PrimPair* __restrict__ pp, double* __restrict__ ppa,
+                                                        KetTables K)
 {
     const int e = blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= I.off[NPAIRCLASS]) return;
@@ -209,6 +210,8 @@ __global__ void __launch_bounds__(256) pair_fill_kernel(PairInput I, const unsig
     const OneeShell a = I.shells[sp.sa], b = I.shells[sp.sb];
     const double AB2 = dist2(a, b);
     int o = sp.pp0;
+    K.scr[e] = KetScreen{sp.q, sp.sa, sp.sb};
+    K.ref[e] = KetRef{sp.bfa, sp.bfb, sp.pp0, sp.npp};
     for (int i = 0; i < a.np; ++i)
         for (int j = 0; j < b.np; ++j) {
             const double ea = I.exps[a.p0 + i], eb = I.exps[b.p0 + j];
@@ -229,6 +232,9 @@ __global__ void __launch_bounds__(256) pair_fill_kernel(PairInput I, const unsig
             pq.invp = 1.0 / pq.p;
             pp[o] = pq;
             ppa[o] = ea;
+            const double f[KET_FIELDS] = {pq.p, pq.K * pq.invp, pq.Px, pq.Py, pq.Pz, pq.inv2p,
+                                          pq.PAx, pq.PAy, pq.PAz, pq.PBx, pq.PBy, pq.PBz};
+            for (int k = 0; k < KET_FIELDS; ++k) K.pp[k * K.stride + o] = f[k];
             ++o;
         }
 }
@@ -394,11 +400,11 @@ hipError_t launch_pair_sort(const PairInput& I, const PairWork& W, ShellPair* pa
 }
 
 hipError_t launch_pair_fill(const PairInput& I, const PairWork& W, const ShellPair* pairs, PrimPair* pp, double* ppa,
-                            hipStream_t st)
+                            const KetTables& K, hipStream_t st)
 {
     const int n = I.off[NPAIRCLASS];
     if (n <= 0) return hipSuccess;
-    hipLaunchKernelGGL(pair_fill_kernel, dim3((n + 255) / 256), dim3(256), 0, st, I, W.qmax, pairs, pp, ppa);
+    hipLaunchKernelGGL(pair_fill_kernel, dim3((n + 255) / 256), dim3(256), 0, st, I, W.qmax, pairs, pp, ppa, K);
     return hipGetLastError();
 }
 

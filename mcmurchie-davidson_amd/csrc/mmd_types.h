@@ -30,6 +30,20 @@ struct PrimPair {
     double inv2p, invp;
 };
 
+// What the row kernels read of a ket pair: its screen, and its functions and
+// primitive pairs.  16 bytes each in the order of the pair table, so that
+// consecutive lanes read consecutive records.
+struct KetScreen {
+    double q;
+    int32_t sa, sb;
+};
+struct KetRef {
+    int32_t bfa, bfb, pp0, npp;
+};
+// Fields of the primitive pairs field by field (KET_FIELDS arrays of the
+// table's length), for lanes that take consecutive primitive pairs.
+enum KetField { KF_P, KF_KQ, KF_X, KF_Y, KF_Z, KF_INV2P, KF_PAX, KF_PAY, KF_PAZ, KF_PBX, KF_PBY, KF_PBZ, KET_FIELDS };
+
 // Arguments of the quartet-class kernels (passed by value).
 struct ClassArgs {
     const int2* quart;          // surviving (bra pair, ket pair) for this class
@@ -93,6 +107,11 @@ struct RowArgs {
     int* row_counter;           // next work unit (zeroed before the launch)
     unsigned long long* stat_nquart;   // optional statistics
     unsigned long long* stat_nprim;
+    const KetScreen* kscr;      // all pairs
+    const KetRef* kref;
+    const double* kpp;          // field f of primitive pair i at kpp[f * kstride + i]
+    int64_t kstride;
+    int ket_npp;                // average primitive pairs per ket pair of the class
 };
 
 // Work of one quartet class of the integral-block kernels: the stored tensor

@@ -1,0 +1,36 @@
+"""Forms of the row kernels: one ket primitive pair at a time or two, which is
+taken by the average contraction of the (ss) pairs (6-31G below the line,
+cc-pVDZ above it, STO-3G's nine at it), over ket slices of one, an odd number
+and all primitive pairs, so that the second of two chains is sometimes without
+a pair.  The symmetrised build against the per-function kernels (functions in
+reversed order form no whole shells); both sum at most 1e6 FP64 terms: 1e-11
+of max |G|."""
+import numpy as np
+import pytest
+
+from geometries import water_cluster
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("basis", ["sto-3g", "6-31g", "cc-pvdz"])
+@pytest.mark.parametrize("kslice", [1, 2, 3, 16])
+def test_ket_chains(basis, kslice):
+    from mmd import _native
+    from mmd.molecule import Molecule
+    mol = Molecule(water_cluster(2, 5.0, seed=4, perturb=True), basis)
+    N = mol.nbasis
+    rng = np.random.default_rng(kslice)
+    D = rng.normal(size=(N, N))
+    D = D + D.T
+    ctx = _native.Context()
+    ctx.set_basis_from_bfs(mol.bfs)
+    ctx.schwarz()
+    ctx.set_ket_slices([kslice] * 21)
+    G = ctx.fock_delta(D, tol=1e-12)[0]
+    r = np.arange(N)[::-1]
+    ref = _native.Context()
+    ref.set_basis_from_bfs([mol.bfs[i] for i in r])
+    ref.schwarz()
+    R = ref.fock_delta(D[np.ix_(r, r)], tol=1e-12, raw=True)[0][np.ix_(r, r)]
+    assert np.max(np.abs(G - 0.5 * (R + R.T))) < 1e-11 * np.max(np.abs(G))
