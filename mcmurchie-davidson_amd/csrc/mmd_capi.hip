@@ -7,6 +7,7 @@
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <stdarg.h>
+#include <stddef.h>
 #include <stdio.h>
 #include <stdlib.h>
 #include <string.h>
@@ -104,6 +105,15 @@ struct DevBuf {
 // ---------------------------------------------------------------------------
 constexpr size_t NOALLOC_SCRATCH_BYTES = size_t(16) << 20;   // 16 MiB
 constexpr int NPRIM_SLOTS = 4 * NQCLASS;   // survivor counters of one Fock build
+// A build's counters, in one block: what the host reads back (survivors, list
+// lengths) first, then the row kernels' unit counters.
+struct FockCounters {
+    unsigned long long nprim[NPRIM_SLOTS];   // see FockScratch::nprim
+    int count[2 * NQCLASS];                  // survivor-list lengths (FP64 lists, then FP32)
+    int rowctr[2 * NQCLASS];
+};
+constexpr int FOCK_COUNTER_WORDS = (int)(sizeof(FockCounters) / sizeof(int));
+constexpr int FOCK_REPORT_WORDS = (int)(offsetof(FockCounters, rowctr) / sizeof(int));
 
 // Per-class sums over profiled builds; index 0 the FP64 launches, 1 the FP32 tier.
 struct ProfileSum {
@@ -198,7 +208,8 @@ struct mmd_ctx {
     int64_t qc_total[NQCLASS] = {0};
     int64_t qc_off[NQCLASS + 1] = {0};
     DevBuf<int2> d_surv;
-    DevBuf<int> d_count;
+    DevBuf<FockCounters> d_ctr;
+    FockCounters* h_ctr = nullptr;   // pinned: the counters of the last build
 
     // atoms
     int natom = 0;
@@ -260,8 +271,6 @@ struct mmd_ctx {
     int tune_phase = 0;
     double tune_ms[2][NQCLASS] = {};
     bool tune_measuring = false;
-    DevBuf<unsigned long long> d_nprim;   // NPRIM_SLOTS counters (FockScratch::nprim)
-    DevBuf<int> d_rowctr;
     // Work units of the row-kernel classes (built once per pair table):
     // class qc owns units [unit_off[qc], unit_off[qc+1]) with ket segment
     // length unit_seg[qc].
@@ -601,7 +610,7 @@ int build_pairs(mmd_ctx* c, const double* diag)
         c->units_ok = true;
     }
     HIP_TRY(hipStreamSynchronize(c->st));
-    HIP_TRY(c->d_count.reserve(2 * NQCLASS));
+    HIP_TRY(c->d_ctr.reserve(1));
     c->pairs_ok = true;
     for (int qc = 0; qc < NQCLASS; ++qc) {
         c->plan_ms[qc] = 0.0;
@@ -694,11 +703,17 @@ ClassArgs base_args(mmd_ctx* c)
 // kernel (class qc at surv + surv_off[qc]).  The context's buffers, or a
 // caller-free static array (mmd_fock_delta_noalloc).
 struct FockScratch {
-    int* rowctr = nullptr;                 // 2 * NQCLASS
-    int* count = nullptr;                  // 2 * NQCLASS: survivor-list lengths (FP64 lists, then FP32)
+    int* rowctr = nullptr;                 // cleared, with the others, by the build's preparation kernel
+    int* count = nullptr;
     // NPRIM_SLOTS counters: primitive quartets (FP64 tier), shell quartets of
     // the row kernels (FP64, FP32 tier), primitive quartets (FP32 tier)
     unsigned long long* nprim = nullptr;
+    void counters(FockCounters* c)
+    {
+        rowctr = c->rowctr;
+        count = c->count;
+        nprim = c->nprim;
+    }
     double* Dsh = nullptr;                 // nshell^2
     const double* mol_dmax = nullptr;      // batches: per-molecule max |dP| (units of molecules at 0 skipped)
     int2* surv = nullptr;
@@ -761,9 +776,6 @@ int run_fock_classes(mmd_ctx* c, ClassArgs A, double tol, FockScratch& W0)
                         (long long)W0.surv_cap);
         }
     }
-    HIP_TRY(launch_fill_int(2 * NQCLASS, W0.rowctr, 0, c->st));
-    HIP_TRY(launch_fill_int(2 * NQCLASS, W0.count, 0, c->st));
-    HIP_TRY(launch_fill_int(2 * NPRIM_SLOTS, reinterpret_cast<int*>(W0.nprim), 0, c->st));
     // Classes run concurrently on the main and side streams (longest first,
     // each to the least loaded stream), so that the small classes fill the
     // GPU beside the large ones.  Profiling mode 1 brackets every class with
@@ -906,16 +918,30 @@ int run_fock_classes(mmd_ctx* c, ClassArgs A, double tol, FockScratch& W0)
     return MMD_OK;
 }
 
+// Survivors of the build whose counters are in h_ctr: per-class lists (wave
+// classes) and FP64 and FP32 row-kernel counts.
+void count_survivors(mmd_ctx* c)
+{
+    const int* h = c->h_ctr->count;
+    const unsigned long long* hq = c->h_ctr->nprim + NQCLASS;
+    int64_t s = 0, s32 = 0;
+    for (int i = 0; i < NQCLASS; ++i) {
+        s += (int64_t)h[i] + (int64_t)h[NQCLASS + i] + (int64_t)hq[i] + (int64_t)hq[NQCLASS + i];
+        s32 += (int64_t)h[NQCLASS + i] + (int64_t)hq[NQCLASS + i];
+    }
+    c->last_nsurv = s;
+    c->last_nsurv_fp32 = s32;
+}
+
 // Per-class statistics and event times of the last build (profiling on),
 // also added to the sums since profiling was turned on.  Called after the
 // build's end event, so the readback is not timed.
 int collect_profile(mmd_ctx* c)
 {
-    int h[2 * NQCLASS];
-    unsigned long long hp[NPRIM_SLOTS];
-    HIP_TRY(hipMemcpyAsync(h, c->d_count.p, sizeof(int) * 2 * NQCLASS, hipMemcpyDeviceToHost, c->st));
-    HIP_TRY(hipMemcpyAsync(hp, c->d_nprim.p, sizeof(hp), hipMemcpyDeviceToHost, c->st));
+    HIP_TRY(hipMemcpyAsync(c->h_ctr, c->d_ctr.p, sizeof(FockCounters), hipMemcpyDeviceToHost, c->st));
     HIP_TRY(hipStreamSynchronize(c->st));
+    const int* h = c->h_ctr->count;
+    const unsigned long long* hp = c->h_ctr->nprim;
     for (int qc = 0; qc < NQCLASS; ++qc) {
         if (!c->qc_total[qc]) {
             c->st_nquart[qc] = c->st_nprim[qc] = 0;
@@ -1021,6 +1047,7 @@ int mmd_ctx_create(mmd_ctx** out, int device_id)
     c->max_lds_device = c->max_lds;
     if (lds_max > 0) c->lds_per_block = (size_t)lds_max;
     hipError_t e = hipStreamCreateWithFlags(&c->st, hipStreamNonBlocking);
+    if (e == hipSuccess) e = hipHostMalloc((void**)&c->h_ctr, sizeof(FockCounters), hipHostMallocDefault);
     if (e == hipSuccess) e = hipEventCreate(&c->ev0);
     if (e == hipSuccess) e = hipEventCreate(&c->ev1);
     if (e == hipSuccess) e = hipEventCreateWithFlags(&c->evfork, hipEventDisableTiming);
@@ -1065,6 +1092,7 @@ void mmd_ctx_destroy(mmd_ctx* ctx)
     if (ctx->evfork) (void)hipEventDestroy(ctx->evfork);
     std::lock_guard<std::recursive_mutex> lk(device_alloc_mutex());
     if (ctx->blas) (void)rocblas_destroy_handle(ctx->blas);
+    if (ctx->h_ctr) (void)hipHostFree(ctx->h_ctr);
     hipStream_t st = ctx->st;
     delete ctx;  // frees device buffers
     if (st) (void)hipStreamDestroy(st);
@@ -1601,27 +1629,25 @@ int mmd_fock_delta(mmd_ctx* ctx, const double* dP_re, const double* dP_im, doubl
     HIP_TRY(hipEventRecord(ctx->ev0, ctx->st));
     HIP_TRY(hipMemcpyAsync(ctx->d_D.p, dP_re, sizeof(double) * nn, k_in, ctx->st));
     if (dP_im) HIP_TRY(hipMemcpyAsync(ctx->d_Dim.p, dP_im, sizeof(double) * nn, k_in, ctx->st));
-    HIP_TRY(launch_abs_density((int)nn, ctx->d_D.p, dP_im ? ctx->d_Dim.p : nullptr, ctx->d_absD.p, ctx->st));
+    if (raw)
+        HIP_TRY(launch_abs_density((int)nn, ctx->d_D.p, dP_im ? ctx->d_Dim.p : nullptr, ctx->d_absD.p, ctx->st));
     if (!raw) {
-        HIP_TRY(launch_shell_block_max((int)ctx->shells.size(), ctx->d_sh_bf0.p, ctx->d_sh_nbf.p, N, ctx->d_absD.p,
-                                       ctx->d_Dsh.p, ctx->st));
+        HIP_TRY(launch_fock_prep(N, ctx->d_D.p, ctx->d_absD.p, ctx->d_G.p, ctx->d_sh_bf0.p, ctx->d_sh_nbf.p,
+                                 (int)ctx->shells.size(), ctx->d_Dsh.p, reinterpret_cast<int*>(ctx->d_ctr.p),
+                                 FOCK_COUNTER_WORDS, ctx->st));
         ClassArgs A = base_args(ctx);
         A.absD = ctx->d_absD.p;
         A.sqS = ctx->d_sqS.p;
         A.tol = tol;
         A.D = ctx->d_D.p;
         A.G = ctx->d_G.p;
-        HIP_TRY(launch_fill(nn, ctx->d_G.p, 0.0, ctx->st));
-        HIP_TRY(ctx->d_rowctr.reserve(2 * NQCLASS));
-        HIP_TRY(ctx->d_nprim.reserve(NPRIM_SLOTS));
         FockScratch W;
-        W.rowctr = ctx->d_rowctr.p;
-        W.count = ctx->d_count.p;
-        W.nprim = ctx->d_nprim.p;
+        W.counters(ctx->d_ctr.p);
         W.Dsh = ctx->d_Dsh.p;
         rc = run_fock_classes(ctx, A, tol, W);
         if (rc) return rc;
-        HIP_TRY(launch_symmetrize(N, ctx->d_G.p, ctx->d_Gout.p, ctx->st));
+        HIP_TRY(launch_symmetrize(N, ctx->d_G.p, ctx->d_Gout.p, ctx->st, reinterpret_cast<const int*>(ctx->d_ctr.p),
+                                  reinterpret_cast<int*>(ctx->h_ctr), FOCK_REPORT_WORDS));
         HIP_TRY(hipMemcpyAsync(G_re, ctx->d_Gout.p, sizeof(double) * nn, k_out, ctx->st));
     } else if (ctx->pairs_ok && ctx->nmol == 1) {
         if ((rc = raw_fock_shells(ctx, dP_im != nullptr, tol))) return rc;
@@ -1637,25 +1663,9 @@ int mmd_fock_delta(mmd_ctx* ctx, const double* dP_re, const double* dP_im, doubl
         }
     }
     HIP_TRY(hipEventRecord(ctx->ev1, ctx->st));
-    if (!raw) {
-        // survivors: per-class lists (wave classes) + FP64 and FP32 row-kernel counts
-        int h[2 * NQCLASS];
-        unsigned long long hq[2 * NQCLASS];
-        HIP_TRY(hipMemcpyAsync(h, ctx->d_count.p, sizeof(int) * 2 * NQCLASS, hipMemcpyDeviceToHost, ctx->st));
-        HIP_TRY(hipMemcpyAsync(hq, ctx->d_nprim.p + NQCLASS, sizeof(hq), hipMemcpyDeviceToHost, ctx->st));
-        HIP_TRY(hipStreamSynchronize(ctx->st));
-        int64_t s = 0, s32 = 0;
-        for (int i = 0; i < NQCLASS; ++i) {
-            s += (int64_t)h[i] + (int64_t)h[NQCLASS + i] + (int64_t)hq[i] + (int64_t)hq[NQCLASS + i];
-            s32 += (int64_t)h[NQCLASS + i] + (int64_t)hq[NQCLASS + i];
-        }
-        ctx->last_nsurv = s;
-        ctx->last_nsurv_fp32 = s32;
-        if (nsurv) *nsurv = s;
-    } else if (nsurv) {
-        *nsurv = -1;
-    }
     HIP_TRY(hipStreamSynchronize(ctx->st));
+    if (!raw) count_survivors(ctx);
+    if (nsurv) *nsurv = raw ? -1 : ctx->last_nsurv;
     float ms = 0.f;
     HIP_TRY(hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
     ctx->last_fock_ms = ms;
@@ -1718,50 +1728,34 @@ int mmd_fock_delta_noalloc(mmd_ctx* ctx, const double* dP, double tol, double* G
     off += up(sizeof(double) * nn);
     double* Dsh = reinterpret_cast<double*>(base + off);
     off += up(sizeof(double) * ns * ns);
-    int* rowctr = reinterpret_cast<int*>(base + off);
-    off += up(sizeof(int) * 2 * NQCLASS);
-    int* count = reinterpret_cast<int*>(base + off);
-    off += up(sizeof(int) * 2 * NQCLASS);
-    unsigned long long* nprim = reinterpret_cast<unsigned long long*>(base + off);
-    off += up(sizeof(unsigned long long) * NPRIM_SLOTS);
+    FockCounters* ctr = reinterpret_cast<FockCounters*>(base + off);
+    off += up(sizeof(FockCounters));
     if (off > NOALLOC_SCRATCH_BYTES)
         return fail(MMD_ERR_ARG, "a basis of %d functions needs %zu bytes of scratch; the limit is %zu", N, off,
                     NOALLOC_SCRATCH_BYTES);
     FockScratch W;
-    W.rowctr = rowctr;
-    W.count = count;
-    W.nprim = nprim;
+    W.counters(ctr);
     W.Dsh = Dsh;
     W.surv = reinterpret_cast<int2*>(base + off);
     W.surv_cap = (int64_t)((NOALLOC_SCRATCH_BYTES - off) / sizeof(int2));
     W.allow_measure = false;
     HIP_TRY(hipEventRecord(ctx->ev0, ctx->st));
-    HIP_TRY(launch_abs_density((int)nn, dP, nullptr, absD, ctx->st));
-    HIP_TRY(launch_shell_block_max((int)ns, ctx->d_sh_bf0.p, ctx->d_sh_nbf.p, N, absD, Dsh, ctx->st));
+    HIP_TRY(launch_fock_prep(N, dP, absD, Gacc, ctx->d_sh_bf0.p, ctx->d_sh_nbf.p, (int)ns, Dsh,
+                             reinterpret_cast<int*>(ctr), FOCK_COUNTER_WORDS, ctx->st));
     ClassArgs A = base_args(ctx);
     A.absD = absD;
     A.sqS = ctx->d_sqS.p;
     A.tol = tol;
     A.D = dP;
     A.G = Gacc;
-    HIP_TRY(launch_fill(nn, Gacc, 0.0, ctx->st));
     rc = run_fock_classes(ctx, A, tol, W);
     if (rc) return rc;
-    HIP_TRY(launch_symmetrize(N, Gacc, G, ctx->st));
+    HIP_TRY(launch_symmetrize(N, Gacc, G, ctx->st, reinterpret_cast<const int*>(ctr),
+                              reinterpret_cast<int*>(ctx->h_ctr), FOCK_REPORT_WORDS));
     HIP_TRY(hipEventRecord(ctx->ev1, ctx->st));
-    int h[2 * NQCLASS];
-    unsigned long long hq[2 * NQCLASS];
-    HIP_TRY(hipMemcpyAsync(h, count, sizeof(int) * 2 * NQCLASS, hipMemcpyDeviceToHost, ctx->st));
-    HIP_TRY(hipMemcpyAsync(hq, nprim + NQCLASS, sizeof(hq), hipMemcpyDeviceToHost, ctx->st));
     HIP_TRY(hipStreamSynchronize(ctx->st));
-    int64_t sum = 0, s32 = 0;
-    for (int i = 0; i < NQCLASS; ++i) {
-        sum += (int64_t)h[i] + (int64_t)h[NQCLASS + i] + (int64_t)hq[i] + (int64_t)hq[NQCLASS + i];
-        s32 += (int64_t)h[NQCLASS + i] + (int64_t)hq[NQCLASS + i];
-    }
-    ctx->last_nsurv = sum;
-    ctx->last_nsurv_fp32 = s32;
-    if (nsurv) *nsurv = sum;
+    count_survivors(ctx);
+    if (nsurv) *nsurv = ctx->last_nsurv;
     float ms = 0.f;
     HIP_TRY(hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
     ctx->last_fock_ms = ms;
@@ -1997,12 +1991,11 @@ int enqueue_fock_sym(mmd_ctx* c, const double* dP, double tol, double* Gout)
     const bool blocks = c->nmol > 1;   // a batch: only the molecules' diagonal blocks are live
     if (blocks) {
         HIP_TRY(launch_block_prep(c->nmol, c->d_mol_blocks.p, N, dP, c->d_absD.p, c->d_G.p, c->d_sh_bf0.p,
-                                  c->d_sh_nbf.p, (int)c->shells.size(), c->d_Dsh.p, c->d_mol_dmax.p, c->st));
+                                  c->d_sh_nbf.p, (int)c->shells.size(), c->d_Dsh.p, c->d_mol_dmax.p,
+                                  reinterpret_cast<int*>(c->d_ctr.p), FOCK_COUNTER_WORDS, c->st));
     } else {
-        HIP_TRY(launch_abs_density((int)nn, dP, nullptr, c->d_absD.p, c->st));
-        HIP_TRY(launch_shell_block_max((int)c->shells.size(), c->d_sh_bf0.p, c->d_sh_nbf.p, N, c->d_absD.p,
-                                       c->d_Dsh.p, c->st));
-        HIP_TRY(launch_fill(nn, c->d_G.p, 0.0, c->st));
+        HIP_TRY(launch_fock_prep(N, dP, c->d_absD.p, c->d_G.p, c->d_sh_bf0.p, c->d_sh_nbf.p, (int)c->shells.size(),
+                                 c->d_Dsh.p, reinterpret_cast<int*>(c->d_ctr.p), FOCK_COUNTER_WORDS, c->st));
     }
     ClassArgs A = base_args(c);
     A.absD = c->d_absD.p;
@@ -2011,9 +2004,7 @@ int enqueue_fock_sym(mmd_ctx* c, const double* dP, double tol, double* Gout)
     A.D = dP;
     A.G = c->d_G.p;
     FockScratch W;
-    W.rowctr = c->d_rowctr.p;
-    W.count = c->d_count.p;
-    W.nprim = c->d_nprim.p;
+    W.counters(c->d_ctr.p);
     W.profile_events = true;
     W.Dsh = c->d_Dsh.p;
     W.mol_dmax = blocks ? c->d_mol_dmax.p : nullptr;
@@ -2103,8 +2094,6 @@ int mmd_batch_rhf(mmd_ctx* ctx, const int32_t* nocc, const double* enuc, const d
     HIP_TRY(c->b_work.reserve(std::max<size_t>(1, wtot)));   // 3 n^2 per molecule: staging for packed blocks
     if ((rc = finish_schwarz(c))) return rc;
     // buffers of the Fock build, reserved before any capture
-    HIP_TRY(c->d_rowctr.reserve(2 * NQCLASS));
-    HIP_TRY(c->d_nprim.reserve(NPRIM_SLOTS));
     {
         int64_t wave = 0;
         for (int qc = 0; qc < NQCLASS; ++qc) {

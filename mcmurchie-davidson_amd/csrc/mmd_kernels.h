@@ -139,17 +139,18 @@ hipError_t launch_rhf_gradient(int nbf, const BFDesc* bfs, const double* pexp, c
 // first shell, end shell}): |dP|, zero G, shell maxima and each molecule's
 // max |dP| (mol_dmax) in the blocks only; the symmetrisation of the blocks.
 hipError_t launch_block_prep(int nmol, const int4* blocks, int N, const double* dP, double* absD, double* G,
-                             const int* sh_bf0, const int* sh_nbf, int nshell, double* Dsh, double* mol_dmax,
+                             const int* sh_bf0, const int* sh_nbf, int nshell, double* Dsh, double* mol_dmax, int* ctr, int nctr,
                              hipStream_t st);
 hipError_t launch_block_symmetrize(int nmol, const int4* blocks, int N, const double* G, double* out,
                                    hipStream_t st);
-hipError_t launch_shell_block_max(int nshell, const int* sh_bf0, const int* sh_nbf, int N, const double* absD,
-                                  double* Dsh, hipStream_t st);
+hipError_t launch_fock_prep(int N, const double* dP, double* absD, double* G, const int* sh_bf0, const int* sh_nbf,
+                            int nshell, double* Dsh, int* ctr, int nctr, hipStream_t st);
 hipError_t launch_count_prims(const int2* surv, const int* count, const ShellPair* pairs, unsigned long long* out,
                               hipStream_t st);
 hipError_t launch_fill(size_t n, double* x, double v, hipStream_t st);
 hipError_t launch_fill_int(int n, int* x, int v, hipStream_t st);
-hipError_t launch_symmetrize(int N, const double* G, double* out, hipStream_t st);
+hipError_t launch_symmetrize(int N, const double* G, double* out, hipStream_t st, const int* report = nullptr,
+                             int* host_report = nullptr, int nreport = 0);
 hipError_t launch_sqrt_clamped(size_t n, const double* x, double* y, hipStream_t st);
 hipError_t launch_jk_tensor(int N, const double* T, const double* Pre, const double* Pim, double* Jre,
                             double* Jim, double* Kre, double* Kim, hipStream_t st);

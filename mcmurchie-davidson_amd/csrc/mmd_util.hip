@@ -818,25 +818,36 @@ hipError_t launch_abs_density(int n, const double* Dre, const double* Dim, doubl
     return hipGetLastError();
 }
 
-__global__ void shell_block_max_kernel(int nshell, const int* __restrict__ bf0, const int* __restrict__ nbf, int N,
-                                       const double* __restrict__ absD, double* __restrict__ Dsh)
+// What a symmetrised build of one molecule needs before its first class
+// kernel: |dP|, its maxima by shell block, G and the counters (nctr words)
+// cleared.  One launch: as six (4 to 5 us each, one after the other) they took
+// a sixth of the build of a small molecule.
+__global__ void __launch_bounds__(256) fock_prep_kernel(int N, const double* __restrict__ dP, double* __restrict__ absD,
+                                                        double* __restrict__ G, const int* __restrict__ bf0,
+                                                        const int* __restrict__ nbf, int nshell,
+                                                        double* __restrict__ Dsh, int* __restrict__ ctr, int nctr)
 {
-    const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= nshell * nshell) return;
-    const int s1 = idx / nshell, s2 = idx % nshell;
-    double m = 0.0;
-    for (int i = 0; i < nbf[s1]; ++i)
-        for (int j = 0; j < nbf[s2]; ++j) m = fmax(m, absD[(size_t)(bf0[s1] + i) * N + bf0[s2] + j]);
-    Dsh[idx] = m;
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < (int64_t)N * N) {
+        absD[i] = fabs(dP[i]);
+        G[i] = 0.0;
+    }
+    if (i < nctr) ctr[i] = 0;
+    if (i < (int64_t)nshell * nshell) {
+        const int s1 = (int)(i / nshell), s2 = (int)(i - (int64_t)s1 * nshell);
+        double m = 0.0;
+        for (int x = 0; x < nbf[s1]; ++x)
+            for (int y = 0; y < nbf[s2]; ++y) m = fmax(m, fabs(dP[(size_t)(bf0[s1] + x) * N + bf0[s2] + y]));
+        Dsh[i] = m;
+    }
 }
 
-hipError_t launch_shell_block_max(int nshell, const int* sh_bf0, const int* sh_nbf, int N, const double* absD,
-                                  double* Dsh, hipStream_t st)
+hipError_t launch_fock_prep(int N, const double* dP, double* absD, double* G, const int* sh_bf0, const int* sh_nbf,
+                            int nshell, double* Dsh, int* ctr, int nctr, hipStream_t st)
 {
-    const int n = nshell * nshell;
-    if (n <= 0) return hipSuccess;
-    hipLaunchKernelGGL(shell_block_max_kernel, dim3((n + 255) / 256), dim3(256), 0, st, nshell, sh_bf0, sh_nbf, N,
-                       absD, Dsh);
+    const int64_t n = std::max<int64_t>((int64_t)N * N, nctr);   // no more shells than functions
+    hipLaunchKernelGGL(fock_prep_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, N, dP, absD, G, sh_bf0,
+                       sh_nbf, nshell, Dsh, ctr, nctr);
     return hipGetLastError();
 }
 
@@ -911,18 +922,25 @@ hipError_t launch_fill_int(int n, int* x, int v, hipStream_t st)
     return hipGetLastError();
 }
 
-__global__ void symmetrize_kernel(int N, const double* __restrict__ G, double* __restrict__ out)
+// report, host_report: nreport words copied to pinned host memory by the way,
+// which saves the build's counters a copy of their own.
+__global__ void symmetrize_kernel(int N, const double* __restrict__ G, double* __restrict__ out,
+                                  const int* __restrict__ report, int* __restrict__ host_report, int nreport)
 {
     const int idx = blockIdx.x * blockDim.x + threadIdx.x;
+    if (blockIdx.x == 0)
+        for (int i = threadIdx.x; i < nreport; i += blockDim.x) host_report[i] = report[i];
     if (idx >= N * N) return;
     const int i = idx / N, j = idx % N;
     out[idx] = 0.5 * (G[(size_t)i * N + j] + G[(size_t)j * N + i]);
 }
 
-hipError_t launch_symmetrize(int N, const double* G, double* out, hipStream_t st)
+hipError_t launch_symmetrize(int N, const double* G, double* out, hipStream_t st, const int* report, int* host_report,
+                             int nreport)
 {
     if (N <= 0) return hipSuccess;
-    hipLaunchKernelGGL(symmetrize_kernel, dim3((N * N + 255) / 256), dim3(256), 0, st, N, G, out);
+    hipLaunchKernelGGL(symmetrize_kernel, dim3((N * N + 255) / 256), dim3(256), 0, st, N, G, out, report,
+                       host_report, nreport);
     return hipGetLastError();
 }
 
@@ -934,9 +952,12 @@ __global__ void __launch_bounds__(256) block_prep_kernel(const int4* __restrict_
                                                          const double* __restrict__ dP, double* __restrict__ absD,
                                                          double* __restrict__ G, const int* __restrict__ bf0,
                                                          const int* __restrict__ nbf, int nshell,
-                                                         double* __restrict__ Dsh, double* __restrict__ mol_dmax)
+                                                         double* __restrict__ Dsh, double* __restrict__ mol_dmax,
+                                                         int* __restrict__ ctr, int nctr)
 {
     __shared__ double red[4];
+    if (blockIdx.x == 0)
+        for (int i = threadIdx.x; i < nctr; i += blockDim.x) ctr[i] = 0;
     const int4 b = blocks[blockIdx.x];
     const int f0 = b.x, n = b.y, s0 = b.z, ns = b.w - b.z;
     double mx = 0.0;
@@ -961,12 +982,12 @@ __global__ void __launch_bounds__(256) block_prep_kernel(const int4* __restrict_
 }
 
 hipError_t launch_block_prep(int nmol, const int4* blocks, int N, const double* dP, double* absD, double* G,
-                             const int* sh_bf0, const int* sh_nbf, int nshell, double* Dsh, double* mol_dmax,
-                             hipStream_t st)
+                             const int* sh_bf0, const int* sh_nbf, int nshell, double* Dsh, double* mol_dmax, int* ctr,
+                             int nctr, hipStream_t st)
 {
     if (nmol <= 0) return hipSuccess;
     hipLaunchKernelGGL(block_prep_kernel, dim3(nmol), dim3(256), 0, st, blocks, N, dP, absD, G, sh_bf0, sh_nbf,
-                       nshell, Dsh, mol_dmax);
+                       nshell, Dsh, mol_dmax, ctr, nctr);
     return hipGetLastError();
 }
 
