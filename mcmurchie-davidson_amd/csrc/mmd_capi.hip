@@ -111,10 +111,12 @@ constexpr int NPRIM_SLOTS = 4 * NQCLASS;   // survivor counters of one Fock buil
 struct FockCounters {
     unsigned long long nprim[NPRIM_SLOTS];   // see FockScratch::nprim
     int count[2 * NQCLASS];                  // survivor-list lengths (FP64 lists, then FP32)
-    int rowctr[2 * NQCLASS];
+    int nlive[NQCLASS];                      // live units of a batch's classes
+    int pad[ROW_QUEUE_PAD];
+    int rowctr[2 * NQCLASS][ROW_QUEUES * ROW_QUEUE_PAD];   // unit queues, FP64 then FP32 pass
 };
 constexpr int FOCK_COUNTER_WORDS = (int)(sizeof(FockCounters) / sizeof(int));
-constexpr int FOCK_REPORT_WORDS = (int)(offsetof(FockCounters, rowctr) / sizeof(int));
+constexpr int FOCK_REPORT_WORDS = (int)(offsetof(FockCounters, nlive) / sizeof(int));
 
 // Per-class sums over profiled builds; index 0 the FP64 launches, 1 the FP32 tier.
 struct ProfileSum {
@@ -281,6 +283,7 @@ struct mmd_ctx {
     // length unit_seg[qc].
     DevBuf<int4> d_units;
     DevBuf<UnitBound> d_ubound;         // per unit, in the same order
+    DevBuf<int> d_live;
     int64_t unit_off[NQCLASS + 1] = {0};
     int unit_seg[NQCLASS] = {0};
     bool units_ok = false;
@@ -611,6 +614,7 @@ int build_pairs(mmd_ctx* c, const double* diag)
         c->unit_off[NQCLASS] = units;
         HIP_TRY(c->d_units.reserve(std::max<size_t>(1, (size_t)units)));
         HIP_TRY(c->d_ubound.reserve(std::max<size_t>(1, (size_t)units)));
+        if (c->nmol > 1) HIP_TRY(c->d_live.reserve(std::max<size_t>(1, (size_t)units)));
         HIP_TRY(launch_unit_scatter(U, d_hist, c->w_q.p, c->d_units.p, c->d_ubound.p, c->st));
         c->units_ok = true;
     }
@@ -723,8 +727,9 @@ ClassArgs base_args(mmd_ctx* c)
 // kernel (class qc at surv + surv_off[qc]).  The context's buffers, or a
 // caller-free static array (mmd_fock_delta_noalloc).
 struct FockScratch {
-    int* rowctr = nullptr;                 // cleared, with the others, by the build's preparation kernel
+    int (*rowctr)[ROW_QUEUES * ROW_QUEUE_PAD] = nullptr;   // cleared, with the others, by the build's preparation kernel
     int* count = nullptr;
+    const int* nlive = nullptr;
     // NPRIM_SLOTS counters: primitive quartets (FP64 tier), shell quartets of
     // the row kernels (FP64, FP32 tier), primitive quartets (FP32 tier)
     unsigned long long* nprim = nullptr;
@@ -733,9 +738,10 @@ struct FockScratch {
         rowctr = c->rowctr;
         count = c->count;
         nprim = c->nprim;
+        nlive = c->nlive;
     }
     double* Dsh = nullptr;                 // nshell^2
-    const double* mol_dmax = nullptr;      // batches: per-molecule max |dP| (units of molecules at 0 skipped)
+    const int* live = nullptr;             // batches: the build's live units (launch_unit_live)
     int2* surv = nullptr;
     int64_t surv_off[NQCLASS] = {0};       // survivor lists, packed: wave classes only
     int64_t surv_cap = -1;                 // entries available at surv; < 0: grow the context's buffer
@@ -860,8 +866,9 @@ int run_fock_classes(mmd_ctx* c, ClassArgs A, double tol, FockScratch& W0)
             R.tri = pcb == pck ? 1 : 0;
             R.nshell = (int)c->shells.size();
             R.Dsh = W0.Dsh;
-            R.mol_dmax = W0.mol_dmax;
-            R.row_counter = W0.rowctr + qc;
+            R.live = W0.live ? W0.live + c->unit_off[qc] : nullptr;
+            R.nlive = W0.nlive + qc;
+            R.row_counter = W0.rowctr[qc];
             R.maxpp = maxpp[qc];
             R.kj = kj_lds[qc] ? 1 : 0;
             R.kslice = c->ket_slice[qc];
@@ -873,7 +880,6 @@ int run_fock_classes(mmd_ctx* c, ClassArgs A, double tol, FockScratch& W0)
             R.kstride = c->kpp_stride;
             R.ket_npp = (int)(c->pc_npp[pck] / std::max(1, nk));
             R.units = c->d_units.p + c->unit_off[qc];
-            R.ubound = c->d_ubound.p + c->unit_off[qc];
             const int64_t units = c->unit_off[qc + 1] - c->unit_off[qc];
             R.nunits = (int)units;
             if (units == 0) {
@@ -894,7 +900,7 @@ int run_fock_classes(mmd_ctx* c, ClassArgs A, double tol, FockScratch& W0)
                 // FP32 tier: the same units, quartets with tol <= bound < fp32_below
                 R.tier_lo = 0.0;
                 R.tier_hi = c->fp32_below;
-                R.row_counter = W0.rowctr + NQCLASS + qc;
+                R.row_counter = W0.rowctr[NQCLASS + qc];
                 R.stat_nquart = W0.nprim + 2 * NQCLASS + qc;
                 R.stat_nprim = c->profiling ? W0.nprim + 3 * NQCLASS + qc : nullptr;
                 // the second traversal holds the many small-bound quartets
@@ -1748,8 +1754,7 @@ int mmd_fock_delta_noalloc(mmd_ctx* ctx, const double* dP, double tol, double* G
     off += up(sizeof(double) * nn);
     double* Dsh = reinterpret_cast<double*>(base + off);
     off += up(sizeof(double) * ns * ns);
-    FockCounters* ctr = reinterpret_cast<FockCounters*>(base + off);
-    off += up(sizeof(FockCounters));
+    FockCounters* ctr = ctx->d_ctr.p;   // allocated with the tables
     if (off > NOALLOC_SCRATCH_BYTES)
         return fail(MMD_ERR_ARG, "a basis of %d functions needs %zu bytes of scratch; the limit is %zu", N, off,
                     NOALLOC_SCRATCH_BYTES);
@@ -2028,7 +2033,17 @@ int enqueue_fock_sym(mmd_ctx* c, const double* dP, double tol, double* Gout)
     W.counters(c->d_ctr.p);
     W.profile_events = true;
     W.Dsh = c->d_Dsh.p;
-    W.mol_dmax = blocks ? c->d_mol_dmax.p : nullptr;
+    if (blocks) {
+        UnitLive U;
+        for (int qc = 0; qc <= NQCLASS; ++qc) U.off[qc] = c->unit_off[qc];
+        U.bound = c->d_ubound.p;
+        U.mol_dmax = c->d_mol_dmax.p;
+        U.tol = tol;
+        U.live = c->d_live.p;
+        U.nlive = c->d_ctr.p->nlive;
+        HIP_TRY(launch_unit_live(U, c->st));
+        W.live = c->d_live.p;
+    }
     W.surv = c->d_surv.p;
     W.surv_cap = (int64_t)c->d_surv.n;   // reserved by the caller
     W.allow_measure = false;

@@ -337,15 +337,16 @@ __global__ void __launch_bounds__(CLASS_BLOCK, (row_min_waves<LA, LB, LC, LD, T>
     const int N = A.N;
     const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int nwv = (int)(blockDim.x >> 6);
-    const int nunits = R.nunits;
+    const int nunits = R.live ? *R.nlive : R.nunits;
+    const int nqueue = min(ROW_QUEUES, (int)gridDim.x), queue = (int)blockIdx.x % nqueue;
     const size_t ns = (size_t)R.nshell;
     unsigned long long my_nprim = 0;   // primitive quartets of this lane (statistics)
     for (;;) {
         __syncthreads();
-        if (threadIdx.x == 0) misc[0] = atomicAdd(R.row_counter, 1);
+        if (threadIdx.x == 0) misc[0] = atomicAdd(&R.row_counter[queue * ROW_QUEUE_PAD], 1) * nqueue + queue;
         __syncthreads();
-        const int u = misc[0];
-        if (u >= nunits) {
+        const int iu = misc[0];
+        if (iu >= nunits) {
             if (R.stat_nprim) {   // one atomic per wavefront
                 for (int off = 32; off > 0; off >>= 1) my_nprim += __shfl_xor(my_nprim, off);
                 if (lane == 0 && my_nprim) atomicAdd(R.stat_nprim, my_nprim);
@@ -354,13 +355,7 @@ __global__ void __launch_bounds__(CLASS_BLOCK, (row_min_waves<LA, LB, LC, LD, T>
         }
         // unit: bra pair P, its primitive pairs [ip0, ip1) and the ket
         // pairs [k0, k1) of its molecule
-        // a unit of a batch whose every quartet fails the screen: pair
-        // factors q_P q_Q <= the unit's bound, and the density weight of the
-        // screen is at most 4 max |dP| of the molecule (0 once converged)
-        if (R.mol_dmax) {
-            const UnitBound ub = R.ubound[u];
-            if ((double)ub.q * 4.0 * R.mol_dmax[ub.mol] < 0.999999 * A.tol) continue;
-        }
+        const int u = R.live ? R.live[iu] : iu;
         const int4 U = R.units[u];
         const int P = U.x, k0 = U.z;
         const int ip0u = U.y & 0xffff, ip1u = U.y >> 16;

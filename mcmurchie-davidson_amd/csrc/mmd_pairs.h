@@ -72,4 +72,19 @@ hipError_t launch_unit_count(const UnitInput& I, int* hist, int* counts, double*
 hipError_t launch_unit_scatter(const UnitInput& I, int* hist, const double* qrun, int4* units, UnitBound* bounds,
                                hipStream_t st);
 
+// Of each class's units [off[qc], off[qc + 1]) those that hold a quartet which
+// can pass the screen: pair factors q_P q_Q <= the unit's bound, and density
+// weights at most 4 max |dP| of the molecule (0 once it has converged).  Their
+// class-local numbers, roughly in order, to live + off[qc]; nlive[qc] of them
+// (cleared before).
+struct UnitLive {
+    int64_t off[NQCLASS + 1];
+    const UnitBound* bound;
+    const double* mol_dmax;
+    double tol;
+    int* live;
+    int* nlive;
+};
+hipError_t launch_unit_live(const UnitLive& I, hipStream_t st);
+
 }  // namespace mmd

@@ -438,4 +438,44 @@ hipError_t launch_unit_scatter(const UnitInput& I, int* hist, const double* qrun
     return hipGetLastError();
 }
 
+namespace {
+// One thread per unit, a row of blocks per class.  A row kernel that drew and
+// dropped the dead units itself spent 0.3 of 0.4 ms on them late in a batch's
+// SCF, when most molecules have converged; this pass takes 6 us.
+__global__ void __launch_bounds__(256) unit_live_kernel(UnitLive I)
+{
+    const int qc = blockIdx.y;
+    const int64_t n = I.off[qc + 1] - I.off[qc];
+    const int64_t u = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if ((int64_t)blockIdx.x * blockDim.x >= n) return;
+    __shared__ int base[4], total;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    bool keep = false;
+    if (u < n) {
+        const UnitBound b = I.bound[I.off[qc] + u];
+        keep = !((double)b.q * 4.0 * I.mol_dmax[b.mol] < 0.999999 * I.tol);
+    }
+    const unsigned long long m = __ballot(keep);
+    if (lane == 0) base[wv] = __popcll(m);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const int c = base[0] + base[1] + base[2] + base[3];
+        total = c ? atomicAdd(&I.nlive[qc], c) : 0;
+    }
+    __syncthreads();
+    int pos = total;
+    for (int w = 0; w < wv; ++w) pos += base[w];
+    if (keep) I.live[I.off[qc] + pos + __popcll(m & ((1ull << lane) - 1ull))] = (int)u;
+}
+}  // namespace
+
+hipError_t launch_unit_live(const UnitLive& I, hipStream_t st)
+{
+    int64_t most = 0;
+    for (int qc = 0; qc < NQCLASS; ++qc) most = I.off[qc + 1] - I.off[qc] > most ? I.off[qc + 1] - I.off[qc] : most;
+    if (most == 0) return hipSuccess;
+    hipLaunchKernelGGL(unit_live_kernel, dim3((unsigned)((most + 255) / 256), NQCLASS), dim3(256), 0, st, I);
+    return hipGetLastError();
+}
+
 }  // namespace mmd

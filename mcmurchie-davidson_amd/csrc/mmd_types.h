@@ -88,6 +88,14 @@ struct UnitBound {
     int32_t mol;
 };
 
+// Queues of work units per class: workgroup b draws from queue b % ROW_QUEUES,
+// which holds every ROW_QUEUES-th unit of the list (costs are sorted, so the
+// queues are alike).  One counter served a draw every 11 to 13 ns whoever
+// asked, 300 us for the (ps|ss) and (ss|ss) units of a 45-molecule batch;
+// counters in cache lines of their own are served side by side.
+constexpr int ROW_QUEUES = 8;
+constexpr int ROW_QUEUE_PAD = 32;      // ints: 128 bytes
+
 struct RowArgs {
     int boff, nb;               // bra pairs of the class: pairs[boff .. boff+nb)
     int koff, nk;               // ket pairs of the class
@@ -101,10 +109,10 @@ struct RowArgs {
     int kslice;                 // ket primitive pairs per lane item of the sliced classes (1 .. 16)
     int nshell;
     const double* Dsh;          // shell-block maxima of |dP| (nshell x nshell)
-    const double* mol_dmax;     // batches: max |dP| of each molecule; or null
-    const UnitBound* ubound;    // with mol_dmax: units with 4 q max|dP| < tol are skipped
+    const int* live;            // batches: the units that this build's density leaves alive; or null for all
+    const int* nlive;           // their number
     double tier_lo, tier_hi;    // this launch takes quartets with tier_lo <= bound < tier_hi
-    int* row_counter;           // next work unit (zeroed before the launch)
+    int* row_counter;           // ROW_QUEUES counters, ROW_QUEUE_PAD apart (zeroed before the launch)
     unsigned long long* stat_nquart;   // optional statistics
     unsigned long long* stat_nprim;
     const KetScreen* kscr;      // all pairs

@@ -956,8 +956,7 @@ __global__ void __launch_bounds__(256) block_prep_kernel(const int4* __restrict_
                                                          int* __restrict__ ctr, int nctr)
 {
     __shared__ double red[4];
-    if (blockIdx.x == 0)
-        for (int i = threadIdx.x; i < nctr; i += blockDim.x) ctr[i] = 0;
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < nctr; i += gridDim.x * blockDim.x) ctr[i] = 0;
     const int4 b = blocks[blockIdx.x];
     const int f0 = b.x, n = b.y, s0 = b.z, ns = b.w - b.z;
     double mx = 0.0;
