@@ -582,6 +582,14 @@ int build_pairs(mmd_ctx* c, const double* diag)
         // more than they gain when classes or molecules share the GPU.)
         int seg = 4096;
         while (seg > 256 && c->qc_total[qc] / std::max(1, c->nmol) / seg < 4096) seg /= 2;
+        // One small molecule leaves most of the GPU idle, and a class lasts as
+        // long as its longest unit: segments of down to 32 kets until the
+        // class has about 512.  (H2O)2, 3 and 5 in 6-31G, 6-31G* and 6-31G
+        // 158, 423 and 239 us per build without, 137, 356 and 204 with; more
+        // units cost more than they gain ((H2O)5 204, 234, 256, 296 us for
+        // 512, 1024, 2048, 4096; (H2O)8 cc-pVDZ 1.76, 1.88, 2.07, 2.37 ms).
+        if (c->nmol == 1)
+            while (seg > 32 && c->qc_total[qc] / seg < 512) seg /= 2;
         c->unit_seg[qc] = U.seg[qc] = seg;
     }
     HIP_TRY(launch_pair_sort(I, W, c->d_pairs.p, reinterpret_cast<PairStats*>(c->w_ints.p), c->st));

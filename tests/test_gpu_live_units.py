@@ -2,7 +2,10 @@
 units than queues or than a wavefront, more than one block of the list, and
 molecules that converge many iterations before the others, so that most units
 of the late builds are dead.  Every energy within 1e-9 Eh of the molecule's
-own run, as for any batch, with the same number of iterations."""
+own run, as for any batch.  Both converge to ||dP|| < 1e-10 and iteration
+counts are not compared: the DIIS equations of two electrons are singular, so
+that H2's runs at 1e-8 end after 10 to 13 iterations and 2e-9 Eh apart from
+one call to the next, with or without a batch."""
 import pytest
 
 from geometries import H2, HELIUM, WATER, water_cluster
@@ -17,12 +20,11 @@ BIG = water_cluster(5, 9.0, seed=8, perturb=True)
 def test_units_of_live_molecules(geoms, basis):
     from mmd.batch import run_batch_device
     from mmd.molecule import Molecule
-    res = run_batch_device(geoms, basis, group=len(geoms))
+    res = run_batch_device(geoms, basis, group=len(geoms), conver=1e-10)
     for g, r in zip(geoms, res):
         m = Molecule(g, basis)
-        m.RHF(doPrint=False, direct=True)
+        m.RHF(doPrint=False, direct=True, conver=1e-10)
         print("%d functions: batch %.10f (%d it)  single %.10f (%d it)" % (r["nbasis"], r["energy"], r["iterations"],
                                                                           m.energy.real, m.iterations))
         assert r["converged"] and m.is_converged
         assert abs(r["energy"] - m.energy.real) < 1e-9
-        assert r["iterations"] == m.iterations
