@@ -886,7 +886,6 @@ int run_fock_classes(mmd_ctx* c, ClassArgs A, double tol, FockScratch& W0)
             R.kref = c->d_kref.p;
             R.kpp = c->d_kpp.p;
             R.kstride = c->kpp_stride;
-            R.ket_npp = (int)(c->pc_npp[pck] / std::max(1, nk));
             R.units = c->d_units.p + c->unit_off[qc];
             const int64_t units = c->unit_off[qc + 1] - c->unit_off[qc];
             R.nunits = (int)units;
@@ -1081,7 +1080,10 @@ int mmd_ctx_create(mmd_ctx** out, int device_id)
     c->max_lds_device = c->max_lds;
     if (lds_max > 0) c->lds_per_block = (size_t)lds_max;
     hipError_t e = hipStreamCreateWithFlags(&c->st, hipStreamNonBlocking);
-    if (e == hipSuccess) e = hipHostMalloc((void**)&c->h_ctr, sizeof(FockCounters), hipHostMallocDefault);
+    if (e == hipSuccess) {
+        std::lock_guard<std::recursive_mutex> lk(device_alloc_mutex());
+        e = hipHostMalloc((void**)&c->h_ctr, sizeof(FockCounters), hipHostMallocDefault);
+    }
     if (e == hipSuccess) e = hipEventCreate(&c->ev0);
     if (e == hipSuccess) e = hipEventCreate(&c->ev1);
     if (e == hipSuccess) e = hipEventCreateWithFlags(&c->evfork, hipEventDisableTiming);

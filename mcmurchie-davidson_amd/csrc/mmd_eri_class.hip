@@ -22,15 +22,8 @@ hipError_t MMD_NAME(fock_class_launch_, QC_LA, QC_LB, QC_LC, QC_LD, QC_SUFFIX)(c
                                                                                int grid, hipStream_t st)
 {
     const size_t lds = fock_class_lds_bytes<QC_LA, QC_LB, QC_LC, QC_LD, QC_T>(R.rw, R.maxpp, R.kj);
-    if constexpr (row_has_ku2<QC_LA, QC_LB, QC_LC, QC_LD>()) {
-        if (R.ket_npp >= KU_MIN_NPP) {
-            hipLaunchKernelGGL((eri_fock_class_kernel<QC_LA, QC_LB, QC_LC, QC_LD, 2, QC_T>), dim3(grid),
-                               dim3(CLASS_BLOCK), lds, st, A, R);
-            return hipGetLastError();
-        }
-    }
-    hipLaunchKernelGGL((eri_fock_class_kernel<QC_LA, QC_LB, QC_LC, QC_LD, 1, QC_T>), dim3(grid), dim3(CLASS_BLOCK),
-                       lds, st, A, R);
+    hipLaunchKernelGGL((eri_fock_class_kernel<QC_LA, QC_LB, QC_LC, QC_LD, QC_T>), dim3(grid), dim3(CLASS_BLOCK), lds,
+                       st, A, R);
     return hipGetLastError();
 }
 

@@ -120,10 +120,7 @@ struct KetArrays {
     __device__ __forceinline__ double operator()(int i, KetField f) const { return p[f * stride + i]; }
 };
 
-// KU ket primitive pairs are taken at a time, as independent chains that hide
-// each other's latency and share the bra reads (the last ones repeat a pair
-// with no weight).
-template <int LA, int LB, int LC, int LD, int A0, int A1, int KU, typename T, class KET>
+template <int LA, int LB, int LC, int LD, int A0, int A1, typename T, class KET>
 __device__ __forceinline__ void quartet_compute(const KET& Q, const T* lds, const T* bp, int ip0, int ip1, int jq0,
                                                 int jq1, T* acc)
 {
@@ -134,32 +131,23 @@ __device__ __forceinline__ void quartet_compute(const KET& Q, const T* lds, cons
     constexpr int HCD = S::HCD;
     sfor<NCH * NCD>([&](auto k) { acc[k] = T(0); });
 
-    for (int jq = jq0; jq < jq1; jq += KU) {
-        T Qp[KU], QK[KU], Qx[KU], Qy[KU], Qz[KU], V[KU][HCD * NCH];
-        sfor<KU>([&](auto u) {
-            const int j = KU == 1 ? jq : min(jq + (int)u, jq1 - 1);
-            Qp[u] = (T)Q(j, KF_P);
-            QK[u] = (T)Q(j, KF_KQ);
-            Qx[u] = (T)Q(j, KF_X);
-            Qy[u] = (T)Q(j, KF_Y);
-            Qz[u] = (T)Q(j, KF_Z);
-            if (KU > 1 && jq + (int)u >= jq1) QK[u] = T(0);
-            sfor<HCD * NCH>([&](auto k) { V[u][k] = T(0); });
-        });
+    for (int jq = jq0; jq < jq1; ++jq) {
+        const T Qp = (T)Q(jq, KF_P), QK = (T)Q(jq, KF_KQ), Qx = (T)Q(jq, KF_X), Qy = (T)Q(jq, KF_Y),
+                Qz = (T)Q(jq, KF_Z);
+        T V[HCD * NCH];
+        sfor<HCD * NCH>([&](auto k) { V[k] = T(0); });
         for (int ip = ip0; ip < ip1; ++ip) {
             const T* b = bp + ip * S::BPS;
-            T R[KU][nherm(L)];
-            sfor<KU>([&](auto u) {
-                const T Pp = b[0];
-                const T rs = dev_rsqrt(Pp + Qp[u]);
-                const T alpha = Pp * Qp[u] * rs * rs;
-                const T X = b[2] - Qx[u], Y = b[3] - Qy[u], Z = b[4] - Qz[u];
-                const T Targ = alpha * (X * X + Y * Y + Z * Z);
-                const T pref = b[1] * QK[u] * rs;   // 2 pi^{5/2} / (p q sqrt(p+q)) K_ab K_cd
-                T F[L + 1];
-                boys_seeds<L, T>(Targ, alpha, pref, lds, F);
-                hermite_R<L, T>(X, Y, Z, F, R[u]);
-            });
+            const T Pp = b[0];
+            const T rs = dev_rsqrt(Pp + Qp);
+            const T alpha = Pp * Qp * rs * rs;
+            const T X = b[2] - Qx, Y = b[3] - Qy, Z = b[4] - Qz;
+            const T Targ = alpha * (X * X + Y * Y + Z * Z);
+            const T pref = b[1] * QK * rs;   // 2 pi^{5/2} / (p q sqrt(p+q)) K_ab K_cd
+            T F[L + 1];
+            boys_seeds<L, T>(Targ, alpha, pref, lds, F);
+            T R[nherm(L)];
+            hermite_R<L, T>(X, Y, Z, F, R);
             const T* Ebx = b + 8;
             const T* Eby = b + 8 + S::EB;
             const T* Ebz = b + 8 + 2 * S::EB;
@@ -173,7 +161,7 @@ __device__ __forceinline__ void quartet_compute(const KET& Q, const T* lds, cons
                 constexpr int iz = (az * (LB + 1) + bz) * S::NTB;
                 sfor<HCD>([&](auto ik) {
                     constexpr Herm3 h = hdecode(decltype(ik)::value);
-                    constexpr int iv = decltype(ik)::value * NCH + decltype(ii)::value;
+                    T v = V[decltype(ik)::value * NCH + decltype(ii)::value];
                     sfor<ax + bx + 1>([&](auto it) {
                         constexpr int t = decltype(it)::value;
                         sfor<ay + by + 1>([&](auto iu) {
@@ -181,53 +169,47 @@ __device__ __forceinline__ void quartet_compute(const KET& Q, const T* lds, cons
                             const T exy = Ebx[ix + t] * Eby[iy + u];
                             sfor<az + bz + 1>([&](auto iw) {
                                 constexpr int w = decltype(iw)::value;
-                                const T e = exy * Ebz[iz + w];
-                                sfor<KU>([&](auto k) {
-                                    V[k][iv] = fma(e, R[k][hidx(t + h.t, u + h.u, w + h.v)], V[k][iv]);
-                                });
+                                v = fma(exy * Ebz[iz + w], R[hidx(t + h.t, u + h.u, w + h.v)], v);
                             });
                         });
                     });
+                    V[decltype(ik)::value * NCH + decltype(ii)::value] = v;
                 });
             });
         }
         // ket expansion, once per ket primitive pair
-        sfor<KU>([&](auto ku) {
-            const int j = KU == 1 ? jq : min(jq + (int)ku, jq1 - 1);
-            T Ekx[(LC + 1) * (LD + 1) * S::NTK], Eky[(LC + 1) * (LD + 1) * S::NTK],
-                Ekz[(LC + 1) * (LD + 1) * S::NTK];
-            if constexpr (LC + LD > 0) {
-                const T qinv2 = (T)Q(j, KF_INV2P);
-                hermite_E<LC, LD, -1, T>(qinv2, (T)Q(j, KF_PAX), (T)Q(j, KF_PBX), Ekx);
-                hermite_E<LC, LD, -1, T>(qinv2, (T)Q(j, KF_PAY), (T)Q(j, KF_PBY), Eky);
-                hermite_E<LC, LD, -1, T>(qinv2, (T)Q(j, KF_PAZ), (T)Q(j, KF_PBZ), Ekz);
-            } else {
-                Ekx[0] = Eky[0] = Ekz[0] = T(1);
-            }
-            sfor<NCD>([&](auto icd) {
-                constexpr int cd = decltype(icd)::value;
-                constexpr int c = cd / S::ND, d = cd % S::ND;
-                constexpr int cx = comp_lx(LC, c), cy = comp_ly(LC, c), cz = comp_lz(LC, c);
-                constexpr int dx = comp_lx(LD, d), dy = comp_ly(LD, d), dz = comp_lz(LD, d);
-                constexpr int kx = (cx * (LD + 1) + dx) * S::NTK;
-                constexpr int ky = (cy * (LD + 1) + dy) * S::NTK;
-                constexpr int kz = (cz * (LD + 1) + dz) * S::NTK;
-                sfor<NCH>([&](auto ii) {
-                    T sacc = acc[decltype(ii)::value * NCD + cd];
-                    sfor<cx + dx + 1>([&](auto itau) {
-                        constexpr int tau = decltype(itau)::value;
-                        sfor<cy + dy + 1>([&](auto inu) {
-                            constexpr int nu = decltype(inu)::value;
-                            const T exy = Ekx[kx + tau] * Eky[ky + nu];
-                            sfor<cz + dz + 1>([&](auto iphi) {
-                                constexpr int phi = decltype(iphi)::value;
-                                sacc = fma(exy * Ekz[kz + phi],
-                                           V[ku][hidx(tau, nu, phi) * NCH + decltype(ii)::value], sacc);
-                            });
+        T Ekx[(LC + 1) * (LD + 1) * S::NTK], Eky[(LC + 1) * (LD + 1) * S::NTK],
+            Ekz[(LC + 1) * (LD + 1) * S::NTK];
+        if constexpr (LC + LD > 0) {
+            const T qinv2 = (T)Q(jq, KF_INV2P);
+            hermite_E<LC, LD, -1, T>(qinv2, (T)Q(jq, KF_PAX), (T)Q(jq, KF_PBX), Ekx);
+            hermite_E<LC, LD, -1, T>(qinv2, (T)Q(jq, KF_PAY), (T)Q(jq, KF_PBY), Eky);
+            hermite_E<LC, LD, -1, T>(qinv2, (T)Q(jq, KF_PAZ), (T)Q(jq, KF_PBZ), Ekz);
+        } else {
+            Ekx[0] = Eky[0] = Ekz[0] = T(1);
+        }
+        sfor<NCD>([&](auto icd) {
+            constexpr int cd = decltype(icd)::value;
+            constexpr int c = cd / S::ND, d = cd % S::ND;
+            constexpr int cx = comp_lx(LC, c), cy = comp_ly(LC, c), cz = comp_lz(LC, c);
+            constexpr int dx = comp_lx(LD, d), dy = comp_ly(LD, d), dz = comp_lz(LD, d);
+            constexpr int kx = (cx * (LD + 1) + dx) * S::NTK;
+            constexpr int ky = (cy * (LD + 1) + dy) * S::NTK;
+            constexpr int kz = (cz * (LD + 1) + dz) * S::NTK;
+            sfor<NCH>([&](auto ii) {
+                T sacc = acc[decltype(ii)::value * NCD + cd];
+                sfor<cx + dx + 1>([&](auto itau) {
+                    constexpr int tau = decltype(itau)::value;
+                    sfor<cy + dy + 1>([&](auto inu) {
+                        constexpr int nu = decltype(inu)::value;
+                        const T exy = Ekx[kx + tau] * Eky[ky + nu];
+                        sfor<cz + dz + 1>([&](auto iphi) {
+                            constexpr int phi = decltype(iphi)::value;
+                            sacc = fma(exy * Ekz[kz + phi], V[hidx(tau, nu, phi) * NCH + decltype(ii)::value], sacc);
                         });
                     });
-                    acc[decltype(ii)::value * NCD + cd] = sacc;
                 });
+                acc[decltype(ii)::value * NCD + cd] = sacc;
             });
         });
     }

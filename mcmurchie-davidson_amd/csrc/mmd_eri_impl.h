@@ -244,8 +244,8 @@ __device__ __forceinline__ void quartet_digest(const ClassArgs& A, int2 qd, cons
 // ---------------------------------------------------------------------------
 // Class kernel.  A work unit is one bra shell pair ("row"), a slice of at
 // most PSLICE of its primitive pairs and a segment of its ket pairs (a
-// host-built table, heaviest first); workgroups take units from a device
-// counter.  The unit's ket pairs are screened a workgroup at a time;
+// table built at set-up, heaviest first); workgroups draw units from the
+// queues of ROW_QUEUES.  The unit's ket pairs are screened a workgroup at a time;
 // survivors are appended to an LDS list that is digested whenever it holds
 // a full batch, as wave items of (bra-component chunk, 64 consecutive
 // (ket primitive slice, quartet) lane items).  Classes with an integral
@@ -269,20 +269,6 @@ struct ClassList {
     static constexpr int QLIST = QB + CLASS_BLOCK;   // batch + one screening step
 };
 
-// Classes built in two forms: one ket primitive pair at a time, and two at a
-// time (KU) where kets are heavily contracted.  Only (ss) kets gain: at
-// (H2O)16 cc-pVDZ two at a time took (ss|ss) 0.77 -> 0.74, (ps|ss) 1.69 ->
-// 1.57, (pp|ss) 0.96 -> 0.82, (ds|ss) 0.70 -> 0.60 ms, while for the shorter
-// 6-31G kets of a batch (ps|ss) lost 10% and (pp|ss) 4% to the weightless
-// chains.  The launch takes two for an average of at least KU_MIN_NPP
-// primitive pairs per (ss) pair (6-31G water about 6, cc-pVDZ 12).
-constexpr int KU_MIN_NPP = 9;
-template <int LA, int LB, int LC, int LD>
-constexpr bool row_has_ku2()
-{
-    return LC + LD == 0 && LA + LB <= 2;
-}
-
 // Least wavefronts per SIMD that the compiler plans the registers for.  The
 // row kernels wait more than they compute (at (H2O)16 cc-pVDZ the vector
 // units are busy 30% of the time), so a second or third wavefront pays where
@@ -301,7 +287,7 @@ constexpr int row_min_waves()
 
 // T is the arithmetic type of the integrals (double, or float for the
 // FP32 tier); screening, digestion and all accumulation into G are FP64.
-template <int LA, int LB, int LC, int LD, int KU, typename T>
+template <int LA, int LB, int LC, int LD, typename T>
 __global__ void __launch_bounds__(CLASS_BLOCK, (row_min_waves<LA, LB, LC, LD, T>())) eri_fock_class_kernel(ClassArgs A, RowArgs R)
 {
     using S = ClassShape<LA, LB, LC, LD>;
@@ -452,7 +438,7 @@ __global__ void __launch_bounds__(CLASS_BLOCK, (row_min_waves<LA, LB, LC, LD, T>
                         constexpr int C = decltype(ic)::value;
                         constexpr int A0 = C * S::CH, A1 = (C + 1) * S::CH;
                         T acc[(A1 - A0) * S::NCD];
-                        quartet_compute<LA, LB, LC, LD, A0, A1, KU, T>(KetArrays{R.kpp, R.kstride}, boys_tab, bp, ip0, ip1,
+                        quartet_compute<LA, LB, LC, LD, A0, A1, T>(KetArrays{R.kpp, R.kstride}, boys_tab, bp, ip0, ip1,
                                                                    ket.pp0 + jq0, ket.pp0 + jq1, acc);
                         if constexpr (S::IBUF) {
                             double* dst = ibuf + (size_t)idx * S::NABCD + A0 * S::NCD;

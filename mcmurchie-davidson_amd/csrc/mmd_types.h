@@ -119,7 +119,6 @@ struct RowArgs {
     const KetRef* kref;
     const double* kpp;          // field f of primitive pair i at kpp[f * kstride + i]
     int64_t kstride;
-    int ket_npp;                // average primitive pairs per ket pair of the class
 };
 
 // Work of one quartet class of the integral-block kernels: the stored tensor

@@ -1,10 +1,8 @@
-"""Forms of the row kernels: one ket primitive pair at a time or two, which is
-taken by the average contraction of the (ss) pairs (6-31G below the line,
-cc-pVDZ above it, STO-3G's nine at it), over ket slices of one, an odd number
-and all primitive pairs, so that the second of two chains is sometimes without
-a pair.  The symmetrised build against the per-function kernels (functions in
-reversed order form no whole shells); both sum at most 1e6 FP64 terms: 1e-11
-of max |G|."""
+"""Ket slices of the row kernels' tables: slices of one, an odd number and all
+primitive pairs of a ket, so that the last slice of a ket is short, for bases
+of short (6-31G) and long (cc-pVDZ) contractions.  The symmetrised build
+against the per-function kernels (functions in reversed order form no whole
+shells); both sum at most 1e6 FP64 terms: 1e-11 of max |G|."""
 import numpy as np
 import pytest
 
@@ -15,7 +13,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("basis", ["sto-3g", "6-31g", "cc-pvdz"])
 @pytest.mark.parametrize("kslice", [1, 2, 3, 16])
-def test_ket_chains(basis, kslice):
+def test_ket_slices(basis, kslice):
     from mmd import _native
     from mmd.molecule import Molecule
     mol = Molecule(water_cluster(2, 5.0, seed=4, perturb=True), basis)
