@@ -43,19 +43,19 @@ FP64_PEAK_TFLOPS = 78.6
 # counters read for a copy of known size (recorded with the command lines in
 # profiles/); a class absent here reports null.
 TRAFFIC = {
-    (0, 0, 0, 0): 2.203e+07, (1, 0, 0, 0): 4.100e+07, (1, 0, 1, 0): 4.481e+07, (1, 1, 0, 0): 2.065e+07,
-    (1, 1, 1, 0): 5.334e+07, (1, 1, 1, 1): 7.910e+06, (2, 0, 0, 0): 1.781e+07, (2, 0, 1, 0): 3.797e+07,
-    (2, 0, 1, 1): 1.138e+07, (2, 0, 2, 0): 6.591e+06, (2, 1, 0, 0): 1.420e+07, (2, 1, 1, 0): 1.657e+07,
-    (2, 1, 1, 1): 7.255e+06, (2, 1, 2, 0): 5.512e+06, (2, 1, 2, 1): 5.707e+06, (2, 2, 0, 0): 3.591e+06,
-    (2, 2, 1, 0): 4.837e+06, (2, 2, 1, 1): 2.786e+06, (2, 2, 2, 0): 2.254e+06, (2, 2, 2, 1): 5.863e+06,
-    (2, 2, 2, 2): 1.207e+06,
+    (0, 0, 0, 0): 1.952e+07, (1, 0, 0, 0): 3.600e+07, (1, 0, 1, 0): 4.309e+07, (1, 1, 0, 0): 1.616e+07,
+    (1, 1, 1, 0): 5.139e+07, (1, 1, 1, 1): 1.611e+07, (2, 0, 0, 0): 1.493e+07, (2, 0, 1, 0): 3.540e+07,
+    (2, 0, 1, 1): 1.892e+07, (2, 0, 2, 0): 9.296e+06, (2, 1, 0, 0): 1.075e+07, (2, 1, 1, 0): 1.506e+07,
+    (2, 1, 1, 1): 7.276e+06, (2, 1, 2, 0): 7.332e+06, (2, 1, 2, 1): 7.053e+06, (2, 2, 0, 0): 5.347e+06,
+    (2, 2, 1, 0): 7.271e+06, (2, 2, 1, 1): 5.876e+06, (2, 2, 2, 0): 4.760e+06, (2, 2, 2, 1): 9.041e+06,
+    (2, 2, 2, 2): 1.212e+06,
 }
 
 
 # The same for the dominant class kernel of the headline workload.
 TRAFFIC_HEADLINE = {
-    (0, 0, 0, 0): 1.001e+09, (1, 0, 0, 0): 8.355e+08, (1, 0, 1, 0): 3.344e+08, (1, 1, 0, 0): 3.327e+08,
-    (1, 1, 1, 0): 2.322e+08, (1, 1, 1, 1): 3.710e+07,
+    (0, 0, 0, 0): 6.223e+08, (1, 0, 0, 0): 4.914e+08, (1, 0, 1, 0): 2.694e+08, (1, 1, 0, 0): 1.652e+08,
+    (1, 1, 1, 0): 1.722e+08, (1, 1, 1, 1): 4.668e+07,
 }
 
 
