@@ -62,7 +62,11 @@ struct ClassShape {
     // (pp|pp) is sliced too: its units hold few surviving kets in batches of
     // small molecules, and slices multiply its lane items (a 6-31G batch
     // pass measured 285 against 298 ms; (H2O)8 cc-pVDZ builds unchanged).
-    static constexpr bool KSL = IBUF || (LC <= 1 && LD == 0) || (LA <= 1 && LC <= 1);
+    // (ds|pp) likewise: a lane with a whole (pp) ket set the length of the build
+    // of a small molecule ((H2O)3 6-31G* 98 us alone, 35 sliced; (H2O)8
+    // cc-pVDZ 146 and 111; (H2O)16, where lanes abound, 300 and 354).
+    static constexpr bool KSL = IBUF || (LC <= 1 && LD == 0) || (LA <= 1 && LC <= 1)
+                             || (LA == 2 && LB == 0 && LC == 1 && LD == 1);
     // The other classes digest each (quartet, chunk) item; when a quartet
     // has several chunks, their ket-side Coulomb blocks are summed in an LDS
     // buffer per batch (KJ) and added to G once per quartet.
