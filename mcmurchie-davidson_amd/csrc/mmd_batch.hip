@@ -342,9 +342,9 @@ __device__ __forceinline__ void jacobi_rotate_v(int n, int ld, int h, lds_d* V, 
 // owns one 2 x 2 block (rows of one rotation, columns of another) of the
 // upper triangle for the whole run, so no index is divided inside the loops
 // and half the matrix is neither read nor written; (c, s) come from
-// rsqrt(d^2 + 4 a^2) and rsqrt(cos^2), without a division.  Inlined, so that
-// the compiler knows that A and V are in LDS: called as a function, every
-// access went through the flat path at four times the time.
+// rsqrt(d^2 + 4 a^2) and rsqrt(cos^2), without a division.  A and V
+// say that they are in LDS: through plain pointers every access took the flat
+// path (S^-1/2 of 45 clusters of up to 65 functions 1.30 ms against 0.78).
 // Convergence: sum of squared off-diagonal elements at most 1e-30 of the
 // squared Frobenius norm.
 //
