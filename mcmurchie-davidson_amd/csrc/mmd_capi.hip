@@ -191,9 +191,9 @@ struct mmd_ctx {
     int pc_off[NPAIRCLASS + 1] = {0};
     int pc_npp[NPAIRCLASS] = {0}, pc_maxpp[NPAIRCLASS] = {0};   // primitive pairs of a class, largest count of a pair
     DevBuf<int2> d_ranges;              // per class and molecule: its pairs {first, end} in the class
-    DevBuf<int> w_count, w_scan, w_ints;   // work of the table build (PairWork; stats, unit counters)
+    DevBuf<int> w_count, w_entry, w_scan, w_ints;   // work of the table build (PairWork; stats, unit counters)
     DevBuf<double> w_q;
-    DevBuf<unsigned long long> w_qmax;
+    DevBuf<unsigned long long> w_qmax, w_keep;
     DevBuf<ShellPair> d_pairs;
     DevBuf<PrimPair> d_pp;
     DevBuf<KetScreen> d_kscr;    // ket tables of the row kernels
@@ -539,9 +539,13 @@ int build_pairs(mmd_ctx* c, const double* diag)
     const size_t n = (size_t)c->pc_off[NPAIRCLASS];
     HIP_TRY(c->d_pairs.reserve(n));
     HIP_TRY(c->w_count.reserve(n));
+    HIP_TRY(c->w_entry.reserve(n));
     HIP_TRY(c->w_q.reserve(n));
     HIP_TRY(c->w_scan.reserve(n + n / 1024 + 2));
     HIP_TRY(c->w_qmax.reserve(1));
+    int maxnp = 1;
+    for (const Shell& s : c->shells) maxnp = std::max(maxnp, s.np);
+    HIP_TRY(c->w_keep.reserve(n * pair_keep_words(maxnp)));
     constexpr int STATS = (int)(sizeof(PairStats) / sizeof(int)), HIST = NQCLASS * UNIT_BUCKETS;
     HIP_TRY(c->w_ints.reserve(STATS + NQCLASS + HIST));
     int* d_counts = c->w_ints.p + STATS;
@@ -558,9 +562,11 @@ int build_pairs(mmd_ctx* c, const double* diag)
     I.N = c->nbf;
     PairWork W;
     W.count = c->w_count.p;
+    W.entry = c->w_entry.p;
     W.q = c->w_q.p;
     W.scan = c->w_scan.p;
     W.qmax = c->w_qmax.p;
+    W.keep = c->w_keep.p;
     UnitInput U;
     U.pairs = c->d_pairs.p;
     U.ranges = c->d_ranges.p;

@@ -26,12 +26,18 @@ struct PairInput {
     int nmol, N;
 };
 
-// Work buffers, npairs entries each but for the last two.
+// 64-bit words of keep bits per pair (PairWork), for shells of at most maxnp
+// primitives.
+inline int pair_keep_words(int maxnp) { return (int)(((int64_t)maxnp * maxnp + 63) / 64); }
+
+// Work buffers, npairs entries each but for the last three.
 struct PairWork {
     int* count;                      // surviving primitive pairs, list order
+    int* entry;                      // list entry of each sorted pair
     double* q;                       // pair factors, list order
     int* scan;                       // npairs + npairs / 1024 + 2
     unsigned long long* qmax;        // largest primitive-pair bound
+    unsigned long long* keep;        // per primitive pair whether it survives: word w of list entry e at w * npairs + e
 };
 
 // Results on the host: largest and total primitive-pair count per class.
@@ -44,8 +50,8 @@ struct PairStats {
 // (molecule, primitive pairs descending, factor descending, list order) into
 // `pairs` with their ranges in the primitive-pair table, class by class.
 hipError_t launch_pair_sort(const PairInput& I, const PairWork& W, ShellPair* pairs, PairStats* stats, hipStream_t st);
-// The primitive-pair table of the sorted pairs, and each entry's first
-// exponent (ppa), and the row kernels' ket tables of both.
+// The primitive-pair table of the sorted pairs (the W of the sort), and each
+// entry's first exponent (ppa), and the row kernels' ket tables of both.
 struct KetTables {
     KetScreen* scr;
     KetRef* ref;

@@ -66,27 +66,37 @@ __global__ void __launch_bounds__(256) pair_bound_kernel(PairInput I, unsigned l
 
 // A primitive pair whose bound, times the largest bound of any pair, is below
 // PRIM_DROP contributes less than that to every primitive quartet and is
-// left out of the table.
-__device__ bool prim_kept(double p, double K, double AB2, int lab, double qmax)
-{
-    return !(prim_bound(p, K, AB2, lab) * qmax < PRIM_DROP);
-}
-
+// left out of the table.  Decided here once, as a bit of the pair's keep words:
+// the count sizes the pair's range of the table and the fill writes it, and a
+// pair at the threshold that each decided for itself, in code that the
+// compiler contracts in its own way, could be one record more than the range.
 __global__ void __launch_bounds__(256) pair_count_kernel(PairInput I, PairWork W)
 {
     const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= I.off[NPAIRCLASS]) return;
+    const int npairs = I.off[NPAIRCLASS];
+    if (e >= npairs) return;
     const double qmax = __longlong_as_double((long long)*W.qmax);
     const int2 pr = I.list[e];
     const OneeShell a = I.shells[pr.x], b = I.shells[pr.y];
     const double AB2 = dist2(a, b);
-    int n = 0;
+    int n = 0, bit = 0;
+    unsigned long long word = 0, *keep = W.keep + e;
     for (int i = 0; i < a.np; ++i)
         for (int j = 0; j < b.np; ++j) {
             const double ea = I.exps[a.p0 + i], eb = I.exps[b.p0 + j], p = ea + eb;
             const double K = I.wts[a.p0 + i] * I.wts[b.p0 + j] * exp(-ea * eb / p * AB2);
-            n += prim_kept(p, K, AB2, a.l + b.l, qmax) ? 1 : 0;
+            if (!(prim_bound(p, K, AB2, a.l + b.l) * qmax < PRIM_DROP)) {
+                word |= 1ull << bit;
+                ++n;
+            }
+            if (++bit == 64) {
+                *keep = word;
+                keep += npairs;
+                word = 0;
+                bit = 0;
+            }
         }
+    if (bit) *keep = word;
     double q = 1.0;
     if (I.diag) {
         q = 0.0;
@@ -131,6 +141,7 @@ __global__ void __launch_bounds__(256) pair_rank_kernel(PairInput I, PairWork W,
     sp.pad = 0;
     sp.q = q;
     pairs[s0 + rank] = sp;
+    W.entry[s0 + rank] = e;
 }
 
 // Exclusive prefix sums of the pairs' primitive counts: inside blocks, then of
@@ -198,27 +209,34 @@ __global__ void __launch_bounds__(256) pair_place_kernel(PairInput I, const int*
     if (i == I.off[c + 1] - 1) stats->total[c] = pairs[i].pad + n;
 }
 
-__global__ void __launch_bounds__(256) pair_fill_kernel(PairInput I, const unsigned long long* __restrict__ qmax_bits,
-                                                        const ShellPair* __restrict__ pairs,
+__global__ void __launch_bounds__(256) pair_fill_kernel(PairInput I, PairWork W, const ShellPair* __restrict__ pairs,
                                                         PrimPair* __restrict__ pp, double* __restrict__ ppa,
                                                         KetTables K)
 {
     const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= I.off[NPAIRCLASS]) return;
-    const double qmax = __longlong_as_double((long long)*qmax_bits);
+    const int npairs = I.off[NPAIRCLASS];
+    if (e >= npairs) return;
     const ShellPair sp = pairs[e];
     const OneeShell a = I.shells[sp.sa], b = I.shells[sp.sb];
     const double AB2 = dist2(a, b);
-    int o = sp.pp0;
+    int o = sp.pp0, bit = 0;
+    const unsigned long long* keep = W.keep + W.entry[e];
+    unsigned long long word = 0;
     K.scr[e] = KetScreen{sp.q, sp.sa, sp.sb};
     K.ref[e] = KetRef{sp.bfa, sp.bfb, sp.pp0, sp.npp};
     for (int i = 0; i < a.np; ++i)
         for (int j = 0; j < b.np; ++j) {
+            if (bit == 0) {
+                word = *keep;
+                keep += npairs;
+            }
+            const bool kept = word >> bit & 1;
+            bit = (bit + 1) & 63;
+            if (!kept) continue;
             const double ea = I.exps[a.p0 + i], eb = I.exps[b.p0 + j];
             PrimPair pq;
             pq.p = ea + eb;
             pq.K = I.wts[a.p0 + i] * I.wts[b.p0 + j] * exp(-ea * eb / pq.p * AB2);
-            if (!prim_kept(pq.p, pq.K, AB2, a.l + b.l, qmax)) continue;
             pq.Px = (ea * a.x + eb * b.x) / pq.p;
             pq.Py = (ea * a.y + eb * b.y) / pq.p;
             pq.Pz = (ea * a.z + eb * b.z) / pq.p;
@@ -404,7 +422,7 @@ hipError_t launch_pair_fill(const PairInput& I, const PairWork& W, const ShellPa
 {
     const int n = I.off[NPAIRCLASS];
     if (n <= 0) return hipSuccess;
-    hipLaunchKernelGGL(pair_fill_kernel, dim3((n + 255) / 256), dim3(256), 0, st, I, W.qmax, pairs, pp, ppa, K);
+    hipLaunchKernelGGL(pair_fill_kernel, dim3((n + 255) / 256), dim3(256), 0, st, I, W, pairs, pp, ppa, K);
     return hipGetLastError();
 }
 
