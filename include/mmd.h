@@ -46,6 +46,14 @@ int mmd_ctx_create(mmd_ctx **out, int device_id);
 void mmd_ctx_destroy(mmd_ctx *ctx);
 
 /*
+ * Frees what the tensor calls (mmd_eri_tensor, mmd_jk_tensor, mmd_ao2mo) keep
+ * on a device for the next one, of whatever context: at most 512 MB of device
+ * memory and 96 MB of pinned host memory.  An allocation of the library that
+ * fails does so by itself.  No counterpart in the reference.
+ */
+int mmd_release_workspaces(int device_id);
+
+/*
  * Basis functions, one per Cartesian component (replaces the list of
  * `Basis` objects, cython/basis.pxi:6-73, built by Molecule.formBasis,
  * mmd/molecule.py:57-73).

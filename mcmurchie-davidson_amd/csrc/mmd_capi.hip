@@ -25,6 +25,7 @@
 #include "mmd_kernels.h"
 #include "mmd_hostcopy.h"
 #include "mmd_pairs.h"
+#include "mmd_pool.h"
 #include "mmd_scf.h"
 #include "mmd_types.h"
 
@@ -88,7 +89,7 @@ struct DevBuf {
         std::lock_guard<std::recursive_mutex> lk(device_alloc_mutex());
         release();
         if (count == 0) count = 1;
-        hipError_t e = hipMalloc((void**)&p, count * sizeof(T));
+        hipError_t e = device_malloc((void**)&p, count * sizeof(T));
         if (e == hipSuccess) n = count;
         return e;
     }
@@ -200,10 +201,7 @@ struct mmd_ctx {
     DevBuf<KetRef> d_kref;
     DevBuf<double> d_kpp;
     int64_t kpp_stride = 0;
-    // staging of large host arrays, and the N^4 workspaces of the tensor calls
-    // that take or return them (up to T4_KEEP doubles each are kept)
-    HostStage stage;
-    DevBuf<double> t4[2], jk_mats;
+    DevBuf<double> jk_mats;      // N x N matrices of the tensor calls
     DevBuf<double> d_onee;   // S, T, V, M (3), L (3) of mmd_one_electron
     DevBuf<double> d_ns;     // overlap powers: S, X, U and the Newton-Schulz work (8 N^2 + 2)
 
@@ -673,21 +671,6 @@ int ensure_streams(mmd_ctx* c)
     return MMD_OK;
 }
 
-// An N^4 workspace kept from call to call costs its memory, one allocated per
-// call 0.1 to 0.3 ms (58 to 85 MB): tensors of up to 256 MB keep it.
-constexpr size_t T4_KEEP = (size_t)32 << 20;
-struct T4Scope {
-    mmd_ctx* c;
-    ~T4Scope()
-    {
-        for (DevBuf<double>& b : c->t4)
-            if (b.n > T4_KEEP) {
-                (void)hipStreamSynchronize(c->st);
-                b.release();
-            }
-    }
-};
-
 // Independent launches spread over the context's streams, largest first and
 // each to the least loaded stream, between a fork from and a join to c->st.
 struct StreamTask {
@@ -1114,6 +1097,16 @@ int mmd_ctx_create(mmd_ctx** out, int device_id)
         return rc;
     }
     *out = c;
+    return MMD_OK;
+}
+
+int mmd_release_workspaces(int device_id)
+{
+    int n = 0;
+    (void)mmd_device_count(&n);
+    if (device_id < 0 || device_id >= n) return fail(MMD_ERR_ARG, "device id out of range");
+    HIP_TRY(hipSetDevice(device_id));
+    (void)pool_release(device_id);
     return MMD_OK;
 }
 
@@ -1614,11 +1607,12 @@ int mmd_eri_tensor(mmd_ctx* ctx, double* out, int out_on_device)
     if (!out) return fail(MMD_ERR_ARG, "null output");
     if (ctx->nbf == 0) return fail(MMD_ERR_STATE, "no basis set");
     const size_t n4 = (size_t)ctx->nbf * ctx->nbf * ctx->nbf * ctx->nbf;
-    T4Scope scope{ctx};
+    Tensor4 t;
+    HostStage stage;
     double* dst = out;
     if (!out_on_device) {
-        HIP_TRY(ctx->t4[0].reserve(n4));
-        dst = ctx->t4[0].p;
+        HIP_TRY(t.reserve(n4));
+        dst = t.p;
     }
     if (ctx->shells_ok) {
         if (!ctx->pairs_ok) {
@@ -1630,8 +1624,9 @@ int mmd_eri_tensor(mmd_ctx* ctx, double* out, int out_on_device)
         HIP_TRY(launch_canonical_quartets(0, ctx->nbf, ctx->d_bf.p, ctx->d_bf_exp.p, ctx->d_bf_w.p, ctx->d_boys.p,
                                           nullptr, nullptr, nullptr, 0.0, dst, ctx->st));
     }
-    if (!out_on_device) HIP_TRY(ctx->stage.to_host(out, dst, sizeof(double) * n4, ctx->st));
+    if (!out_on_device) HIP_TRY(stage.to_host(out, dst, sizeof(double) * n4, ctx->st));
     HIP_TRY(hipStreamSynchronize(ctx->st));
+    t.done();
     return MMD_OK;
 }
 
@@ -1812,13 +1807,14 @@ int mmd_jk_tensor(mmd_ctx* ctx, const double* T, int t_on_device, const double* 
     if (!T || !P_re || !J_re || !K_re || (P_im && (!J_im || !K_im))) return fail(MMD_ERR_ARG, "null pointer");
     const int N = ctx->nbf;
     const size_t nn = (size_t)N * N, n4 = nn * nn;
-    T4Scope scope{ctx};
+    Tensor4 dT;
+    HostStage stage;
     DevBuf<double>& d = ctx->jk_mats;
     const double* t = T;
     if (!t_on_device) {
-        HIP_TRY(ctx->t4[0].reserve(n4));
-        HIP_TRY(ctx->stage.to_device(ctx->t4[0].p, T, sizeof(double) * n4, ctx->st));
-        t = ctx->t4[0].p;
+        HIP_TRY(dT.reserve(n4));
+        HIP_TRY(stage.to_device(dT.p, T, sizeof(double) * n4, ctx->st));
+        t = dT.p;
     }
     HIP_TRY(d.reserve(6 * nn));
     HIP_TRY(hipMemcpyAsync(d.p, P_re, sizeof(double) * nn, hipMemcpyHostToDevice, ctx->st));
@@ -1832,6 +1828,7 @@ int mmd_jk_tensor(mmd_ctx* ctx, const double* T, int t_on_device, const double* 
         HIP_TRY(hipMemcpyAsync(K_im, d.p + 5 * nn, sizeof(double) * nn, hipMemcpyDeviceToHost, ctx->st));
     }
     HIP_TRY(hipStreamSynchronize(ctx->st));
+    dT.done();
     return MMD_OK;
 }
 
@@ -2428,8 +2425,9 @@ int mmd_ao2mo(mmd_ctx* ctx, const double* T, int t_on_device, const double* C, d
     const int N = ctx->nbf;
     const size_t nn = (size_t)N * N, n3 = nn * N, n4 = nn * nn;
     if (n3 > (size_t)INT32_MAX) return fail(MMD_ERR_UNSUPPORTED, "basis too large for the transform");
-    T4Scope scope{ctx};
-    DevBuf<double>&a = ctx->t4[0], &b = ctx->t4[1], &dC = ctx->jk_mats;
+    Tensor4 a, b;
+    HostStage stage;
+    DevBuf<double>& dC = ctx->jk_mats;
     HIP_TRY(a.reserve(n4));
     HIP_TRY(b.reserve(n4));
     HIP_TRY(dC.reserve(nn));
@@ -2437,7 +2435,7 @@ int mmd_ao2mo(mmd_ctx* ctx, const double* T, int t_on_device, const double* C, d
     if (t_on_device)
         HIP_TRY(hipMemcpyAsync(a.p, T, sizeof(double) * n4, hipMemcpyDeviceToDevice, ctx->st));
     else
-        HIP_TRY(ctx->stage.to_device(a.p, T, sizeof(double) * n4, ctx->st));
+        HIP_TRY(stage.to_device(a.p, T, sizeof(double) * n4, ctx->st));
     // Four quarter transforms.  Each contracts the last index of X (M x N,
     // M = N^3) with C and writes it first: Y[S][pqr] = sum_s C[s][S] X[pqr][s],
     // i.e. Y = C^T X^T; after four passes the index order is (P,Q,R,S) again.
@@ -2452,8 +2450,10 @@ int mmd_ao2mo(mmd_ctx* ctx, const double* T, int t_on_device, const double* C, d
     if (out_on_device)
         HIP_TRY(hipMemcpyAsync(out, x, sizeof(double) * n4, hipMemcpyDeviceToDevice, ctx->st));
     else
-        HIP_TRY(ctx->stage.to_host(out, x, sizeof(double) * n4, ctx->st));
+        HIP_TRY(stage.to_host(out, x, sizeof(double) * n4, ctx->st));
     HIP_TRY(hipStreamSynchronize(ctx->st));
+    a.done();
+    b.done();
     if (gemm_ms) {
         float ms = 0.f;
         HIP_TRY(hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));

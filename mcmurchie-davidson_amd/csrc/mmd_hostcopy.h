@@ -3,11 +3,12 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stddef.h>
+#include "mmd_pool.h"
 
 namespace mmd {
 
-// The pinned slots of one context, allocated by its first large copy and freed
-// with it.  Not for use by two threads at once (neither is a context).
+// The copies of one call: its slots come from the device's pool at the first
+// large copy, as many as the array fills, and go back when the call ends.
 class HostStage {
 public:
     HostStage() = default;
@@ -21,11 +22,12 @@ public:
 
 private:
     static constexpr int SLOTS = 6;
-    bool prepare();
+    bool prepare(size_t bytes);
     hipError_t drain();
-    char* slots = nullptr;
-    hipEvent_t ev[SLOTS] = {};
+    StageSlot slot[SLOTS];
+    int nslots = 0;
     bool busy[SLOTS] = {};
+    hipStream_t broken = nullptr;   // where a copy failed: one without its event may still run there
 };
 
 }  // namespace mmd

@@ -4,7 +4,7 @@
 // thread: 17.6 GB/s to the host and 28.9 GB/s to the device, where the link
 // carries 57 GB/s to or from pinned memory.  The stored tensor, its J/K
 // contraction and the four-index transformation move N^4 doubles per call and
-// were bound by that.  Here the array goes through six pinned slots of 8 MiB: the
+// were bound by that.  Here the array goes through up to six pinned slots of 8 MiB: the
 // calling thread keeps the copy engine busy, and a few helper threads move the
 // slots to or from the caller's array (one thread moves 31 GB/s at most), a
 // sixteenth of a slot at a time, so that the first slot is soon full and the
@@ -30,7 +30,7 @@ std::recursive_mutex& device_alloc_mutex();
 
 namespace {
 
-constexpr size_t SLOT_BYTES = (size_t)8 << 20;
+constexpr size_t SLOT_BYTES = STAGE_SLOT_BYTES;
 constexpr int PARTS = 16;                           // of a slot
 constexpr size_t PART_BYTES = SLOT_BYTES / PARTS;
 constexpr size_t STAGE_MIN = (size_t)12 << 20;
@@ -78,37 +78,27 @@ struct Helpers {
 
 HostStage::~HostStage()
 {
-    (void)drain();
-    std::lock_guard<std::recursive_mutex> lk(device_alloc_mutex());
-    for (hipEvent_t e : ev)
-        if (e) (void)hipEventDestroy(e);
-    if (slots) (void)hipHostFree(slots);
+    hipError_t e = drain();
+    if (broken) e = hipStreamSynchronize(broken);
+    if (nslots) pool_give_slots(nslots, slot, e == hipSuccess);
 }
 
-bool HostStage::prepare()
+// Slots for an array of `bytes`, two at least; false: copy without.
+bool HostStage::prepare(size_t bytes)
 {
-    if (slots) return true;
-    std::lock_guard<std::recursive_mutex> lk(device_alloc_mutex());
-    for (hipEvent_t& e : ev)
-        if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
-            (void)hipGetLastError();
-            return false;
-        }
-    if (hipHostMalloc((void**)&slots, SLOTS * SLOT_BYTES, hipHostMallocDefault) != hipSuccess) {
-        (void)hipGetLastError();
-        slots = nullptr;
-        return false;
-    }
-    return true;
+    const size_t n = (bytes + SLOT_BYTES - 1) / SLOT_BYTES;
+    const int want = n < (size_t)SLOTS ? (int)n : SLOTS;
+    if (nslots < want) nslots += pool_take_slots(want - nslots, slot + nslots);
+    return nslots >= 2;
 }
 
 // Waits for copies that still read or write slots.
 hipError_t HostStage::drain()
 {
     hipError_t r = hipSuccess;
-    for (int s = 0; s < SLOTS; ++s) {
+    for (int s = 0; s < nslots; ++s) {
         if (!busy[s]) continue;
-        const hipError_t e = hipEventSynchronize(ev[s]);
+        const hipError_t e = hipEventSynchronize(slot[s].ev);
         if (e != hipSuccess) r = e;
         busy[s] = false;
     }
@@ -117,31 +107,32 @@ hipError_t HostStage::drain()
 
 hipError_t HostStage::to_host(void* dst, const void* src, size_t bytes, hipStream_t st)
 {
-    if (bytes < STAGE_MIN || !pageable(dst) || !prepare()) {
+    if (bytes < STAGE_MIN || !pageable(dst) || !prepare(bytes)) {
         const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st);
         return e == hipSuccess ? hipStreamSynchronize(st) : e;
     }
     hipError_t err = drain();
     if (err != hipSuccess) return err;
+    const int ns = nslots, half = (ns + 1) / 2;
     const int n = (int)((bytes + SLOT_BYTES - 1) / SLOT_BYTES);
     auto size_of = [&](int i) { return i + 1 < n ? SLOT_BYTES : bytes - (size_t)i * SLOT_BYTES; };
     const int64_t parts = (int64_t)((bytes + PART_BYTES - 1) / PART_BYTES);
     // bytes of a slot's chunks up to and including chunk i
-    auto through = [&](int i) { return (int64_t)(i / SLOTS) * (int64_t)SLOT_BYTES + (int64_t)size_of(i); };
+    auto through = [&](int i) { return (int64_t)(i / ns) * (int64_t)SLOT_BYTES + (int64_t)size_of(i); };
     std::atomic<int> ready{0};
     std::atomic<int64_t> ticket{0}, emptied[SLOTS];
     std::atomic<bool> stop{false};
     for (auto& x : emptied) x = 0;
     Helpers helpers([&] {
         for (int64_t k = ticket++; k < parts; k = ticket++) {
-            const int i = (int)(k / PARTS), s = i % SLOTS;
+            const int i = (int)(k / PARTS), s = i % ns;
             const size_t in = (size_t)(k % PARTS) * PART_BYTES, at = (size_t)k * PART_BYTES;
             const size_t len = bytes - at < PART_BYTES ? bytes - at : PART_BYTES;
             while (ready.load(std::memory_order_acquire) <= i) {
                 if (stop) return;
                 std::this_thread::yield();
             }
-            memcpy((char*)dst + at, slots + (size_t)s * SLOT_BYTES + in, len);
+            memcpy((char*)dst + at, slot[s].p + in, len);
             emptied[s].fetch_add((int64_t)len, std::memory_order_release);
         }
     });
@@ -151,71 +142,78 @@ hipError_t HostStage::to_host(void* dst, const void* src, size_t bytes, hipStrea
     }
     // copies up to half the slots ahead of the wait, so that the engine runs
     // while the helpers empty the other half
-    int queued = 0;
+    int next = 0;
     for (int i = 0; i < n && err == hipSuccess; ++i) {
-        for (; queued < n && queued < i + SLOTS / 2 && err == hipSuccess; ++queued) {
-            const int s = queued % SLOTS;
-            if (queued >= SLOTS)
-                while (emptied[s].load(std::memory_order_acquire) < through(queued - SLOTS)) std::this_thread::yield();
-            err = hipMemcpyAsync(slots + (size_t)s * SLOT_BYTES, (const char*)src + (size_t)queued * SLOT_BYTES,
-                                 size_of(queued), hipMemcpyDeviceToHost, st);
-            if (err == hipSuccess) err = hipEventRecord(ev[s], st);
+        for (; next < n && next < i + half && err == hipSuccess; ++next) {
+            const int s = next % ns;
+            if (next >= ns)
+                while (emptied[s].load(std::memory_order_acquire) < through(next - ns)) std::this_thread::yield();
+            err = hipMemcpyAsync(slot[s].p, (const char*)src + (size_t)next * SLOT_BYTES,
+                                 size_of(next), hipMemcpyDeviceToHost, st);
+            if (err == hipSuccess) err = hipEventRecord(slot[s].ev, st);
             if (err == hipSuccess) busy[s] = true;
         }
-        if (err == hipSuccess) err = hipEventSynchronize(ev[i % SLOTS]);
+        if (err == hipSuccess) err = hipEventSynchronize(slot[i % ns].ev);
         if (err == hipSuccess) {
-            busy[i % SLOTS] = false;
+            busy[i % ns] = false;
             ready.store(i + 1, std::memory_order_release);
         }
     }
-    if (err != hipSuccess) stop = true;
+    if (err != hipSuccess) {
+        stop = true;
+        broken = st;
+    }
     helpers.join();
     return err;
 }
 
 hipError_t HostStage::to_device(void* dst, const void* src, size_t bytes, hipStream_t st)
 {
-    if (bytes < STAGE_MIN || !pageable(src) || !prepare())
+    if (bytes < STAGE_MIN || !pageable(src) || !prepare(bytes))
         return hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, st);
     hipError_t err = drain();
     if (err != hipSuccess) return err;
+    const int ns = nslots, half = (ns + 1) / 2;
     const int n = (int)((bytes + SLOT_BYTES - 1) / SLOT_BYTES);
     auto size_of = [&](int i) { return i + 1 < n ? SLOT_BYTES : bytes - (size_t)i * SLOT_BYTES; };
     const int64_t parts = (int64_t)((bytes + PART_BYTES - 1) / PART_BYTES);
-    auto through = [&](int i) { return (int64_t)(i / SLOTS) * (int64_t)SLOT_BYTES + (int64_t)size_of(i); };
-    std::atomic<int> freed{SLOTS};
+    auto through = [&](int i) { return (int64_t)(i / ns) * (int64_t)SLOT_BYTES + (int64_t)size_of(i); };
+    std::atomic<int> freed{ns};
     std::atomic<int64_t> ticket{0}, filled[SLOTS];
     std::atomic<bool> stop{false};
     for (auto& x : filled) x = 0;
     Helpers helpers([&] {
         for (int64_t k = ticket++; k < parts; k = ticket++) {
-            const int i = (int)(k / PARTS), s = i % SLOTS;
+            const int i = (int)(k / PARTS), s = i % ns;
             const size_t in = (size_t)(k % PARTS) * PART_BYTES, at = (size_t)k * PART_BYTES;
             const size_t len = bytes - at < PART_BYTES ? bytes - at : PART_BYTES;
             while (freed.load(std::memory_order_acquire) <= i) {
                 if (stop) return;
                 std::this_thread::yield();
             }
-            memcpy(slots + (size_t)s * SLOT_BYTES + in, (const char*)src + at, len);
+            memcpy(slot[s].p + in, (const char*)src + at, len);
             filled[s].fetch_add((int64_t)len, std::memory_order_release);
         }
     });
     if (helpers.n == 0) return hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, st);
     for (int i = 0; i < n && err == hipSuccess; ++i) {
-        const int s = i % SLOTS;
+        const int s = i % ns;
         while (filled[s].load(std::memory_order_acquire) < through(i)) std::this_thread::yield();
-        err = hipMemcpyAsync((char*)dst + (size_t)i * SLOT_BYTES, slots + (size_t)s * SLOT_BYTES, size_of(i),
+        err = hipMemcpyAsync((char*)dst + (size_t)i * SLOT_BYTES, slot[s].p, size_of(i),
                              hipMemcpyHostToDevice, st);
-        if (err == hipSuccess) err = hipEventRecord(ev[s], st);
+        if (err == hipSuccess) err = hipEventRecord(slot[s].ev, st);
         if (err == hipSuccess) busy[s] = true;
-        const int back = i - (SLOTS / 2 - 1);   // half the slots in flight, half with the helpers
+        const int back = i - (half - 1);   // half the slots in flight, half with the helpers
         if (err == hipSuccess && back >= 0) {
-            err = hipEventSynchronize(ev[back % SLOTS]);
-            busy[back % SLOTS] = false;
-            freed.store(back + 1 + SLOTS, std::memory_order_release);
+            err = hipEventSynchronize(slot[back % ns].ev);
+            busy[back % ns] = false;
+            freed.store(back + 1 + ns, std::memory_order_release);
         }
     }
-    if (err != hipSuccess) stop = true;
+    if (err != hipSuccess) {
+        stop = true;
+        broken = st;
+    }
     helpers.join();
     return err;
 }

@@ -20,6 +20,7 @@
 namespace mmd {
 void set_last_error(const char* msg);   // the library's mmd_last_error() text
 std::recursive_mutex& device_alloc_mutex();   // held around allocations and graph captures
+hipError_t device_malloc(void** p, size_t bytes);   // frees what is kept between calls when memory runs out
 }
 
 namespace {
@@ -52,7 +53,7 @@ struct Buf {
         if (p) (void)hipFree(p);
         p = nullptr;
         n = 0;
-        hipError_t e = hipMalloc((void**)&p, std::max<size_t>(count, 1) * sizeof(T));
+        hipError_t e = mmd::device_malloc((void**)&p, std::max<size_t>(count, 1) * sizeof(T));
         if (e == hipSuccess) n = count;
         return e;
     }

@@ -48,6 +48,8 @@ lib.mmd_ctx_create.restype = _c_int
 lib.mmd_ctx_create.argtypes = [ctypes.POINTER(_ctx_p), _c_int]
 lib.mmd_ctx_destroy.restype = None
 lib.mmd_ctx_destroy.argtypes = [_ctx_p]
+lib.mmd_release_workspaces.restype = _c_int
+lib.mmd_release_workspaces.argtypes = [_c_int]
 lib.mmd_set_basis.restype = _c_int
 lib.mmd_set_basis.argtypes = [_ctx_p, _c_int, _vp, _vp, _vp, _vp, _vp]
 lib.mmd_set_atoms.restype = _c_int
@@ -134,7 +136,7 @@ lib.mmd_mlp_train.restype = _c_int
 lib.mmd_mlp_train.argtypes = [_vp, _c_int, _vp, _vp, _c_int, _c_int, ctypes.c_float, ctypes.c_uint64, _vp]
 
 EXPORTED = [
-    "mmd_last_error", "mmd_version", "mmd_device_count", "mmd_ctx_create", "mmd_ctx_destroy",
+    "mmd_last_error", "mmd_version", "mmd_device_count", "mmd_ctx_create", "mmd_ctx_destroy", "mmd_release_workspaces",
     "mmd_set_basis", "mmd_set_atoms", "mmd_one_electron", "mmd_schwarz", "mmd_set_schwarz",
     "mmd_eri_tensor", "mmd_eri_list", "mmd_fock_delta", "mmd_fock_delta_noalloc", "mmd_jk_tensor", "mmd_boys",
     "mmd_last_fock_ms", "mmd_set_profiling", "mmd_fock_stats", "mmd_fock_profile_sums", "mmd_rhf_gradient", "mmd_rhf_total_gradient",
@@ -165,6 +167,11 @@ def device_count():
     n = _c_int(0)
     check(lib.mmd_device_count(ctypes.byref(n)))
     return n.value
+
+
+def release_workspaces(device=0):
+    """Frees the buffers that the tensor calls keep on a device between calls."""
+    check(lib.mmd_release_workspaces(int(device)))
 
 
 def _ptr(a):
