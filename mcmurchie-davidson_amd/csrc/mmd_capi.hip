@@ -192,9 +192,12 @@ struct mmd_ctx {
     int pc_off[NPAIRCLASS + 1] = {0};
     int pc_npp[NPAIRCLASS] = {0}, pc_maxpp[NPAIRCLASS] = {0};   // primitive pairs of a class, largest count of a pair
     DevBuf<int2> d_ranges;              // per class and molecule: its pairs {first, end} in the class
-    DevBuf<int> w_count, w_entry, w_scan, w_ints;   // work of the table build (PairWork; stats, unit counters)
+    std::vector<int2> pair_ranges;      // and on the host, with the bra slices if no primitive pair is
+    std::vector<int64_t> pair_slices;   // screened out, and the primitive pairs of each class
+    int64_t pair_prims[NPAIRCLASS] = {0};
+    DevBuf<int> w_count, w_entry, w_scan, w_ints;   // work of the table build (PairWork)
     DevBuf<double> w_q;
-    DevBuf<unsigned long long> w_qmax, w_keep;
+    DevBuf<uint16_t> w_keep;
     DevBuf<ShellPair> d_pairs;
     DevBuf<PrimPair> d_pp;
     DevBuf<KetScreen> d_kscr;    // ket tables of the row kernels
@@ -215,6 +218,7 @@ struct mmd_ctx {
     DevBuf<int2> d_surv;
     DevBuf<FockCounters> d_ctr;
     FockCounters* h_ctr = nullptr;   // pinned: the counters of the last build
+    int* h_pairs = nullptr;          // and the table build's report, after them
 
     // atoms
     int natom = 0;
@@ -435,14 +439,20 @@ int onee_pair_list(mmd_ctx* c)
     if (c->onee_list_ok) return MMD_OK;
     if (int rc = molecule_shell_ranges(c)) return rc;
     std::vector<std::vector<int2>> byclass(NPAIRCLASS);
-    std::vector<int2> ranges((size_t)NPAIRCLASS * c->nmol);
+    std::vector<int2>& ranges = c->pair_ranges;
+    ranges.assign((size_t)NPAIRCLASS * c->nmol, make_int2(0, 0));
+    c->pair_slices.assign((size_t)NPAIRCLASS * c->nmol, 0);
+    for (int64_t& p : c->pair_prims) p = 0;
     for (int m = 0; m < c->nmol; ++m) {
         for (int pc = 0; pc < NPAIRCLASS; ++pc) ranges[(size_t)pc * c->nmol + m].x = (int)byclass[pc].size();
         for (int I = c->mol_s0[m]; I < c->mol_s0[m + 1]; ++I)
             for (int J = c->mol_s0[m]; J <= I; ++J) {
                 int a = I, b = J;
                 if (c->shells[I].l < c->shells[J].l) std::swap(a, b);
-                byclass[pair_class(c->shells[a].l, c->shells[b].l)].push_back(make_int2(a, b));
+                const int pc = pair_class(c->shells[a].l, c->shells[b].l), np = c->shells[a].np * c->shells[b].np;
+                byclass[pc].push_back(make_int2(a, b));
+                c->pair_prims[pc] += np;
+                c->pair_slices[(size_t)pc * c->nmol + m] += (np + PSLICE - 1) / PSLICE;
             }
         for (int pc = 0; pc < NPAIRCLASS; ++pc) ranges[(size_t)pc * c->nmol + m].y = (int)byclass[pc].size();
     }
@@ -540,14 +550,11 @@ int build_pairs(mmd_ctx* c, const double* diag)
     HIP_TRY(c->w_entry.reserve(n));
     HIP_TRY(c->w_q.reserve(n));
     HIP_TRY(c->w_scan.reserve(n + n / 1024 + 2));
-    HIP_TRY(c->w_qmax.reserve(1));
     int maxnp = 1;
     for (const Shell& s : c->shells) maxnp = std::max(maxnp, s.np);
-    HIP_TRY(c->w_keep.reserve(n * pair_keep_words(maxnp)));
-    constexpr int STATS = (int)(sizeof(PairStats) / sizeof(int)), HIST = NQCLASS * UNIT_BUCKETS;
-    HIP_TRY(c->w_ints.reserve(STATS + NQCLASS + HIST));
-    int* d_counts = c->w_ints.p + STATS;
-    int* d_hist = d_counts + NQCLASS;
+    HIP_TRY(c->w_keep.reserve(n * pair_keep_pieces(maxnp)));
+    constexpr int HEAD = (PAIR_REPORT + UNIT_HIST + 1) & ~1;   // the bound after it is 8 bytes
+    HIP_TRY(c->w_ints.reserve(HEAD + 2));
     PairInput I;
     I.shells = c->d_oshell.p;
     I.exps = c->d_sh_exp.p;
@@ -563,8 +570,11 @@ int build_pairs(mmd_ctx* c, const double* diag)
     W.entry = c->w_entry.p;
     W.q = c->w_q.p;
     W.scan = c->w_scan.p;
-    W.qmax = c->w_qmax.p;
     W.keep = c->w_keep.p;
+    W.report = c->w_ints.p;
+    W.hist = W.report + PAIR_REPORT;
+    W.qmax = reinterpret_cast<unsigned long long*>(W.report + HEAD);
+    W.nclear = HEAD + 2;
     UnitInput U;
     U.pairs = c->d_pairs.p;
     U.ranges = c->d_ranges.p;
@@ -596,41 +606,64 @@ int build_pairs(mmd_ctx* c, const double* diag)
             while (seg > 32 && c->qc_total[qc] / seg < 512) seg /= 2;
         c->unit_seg[qc] = U.seg[qc] = seg;
     }
-    HIP_TRY(launch_pair_sort(I, W, c->d_pairs.p, reinterpret_cast<PairStats*>(c->w_ints.p), c->st));
-    if (diag) HIP_TRY(launch_unit_count(U, d_hist, d_counts, c->w_q.p, c->st));   // the factors are in the pairs now
-    int h[STATS + NQCLASS] = {0};
-    HIP_TRY(hipMemcpyAsync(h, c->w_ints.p, sizeof(int) * (STATS + (diag ? NQCLASS : 0)), hipMemcpyDeviceToHost, c->st));
-    HIP_TRY(hipStreamSynchronize(c->st));
-    PairStats stats;
-    memcpy(&stats, h, sizeof(stats));
-    size_t npp = 0;
-    for (int pc = 0; pc < NPAIRCLASS; ++pc) {
-        c->pc_npp[pc] = stats.total[pc];
-        c->pc_maxpp[pc] = std::max(1, stats.maxpp[pc]);
-        npp += (size_t)stats.total[pc];
+    HIP_TRY(launch_pair_sort(I, W, U, diag != nullptr, c->d_pairs.p, c->st));
+    // Sizes of the tables: as if no primitive pair were screened out, so that
+    // the device need not be waited for between the sort and the tables; the
+    // counts themselves where that could waste more than TABLE_SLACK bytes.
+    size_t npp = 0, units = 0;
+    for (int pc = 0; pc < NPAIRCLASS; ++pc) npp += (size_t)c->pair_prims[pc];
+    if (diag)
+        for (int qc = 0; qc < NQCLASS; ++qc) {
+            int pcb, pck;
+            class_of(qc, &pcb, &pck);
+            for (int m = 0; m < c->nmol; ++m) {
+                const int2 r = c->pair_ranges[(size_t)pck * c->nmol + m];
+                units += (size_t)c->pair_slices[(size_t)pcb * c->nmol + m]
+                       * (size_t)((r.y - r.x + U.seg[qc] - 1) / U.seg[qc]);
+            }
+        }
+    constexpr size_t TABLE_SLACK = (size_t)64 << 20;
+    if (npp * (sizeof(PrimPair) + sizeof(double) * (1 + KET_FIELDS)) + units * (sizeof(int4) + sizeof(UnitBound))
+        > TABLE_SLACK) {
+        int h[PAIR_REPORT];
+        HIP_TRY(hipMemcpyAsync(h, W.report, sizeof(h), hipMemcpyDeviceToHost, c->st));
+        HIP_TRY(hipStreamSynchronize(c->st));
+        PairStats stats;
+        memcpy(&stats, h, sizeof(stats));
+        npp = units = 0;
+        for (int pc = 0; pc < NPAIRCLASS; ++pc) npp += (size_t)stats.total[pc];
+        if (diag)
+            for (int qc = 0; qc < NQCLASS; ++qc) units += (size_t)h[PAIR_STATS + qc];
     }
-    HIP_TRY(c->d_pp.reserve(std::max<size_t>(1, npp)));
-    HIP_TRY(c->d_ppa.reserve(std::max<size_t>(1, npp)));
-    c->kpp_stride = (int64_t)((std::max<size_t>(1, npp) + 15) & ~(size_t)15);   // fields start on cache lines
+    npp = std::max<size_t>(1, npp);
+    units = std::max<size_t>(1, units);
+    HIP_TRY(c->d_pp.reserve(npp));
+    HIP_TRY(c->d_ppa.reserve(npp));
+    c->kpp_stride = (int64_t)((npp + 15) & ~(size_t)15);   // fields start on cache lines
     HIP_TRY(c->d_kscr.reserve(n));
     HIP_TRY(c->d_kref.reserve(n));
     HIP_TRY(c->d_kpp.reserve((size_t)(KET_FIELDS * c->kpp_stride)));
     const KetTables K = {c->d_kscr.p, c->d_kref.p, c->d_kpp.p, c->kpp_stride};
-    HIP_TRY(launch_pair_fill(I, W, c->d_pairs.p, c->d_pp.p, c->d_ppa.p, K, c->st));
+    UnitTables T = {nullptr, nullptr};
     if (diag) {
-        int64_t units = 0;
-        for (int qc = 0; qc < NQCLASS; ++qc) {
-            c->unit_off[qc] = units;
-            units += h[STATS + qc];
-        }
-        c->unit_off[NQCLASS] = units;
-        HIP_TRY(c->d_units.reserve(std::max<size_t>(1, (size_t)units)));
-        HIP_TRY(c->d_ubound.reserve(std::max<size_t>(1, (size_t)units)));
-        if (c->nmol > 1) HIP_TRY(c->d_live.reserve(std::max<size_t>(1, (size_t)units)));
-        HIP_TRY(launch_unit_scatter(U, d_hist, c->w_q.p, c->d_units.p, c->d_ubound.p, c->st));
+        HIP_TRY(c->d_units.reserve(units));
+        HIP_TRY(c->d_ubound.reserve(units));
+        if (c->nmol > 1) HIP_TRY(c->d_live.reserve(units));
+        T = {c->d_units.p, c->d_ubound.p};
+    }
+    HIP_TRY(launch_pair_tables(I, W, c->d_pairs.p, c->d_pp.p, c->d_ppa.p, K, U, T, c->h_pairs, c->st));
+    HIP_TRY(hipStreamSynchronize(c->st));
+    PairStats stats;
+    memcpy(&stats, c->h_pairs, sizeof(stats));
+    for (int pc = 0; pc < NPAIRCLASS; ++pc) {
+        c->pc_npp[pc] = stats.total[pc];
+        c->pc_maxpp[pc] = std::max(1, stats.maxpp[pc]);
+    }
+    if (diag) {
+        c->unit_off[0] = 0;
+        for (int qc = 0; qc < NQCLASS; ++qc) c->unit_off[qc + 1] = c->unit_off[qc] + c->h_pairs[PAIR_STATS + qc];
         c->units_ok = true;
     }
-    HIP_TRY(hipStreamSynchronize(c->st));
     HIP_TRY(c->d_ctr.reserve(1));
     c->pairs_ok = true;
     for (int qc = 0; qc < NQCLASS; ++qc) {
@@ -1071,7 +1104,8 @@ int mmd_ctx_create(mmd_ctx** out, int device_id)
     hipError_t e = hipStreamCreateWithFlags(&c->st, hipStreamNonBlocking);
     if (e == hipSuccess) {
         std::lock_guard<std::recursive_mutex> lk(device_alloc_mutex());
-        e = hipHostMalloc((void**)&c->h_ctr, sizeof(FockCounters), hipHostMallocDefault);
+        e = hipHostMalloc((void**)&c->h_ctr, sizeof(FockCounters) + sizeof(int) * PAIR_REPORT, hipHostMallocDefault);
+        if (e == hipSuccess) c->h_pairs = reinterpret_cast<int*>(c->h_ctr + 1);
     }
     if (e == hipSuccess) e = hipEventCreate(&c->ev0);
     if (e == hipSuccess) e = hipEventCreate(&c->ev1);

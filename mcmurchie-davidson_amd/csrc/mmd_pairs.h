@@ -26,40 +26,33 @@ struct PairInput {
     int nmol, N;
 };
 
-// 64-bit words of keep bits per pair (PairWork), for shells of at most maxnp
-// primitives.
-inline int pair_keep_words(int maxnp) { return (int)(((int64_t)maxnp * maxnp + 63) / 64); }
-
-// Work buffers, npairs entries each but for the last three.
-struct PairWork {
-    int* count;                      // surviving primitive pairs, list order
-    int* entry;                      // list entry of each sorted pair
-    double* q;                       // pair factors, list order
-    int* scan;                       // npairs + npairs / 1024 + 2
-    unsigned long long* qmax;        // largest primitive-pair bound
-    unsigned long long* keep;        // per primitive pair whether it survives: word w of list entry e at w * npairs + e
-};
-
-// Results on the host: largest and total primitive-pair count per class.
+// Results per class: the largest and total primitive-pair count; and units.
 struct PairStats {
     int maxpp[NPAIRCLASS];
     int total[NPAIRCLASS];
 };
+constexpr int PAIR_STATS = (int)(sizeof(PairStats) / sizeof(int));
+constexpr int PAIR_REPORT = PAIR_STATS + NQCLASS;   // ints: PairStats, units of each quartet class
+constexpr int UNIT_HIST = NQCLASS * UNIT_BUCKETS;
 
-// Primitive pairs counted and screened, the pairs sorted inside each class by
-// (molecule, primitive pairs descending, factor descending, list order) into
-// `pairs` with their ranges in the primitive-pair table, class by class.
-hipError_t launch_pair_sort(const PairInput& I, const PairWork& W, ShellPair* pairs, PairStats* stats, hipStream_t st);
-// The primitive-pair table of the sorted pairs (the W of the sort), and each
-// entry's first exponent (ppa), and the row kernels' ket tables of both.
-struct KetTables {
-    KetScreen* scr;
-    KetRef* ref;
-    double* pp;
-    int64_t stride;
+// Keep bits of a pair's primitive pairs come in pieces of 16; the pieces of a
+// pair of shells of at most maxnp primitives.
+constexpr int PAIR_KEEP_BITS = 16;
+inline size_t pair_keep_pieces(int maxnp) { return ((size_t)maxnp * maxnp + PAIR_KEEP_BITS - 1) / PAIR_KEEP_BITS; }
+
+// Work buffers, npairs entries each but for the last four.
+struct PairWork {
+    int* count;                      // surviving primitive pairs, list order
+    int* entry;                      // list entry of each sorted pair
+    double* q;                       // pair factors, list order; then the units' running maxima
+    uint16_t* keep;                  // piece t of list entry e at t * npairs + e (pair_keep_pieces)
+    int* scan;                       // npairs + npairs / 1024 + 2
+    // nclear ints one after the other, cleared together:
+    int* report;                     // PAIR_REPORT
+    int* hist;                       // UNIT_HIST counters of the units' cost buckets, then their cursors
+    unsigned long long* qmax;        // largest primitive-pair bound
+    int nclear;
 };
-hipError_t launch_pair_fill(const PairInput& I, const PairWork& W, const ShellPair* pairs, PrimPair* pp, double* ppa,
-                            const KetTables& K, hipStream_t st);
 
 // Work units of the row kernels.  One per (bra pair, slice of at most PSLICE
 // of its primitive pairs, segment of seg[qc] kets of its molecule), in
@@ -71,12 +64,31 @@ struct UnitInput {
     int seg[NQCLASS];
     int nmol;
 };
-// hist: NQCLASS x UNIT_BUCKETS counters; counts[qc]: units of class qc;
-// qrun: npairs running maxima.  The scatter takes the cursors that the count
-// left in hist, and writes class qc at units + (sum of the counts before it).
-hipError_t launch_unit_count(const UnitInput& I, int* hist, int* counts, double* qrun, hipStream_t st);
-hipError_t launch_unit_scatter(const UnitInput& I, int* hist, const double* qrun, int4* units, UnitBound* bounds,
-                               hipStream_t st);
+
+// Primitive pairs counted and screened, the pairs sorted inside each class by
+// (molecule, primitive pairs descending, factor descending, list order) into
+// `pairs` with their ranges in the primitive-pair table, class by class; and
+// the units counted, where asked for.
+hipError_t launch_pair_sort(const PairInput& I, const PairWork& W, const UnitInput& U, bool units, ShellPair* pairs,
+                            hipStream_t st);
+
+// The tables of the sorted pairs (the W of the sort): their primitive pairs,
+// each entry's first exponent (ppa), and the row kernels' ket tables of both;
+// the units (T.units null: none), class qc after the classes before it.  The
+// report goes to pinned host memory.
+struct KetTables {
+    KetScreen* scr;
+    KetRef* ref;
+    double* pp;
+    int64_t stride;
+};
+struct UnitTables {
+    int4* units;
+    UnitBound* bounds;
+};
+hipError_t launch_pair_tables(const PairInput& I, const PairWork& W, const ShellPair* pairs, PrimPair* pp, double* ppa,
+                              const KetTables& K, const UnitInput& U, const UnitTables& T, int* host_report,
+                              hipStream_t st);
 
 // Of each class's units [off[qc], off[qc + 1]) those that hold a quartet which
 // can pass the screen: pair factors q_P q_Q <= the unit's bound, and density
