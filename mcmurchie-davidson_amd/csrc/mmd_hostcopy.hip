@@ -16,17 +16,14 @@
 // below STAGE_MIN keep the runtime's copy, as does pinned memory, which needs
 // no staging).
 #include "mmd_hostcopy.h"
+#include "mmd_helpers.h"
 
 #include <atomic>
-#include <mutex>
 #include <stdint.h>
 #include <string.h>
-#include <system_error>
 #include <thread>
 
 namespace mmd {
-
-std::recursive_mutex& device_alloc_mutex();
 
 namespace {
 
@@ -34,7 +31,6 @@ constexpr size_t SLOT_BYTES = STAGE_SLOT_BYTES;
 constexpr int PARTS = 16;                           // of a slot
 constexpr size_t PART_BYTES = SLOT_BYTES / PARTS;
 constexpr size_t STAGE_MIN = (size_t)12 << 20;
-constexpr int HELPERS = 4;
 
 bool pageable(const void* p)
 {
@@ -46,33 +42,6 @@ bool pageable(const void* p)
     }
     return a.type == hipMemoryTypeUnregistered;
 }
-
-int helper_count()
-{
-    const int cpus = (int)std::thread::hardware_concurrency();
-    return cpus <= 2 ? 1 : (cpus - 1 < HELPERS ? cpus - 1 : HELPERS);
-}
-
-// Helper threads that run f until it returns; joined on destruction.
-struct Helpers {
-    std::thread t[HELPERS];
-    int n = 0;
-    template <class F>
-    explicit Helpers(F f)
-    {
-        const int want = helper_count();
-        try {
-            for (; n < want; ++n) t[n] = std::thread(f);
-        } catch (const std::system_error&) {   // fewer threads, or none
-        }
-    }
-    ~Helpers() { join(); }
-    void join()
-    {
-        for (int i = 0; i < n; ++i) t[i].join();
-        n = 0;
-    }
-};
 
 }  // namespace
 
