@@ -691,13 +691,13 @@ int grid_for(int64_t items)
     return (int)g;
 }
 
-// The side streams that nstreams asks for, created when a basis is set: HIP
+// The side streams of n streams, created when a basis is set: HIP
 // deals streams to its few hardware queues in order of creation, so contexts
 // that each made all seven at once had their main streams on one queue, and
 // batch groups on different contexts ran one after the other.
-int ensure_streams(mmd_ctx* c)
+int ensure_streams(mmd_ctx* c, int n)
 {
-    for (int i = 0; i + 1 < c->nstreams; ++i) {
+    for (int i = 0; i + 1 < n; ++i) {
         if (!c->side[i]) HIP_TRY(hipStreamCreateWithFlags(&c->side[i], hipStreamNonBlocking));
         if (!c->evjoin[i]) HIP_TRY(hipEventCreateWithFlags(&c->evjoin[i], hipEventDisableTiming));
     }
@@ -1173,6 +1173,7 @@ int mmd_set_basis(mmd_ctx* ctx, int nbf, const double* origin, const int32_t* lm
     int rc = check_ctx(ctx);
     if (rc) return rc;
     if (nbf <= 0 || !origin || !lmn || !nprim || !exps || !weights) return fail(MMD_ERR_ARG, "invalid basis arguments");
+    if ((rc = ensure_streams(ctx, ctx->nstreams))) return rc;   // a context with a basis has its streams
     ctx->bf.assign(nbf, BFDesc{});
     ctx->bf_exp.clear();
     ctx->bf_w.clear();
@@ -1222,7 +1223,6 @@ int mmd_set_basis(mmd_ctx* ctx, int nbf, const double* origin, const int32_t* lm
         rc = upload_shells(ctx);
         if (rc) return rc;
     }
-    if ((rc = ensure_streams(ctx))) return rc;
     const size_t nn = (size_t)nbf * nbf;
     HIP_TRY(ctx->d_D.reserve(nn));
     HIP_TRY(ctx->d_Dim.reserve(nn));
@@ -1977,10 +1977,12 @@ int mmd_set_streams(mmd_ctx* ctx, int n)
 {
     if (!ctx) return fail(MMD_ERR_ARG, "null context");
     if (n < 1 || n > 1 + mmd_ctx::NSIDE) return fail(MMD_ERR_ARG, "streams must be in [1, %d]", 1 + mmd_ctx::NSIDE);
+    if (ctx->nbf > 0) {
+        HIP_TRY(hipSetDevice(ctx->device));
+        if (int rc = ensure_streams(ctx, n)) return rc;
+    }
     ctx->nstreams = n;
-    if (ctx->nbf == 0) return MMD_OK;
-    HIP_TRY(hipSetDevice(ctx->device));
-    return ensure_streams(ctx);
+    return MMD_OK;
 }
 
 int mmd_set_lds_limit(mmd_ctx* ctx, int64_t bytes)
