@@ -228,7 +228,7 @@ struct mmd_ctx {
     double last_grad_ms = 0.0;
     // gradient by shell class: exponent of the first function of every
     // primitive pair, the classes' bra slices (of grad_pslice primitive pairs,
-    // and of one for the wavefront kernels) and flat primitive-pair lists,
+    // and of one for the workgroup-per-primitive-quartet kernels) and flat primitive-pair lists,
     // made from the pair table on first use
     DevBuf<double> d_ppa, g_rep;
     DevBuf<int4> g_slices;
@@ -281,13 +281,11 @@ struct mmd_ctx {
     double tune_ms[2][NQCLASS] = {};
     bool tune_measuring = false;
     // Work units of the row-kernel classes (built once per pair table):
-    // class qc owns units [unit_off[qc], unit_off[qc+1]) with ket segment
-    // length unit_seg[qc].
+    // class qc owns units [unit_off[qc], unit_off[qc+1]).
     DevBuf<int4> d_units;
     DevBuf<UnitBound> d_ubound;         // per unit, in the same order
     DevBuf<int> d_live;
     int64_t unit_off[NQCLASS + 1] = {0};
-    int unit_seg[NQCLASS] = {0};
     bool units_ok = false;
     size_t max_lds = 65536;             // LDS a class launch may use (mmd_set_lds_limit)
     size_t max_lds_device = 65536;      // the device's limit per workgroup
@@ -604,7 +602,7 @@ int build_pairs(mmd_ctx* c, const double* diag)
         // 512, 1024, 2048, 4096; (H2O)8 cc-pVDZ 1.76, 1.88, 2.07, 2.37 ms).
         if (c->nmol == 1)
             while (seg > 32 && c->qc_total[qc] / seg < 512) seg /= 2;
-        c->unit_seg[qc] = U.seg[qc] = seg;
+        U.seg[qc] = seg;
     }
     HIP_TRY(launch_pair_sort(I, W, U, diag != nullptr, c->d_pairs.p, c->st));
     // Sizes of the tables: as if no primitive pair were screened out, so that
@@ -902,7 +900,6 @@ int run_fock_classes(mmd_ctx* c, ClassArgs A, double tol, FockScratch& W0)
             R.maxpp = maxpp[qc];
             R.kj = kj_lds[qc] ? 1 : 0;
             R.kslice = c->ket_slice[qc];
-            R.seg = c->unit_seg[qc];
             R.rw = c->rw;
             R.kscr = c->d_kscr.p;
             R.kref = c->d_kref.p;
@@ -1336,7 +1333,7 @@ int build_grad_plan(mmd_ctx* c)
             for (int i = 0; i < npp; ++i) flat.push_back(make_int2(P, i));
             const int end = (int)flat.size() - c->g_flat_off[pc];
             for (int i = 0; i < npp; i += step) sl.push_back(make_int4(P, i, std::min(npp, i + step), end));
-            if (pc >= 4)   // (dp) and (dd): the bras of the wavefront classes
+            if (pc >= 4)   // (dp) and (dd): the bras of those classes
                 for (int i = 0; i < npp; ++i) one.push_back(make_int4(P, i, i + 1, end));
         }
     }
@@ -1383,8 +1380,8 @@ int gradient_shells(mmd_ctx* c, const double* dP, const double* dW, const double
         int pcb, pck, la, lb, lc, ld;
         class_of(qc, &pcb, &pck);
         qclass_decode(qc, &la, &lb, &lc, &ld);
-        const bool wave = fock_class_is_mfma(la, lb, lc, ld);
-        const int* off = wave ? c->g_one_off : c->g_slice_off;
+        const bool block = fock_class_is_mfma(la, lb, lc, ld);   // a workgroup per primitive quartet
+        const int* off = block ? c->g_one_off : c->g_slice_off;
         GradClass& C = cls[qc];
         C.slices = c->g_slices.p + off[pcb];
         C.nslice = off[pcb + 1] - off[pcb];

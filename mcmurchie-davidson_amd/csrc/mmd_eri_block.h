@@ -139,7 +139,7 @@ __global__ void __launch_bounds__(256) eri_block_kernel(ClassArgs A, BlockArgs B
         static_switch<0, S::NCHUNK>(chunk, [&](auto ic) {
             constexpr int A0 = decltype(ic)::value * S::CH, A1 = A0 + S::CH;
             double acc[NV];
-            quartet_compute<LA, LB, LC, LD, A0, A1, double>(KetRecords{A.pp}, boys, B.table + (size_t)bra.pad * S::BPS,
+            quartet_compute<LA, LB, LC, LD, A0, A1, double>(KetRecords{A.pp}, boys, B.table + (size_t)bra.class_pp0 * S::BPS,
                                                             ip0, ip1, ket.pp0 + jq0, ket.pp0 + jq1, acc);
             for (int off = 1; off < G; off <<= 1)
                 sfor<NV>([&](auto k) { acc[decltype(k)::value] += __shfl_xor(acc[decltype(k)::value], off); });

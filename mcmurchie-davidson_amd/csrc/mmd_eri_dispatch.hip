@@ -31,7 +31,7 @@ __global__ void __launch_bounds__(64) bra_table_kernel(const ShellPair* __restri
     for (int idx = threadIdx.x; idx < 3 * bra.npp; idx += blockDim.x) {
         const int ip = idx / 3, x = idx - 3 * ip;
         const PrimPair* P = pp + bra.pp0 + ip;
-        double* b = table + (size_t)(bra.pad + ip) * S::BPS;
+        double* b = table + (size_t)(bra.class_pp0 + ip) * S::BPS;
         if (x == 0) {
             b[0] = P->p;
             b[1] = TWO_PI_2_5 * P->K * P->invp;

@@ -269,10 +269,10 @@ struct ClassList {
     static constexpr int QLIST = QB + CLASS_BLOCK;   // batch + one screening step
 };
 
-// Least wavefronts per SIMD that the compiler plans the registers for.  The
-// row kernels wait more than they compute (at (H2O)16 cc-pVDZ the vector
-// units are busy 30% of the time), so a second or third wavefront pays where
-// it costs few spills: (pp|pp) 0.385 -> 0.284, (ds|pp) 0.451 -> 0.321, (ds|ds)
+// Least wavefronts per SIMD that the compiler plans the registers for, class
+// by class as measured.  The row kernels wait more than they compute (at
+// (H2O)16 cc-pVDZ the vector units are busy 30% of the time), so a second or
+// third wavefront can pay for the registers it spills: (pp|pp) 0.385 -> 0.284, (ds|pp) 0.451 -> 0.321, (ds|ds)
 // 0.332 -> 0.281 ms for two instead of one (2-15 registers spilled), (ps|ps)
 // 1.21 -> 1.10 ms for three instead of two (none).  (pp|ps), (dp|ss), (dp|ps)
 // and (dd|ss) were slower with more.

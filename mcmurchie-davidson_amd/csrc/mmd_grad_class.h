@@ -351,7 +351,7 @@ __global__ void __launch_bounds__(GRAD_BLOCK) grad_class_kernel(GradArgs A, Grad
 // primitives in turn (13.6 ms for the whole two-electron part with the
 // per-function kernel).
 template <int LA, int LB, int LC, int LD>
-struct GradWaveShape {
+struct GradBlockShape {
     static constexpr int LAB = LA + LB, LCD = LC + LD, L1 = LAB + LCD + 1, HL = nherm(L1);
     static constexpr int NAB = ncart(LA) * ncart(LB), NCD = ncart(LC) * ncart(LD);
     static constexpr int HAB = nherm(LAB), HCD = nherm(LCD);
@@ -390,9 +390,9 @@ __device__ inline void grad_tables(double a, double ap, double inv2p, double PA,
 }
 
 template <int LA, int LB, int LC, int LD>
-__global__ void __launch_bounds__(GRAD_BLOCK) grad_wave_kernel(GradArgs A, GradClass C)
+__global__ void __launch_bounds__(GRAD_BLOCK) grad_block_kernel(GradArgs A, GradClass C)
 {
-    using S = GradWaveShape<LA, LB, LC, LD>;
+    using S = GradBlockShape<LA, LB, LC, LD>;
     constexpr int NAB = S::NAB, NCD = S::NCD, HAB = S::HAB, HCD = S::HCD, HL = S::HL, L1 = S::L1;
     constexpr int NB = ncart(LB), ND = ncart(LD);
     constexpr int NTB = S::LAB + 1, NTK = S::LCD + 1;

@@ -160,7 +160,7 @@ __device__ void pair_rank(const PairInput& I, const PairWork& W, ShellPair* pair
     sp.same = pr.x == pr.y ? 1 : 0;
     sp.mol = a.mol;
     sp.c0 = I.mol_blocks ? I.mol_blocks[a.mol].x : 0;
-    sp.pad = 0;
+    sp.class_pp0 = 0;
     sp.q = q;
     pairs[s0 + rank] = sp;
     W.entry[s0 + rank] = e;
@@ -198,7 +198,7 @@ __device__ void pair_place(const PairInput& I, const int* scan, const int* sums,
     const int at = p0 - pair_start(scan, sums, I.off[c]);
     const int n = pairs[i].npp;
     pairs[i].pp0 = p0;
-    pairs[i].pad = at;
+    pairs[i].class_pp0 = at;
     // the first pair of a molecule holds its largest count
     if (i == I.off[c] + I.ranges[(size_t)c * I.nmol + pairs[i].mol].x) atomicMax(&stats->maxpp[c], n);
     if (i == I.off[c + 1] - 1) stats->total[c] = at + n;

@@ -15,7 +15,7 @@ struct ShellPair {
     int32_t same;        // sa == sb
     int32_t mol;         // molecule of the pair (a basis can hold several, block-diagonally)
     int32_t c0;          // first basis function of that molecule
-    int32_t pad;         // its first primitive pair's position among those of its pair class
+    int32_t class_pp0;   // its first primitive pair's position among those of its pair class
     double q;            // max over the pair's functions of sqrt((ab|ab))
 };
 
@@ -100,7 +100,6 @@ struct RowArgs {
     int boff, nb;               // bra pairs of the class: pairs[boff .. boff+nb)
     int koff, nk;               // ket pairs of the class
     int tri;                    // same pair class: ket index <= bra index
-    int seg;                    // ket pairs per work unit
     int rw;                     // width of the LDS rows: the largest molecule of the basis
     const int4* units;          // work units: {bra pair, first | end << 16 bra primitive pair, first ket, end ket}
     int nunits;
