@@ -1860,6 +1860,7 @@ int mmd_jk_tensor(mmd_ctx* ctx, const double* T, int t_on_device, const double* 
     }
     HIP_TRY(hipStreamSynchronize(ctx->st));
     dT.done();
+    stage.done();
     return MMD_OK;
 }
 
@@ -2487,6 +2488,7 @@ int mmd_ao2mo(mmd_ctx* ctx, const double* T, int t_on_device, const double* C, d
     HIP_TRY(hipStreamSynchronize(ctx->st));
     a.done();
     b.done();
+    stage.done();
     if (gemm_ms) {
         float ms = 0.f;
         HIP_TRY(hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));

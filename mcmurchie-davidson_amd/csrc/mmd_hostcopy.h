@@ -19,6 +19,11 @@ public:
     hipError_t to_host(void* dst, const void* src, size_t bytes, hipStream_t st);
     // Returns when src has been read; dst is complete for later work on st.
     hipError_t to_device(void* dst, const void* src, size_t bytes, hipStream_t st);
+    // The caller has waited for st since.
+    void done()
+    {
+        for (bool& b : busy) b = false;
+    }
 
 private:
     static constexpr int SLOTS = 6;

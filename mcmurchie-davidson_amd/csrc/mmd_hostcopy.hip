@@ -82,8 +82,8 @@ hipError_t HostStage::to_host(void* dst, const void* src, size_t bytes, hipStrea
     }
     hipError_t err = drain();
     if (err != hipSuccess) return err;
-    const int ns = nslots, half = (ns + 1) / 2;
     const int n = (int)((bytes + SLOT_BYTES - 1) / SLOT_BYTES);
+    const int ns = nslots, half = ns < n ? (ns + 1) / 2 : n;   // no slot is used twice where all chunks fit
     auto size_of = [&](int i) { return i + 1 < n ? SLOT_BYTES : bytes - (size_t)i * SLOT_BYTES; };
     const int64_t parts = (int64_t)((bytes + PART_BYTES - 1) / PART_BYTES);
     // bytes of a slot's chunks up to and including chunk i
@@ -142,8 +142,8 @@ hipError_t HostStage::to_device(void* dst, const void* src, size_t bytes, hipStr
         return hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, st);
     hipError_t err = drain();
     if (err != hipSuccess) return err;
-    const int ns = nslots, half = (ns + 1) / 2;
     const int n = (int)((bytes + SLOT_BYTES - 1) / SLOT_BYTES);
+    const int ns = nslots, half = ns < n ? (ns + 1) / 2 : n;   // no slot is used twice where all chunks fit
     auto size_of = [&](int i) { return i + 1 < n ? SLOT_BYTES : bytes - (size_t)i * SLOT_BYTES; };
     const int64_t parts = (int64_t)((bytes + PART_BYTES - 1) / PART_BYTES);
     auto through = [&](int i) { return (int64_t)(i / ns) * (int64_t)SLOT_BYTES + (int64_t)size_of(i); };
@@ -173,7 +173,7 @@ hipError_t HostStage::to_device(void* dst, const void* src, size_t bytes, hipStr
         if (err == hipSuccess) err = hipEventRecord(slot[s].ev, st);
         if (err == hipSuccess) busy[s] = true;
         const int back = i - (half - 1);   // half the slots in flight, half with the helpers
-        if (err == hipSuccess && back >= 0) {
+        if (err == hipSuccess && back >= 0 && back + ns < n) {
             err = hipEventSynchronize(slot[back % ns].ev);
             busy[back % ns] = false;
             freed.store(back + 1 + ns, std::memory_order_release);
