@@ -43,19 +43,19 @@ FP64_PEAK_TFLOPS = 78.6
 # counters read for a copy of known size (recorded with the command lines in
 # profiles/); a class absent here reports null.
 TRAFFIC = {
-    (0, 0, 0, 0): 1.952e+07, (1, 0, 0, 0): 3.600e+07, (1, 0, 1, 0): 4.309e+07, (1, 1, 0, 0): 1.616e+07,
-    (1, 1, 1, 0): 5.139e+07, (1, 1, 1, 1): 1.611e+07, (2, 0, 0, 0): 1.493e+07, (2, 0, 1, 0): 3.540e+07,
-    (2, 0, 1, 1): 1.892e+07, (2, 0, 2, 0): 9.296e+06, (2, 1, 0, 0): 1.075e+07, (2, 1, 1, 0): 1.506e+07,
-    (2, 1, 1, 1): 7.276e+06, (2, 1, 2, 0): 7.332e+06, (2, 1, 2, 1): 7.053e+06, (2, 2, 0, 0): 5.347e+06,
-    (2, 2, 1, 0): 7.271e+06, (2, 2, 1, 1): 5.876e+06, (2, 2, 2, 0): 4.760e+06, (2, 2, 2, 1): 9.041e+06,
-    (2, 2, 2, 2): 1.212e+06,
+    (0, 0, 0, 0): 1.952e+07, (1, 0, 0, 0): 3.593e+07, (1, 0, 1, 0): 4.307e+07, (1, 1, 0, 0): 1.612e+07,
+    (1, 1, 1, 0): 5.138e+07, (1, 1, 1, 1): 1.609e+07, (2, 0, 0, 0): 1.492e+07, (2, 0, 1, 0): 3.541e+07,
+    (2, 0, 1, 1): 2.083e+07, (2, 0, 2, 0): 9.272e+06, (2, 1, 0, 0): 1.078e+07, (2, 1, 1, 0): 1.505e+07,
+    (2, 1, 1, 1): 7.267e+06, (2, 1, 2, 0): 7.338e+06, (2, 1, 2, 1): 7.045e+06, (2, 2, 0, 0): 5.339e+06,
+    (2, 2, 1, 0): 7.265e+06, (2, 2, 1, 1): 5.863e+06, (2, 2, 2, 0): 4.766e+06, (2, 2, 2, 1): 3.505e+06,
+    (2, 2, 2, 2): 1.195e+06,
 }
 
 
 # The same for the dominant class kernel of the headline workload.
 TRAFFIC_HEADLINE = {
-    (0, 0, 0, 0): 6.223e+08, (1, 0, 0, 0): 4.914e+08, (1, 0, 1, 0): 2.694e+08, (1, 1, 0, 0): 1.652e+08,
-    (1, 1, 1, 0): 1.722e+08, (1, 1, 1, 1): 4.668e+07,
+    (0, 0, 0, 0): 5.743e+08, (1, 0, 0, 0): 4.618e+08, (1, 0, 1, 0): 2.574e+08, (1, 1, 0, 0): 1.647e+08,
+    (1, 1, 1, 0): 1.733e+08, (1, 1, 1, 1): 4.770e+07,
 }
 
 
