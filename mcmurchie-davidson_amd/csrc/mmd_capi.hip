@@ -238,9 +238,9 @@ struct mmd_ctx {
 
     // integral-block kernels: staged bra data per pair class (made from the
     // pair table on first use), copies of the raw G
-    DevBuf<double> d_btab, d_graw;
+    DevBuf<double> d_btab, d_graw, d_qraw;
     size_t btab_off[NPAIRCLASS] = {0};
-    bool btab_ok = false;
+    bool btab_ok = false, qraw_ok = false;
 
     // Molecules of a block-diagonal basis (mmd_set_molecules; one molecule
     // unless set): molecule m owns functions [mol_f0[m], mol_f0[m] + mol_n[m])
@@ -539,7 +539,7 @@ int build_pairs(mmd_ctx* c, const double* diag)
 {
     if (int rc = onee_pair_list(c)) return rc;
     c->grad_plan_ok = false;
-    c->btab_ok = false;
+    c->btab_ok = c->qraw_ok = false;
     c->pairs_ok = c->units_ok = false;
     for (int pc = 0; pc <= NPAIRCLASS; ++pc) c->pc_off[pc] = c->onee_off[pc];
     const size_t n = (size_t)c->pc_off[NPAIRCLASS];
@@ -1607,6 +1607,12 @@ int raw_fock_shells(mmd_ctx* c, bool complex_dP, double tol)
     const size_t nn = (size_t)c->nbf * c->nbf;
     HIP_TRY(launch_shell_block_max_raw((int)c->shells.size(), c->d_sh_bf0.p, c->d_sh_nbf.p, c->nbf, c->d_absD.p,
                                        c->d_Dsh.p, c->st));
+    if (!c->qraw_ok) {   // from the pair table and the Schwarz diagonal, which rebuilds it
+        const int n = c->pc_off[NPAIRCLASS];
+        HIP_TRY(c->d_qraw.reserve((size_t)n));
+        HIP_TRY(launch_pair_qraw(n, c->d_pairs.p, c->d_sh_nbf.p, c->nbf, c->d_sqS.p, c->d_qraw.p, c->st));
+        c->qraw_ok = true;
+    }
     // copies of G, so that the updates of a small matrix do not queue at the
     // same addresses; 128 MB of them at most
     const int nrep = (int)std::max<size_t>(1, std::min<size_t>(16, (size_t(8) << 20) / nn));
@@ -1624,6 +1630,7 @@ int raw_fock_shells(mmd_ctx* c, bool complex_dP, double tol)
     B.nrep = nrep;
     B.Dim = complex_dP ? c->d_Dim.p : nullptr;
     B.Dsh = c->d_Dsh.p;
+    B.qraw = c->d_qraw.p;
     B.nshell = (int)c->shells.size();
     if (int rc = run_block_classes(c, A, B)) return rc;
     HIP_TRY(launch_sum_copies((complex_dP ? 2 : 1) * nn, nrep, 2 * nn, c->d_graw.p, c->d_graw.p, c->st));

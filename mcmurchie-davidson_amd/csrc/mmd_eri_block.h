@@ -94,10 +94,13 @@ __device__ __forceinline__ void block_quartet(const BlockArgs& B, int64_t q, int
     }
 }
 
-// Shell-level form of raw_digest's test: q is the largest sqrt((ab|ab)) of a
-// pair and Dsh the largest |dP| of a shell block, so a quartet that fails it
-// has no component that passes the test above.
-__device__ __forceinline__ bool raw_keeps(const ClassArgs& A, const BlockArgs& B, const ShellPair& bra,
+// Shell-level form of raw_digest's test for the pairs P and Q: qraw is the
+// largest root of a pair's Schwarz values and Dsh the largest |dP| of a shell
+// block, infinity where a value is not a number (the test above keeps what
+// does not compare as small), so a quartet that fails it has no component that
+// passes.  A pair without primitive pairs has integrals that are zero to 1e-20,
+// and takes part only where |dP| is not finite.
+__device__ __forceinline__ bool raw_keeps(const ClassArgs& A, const BlockArgs& B, int P, int Q, const ShellPair& bra,
                                           const ShellPair& ket)
 {
     const size_t ns = (size_t)B.nshell;
@@ -105,7 +108,8 @@ __device__ __forceinline__ bool raw_keeps(const ClassArgs& A, const BlockArgs& B
     const double dm = fmax(fmax(fmax(4.0 * D[bra.sa * ns + bra.sb], 4.0 * D[ket.sa * ns + ket.sb]),
                                 fmax(D[bra.sa * ns + ket.sa], D[bra.sa * ns + ket.sb])),
                            fmax(D[bra.sb * ns + ket.sa], D[bra.sb * ns + ket.sb]));
-    return !(bra.q * ket.q * dm < A.tol);
+    if ((bra.npp == 0 || ket.npp == 0) && dm < HUGE_VAL) return false;
+    return !(B.qraw[P] * B.qraw[Q] * dm < A.tol);
 }
 
 template <int LA, int LB, int LC, int LD>
@@ -131,7 +135,7 @@ __global__ void __launch_bounds__(256) eri_block_kernel(ClassArgs A, BlockArgs B
         bool on = q < nq;
         if (on) block_quartet(B, q, P, Q);
         const ShellPair bra = A.pairs[P], ket = A.pairs[Q];
-        if (B.raw) on = on && bra.npp > 0 && ket.npp > 0 && raw_keeps(A, B, bra, ket);
+        if (B.raw) on = on && raw_keeps(A, B, P, Q, bra, ket);
         if (!__any(on)) continue;
         const int nb_ = on ? bra.npp : 0, nk_ = on ? ket.npp : 0;
         const int ip0 = nb_ * lib / gb, ip1 = nb_ * (lib + 1) / gb;

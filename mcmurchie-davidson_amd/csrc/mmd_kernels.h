@@ -54,6 +54,9 @@ hipError_t launch_bra_table(int pc, const ShellPair* pairs, const PrimPair* pp, 
 // that the screen keeps what meets it.
 hipError_t launch_shell_block_max_raw(int nshell, const int* sh_bf0, const int* sh_nbf, int N, const double* absD,
                                       double* Dsh, hipStream_t st);
+// The largest roots of the pairs' Schwarz values, for a raw build's screen.
+hipError_t launch_pair_qraw(int npairs, const ShellPair* pairs, const int* sh_nbf, int N, const double* sqS,
+                            double* qraw, hipStream_t st);
 // out (n elements; may be the first copy) = the sum of nrep copies `stride` apart
 hipError_t launch_sum_copies(size_t n, int nrep, size_t stride, const double* rep, double* out, hipStream_t st);
 // High angular-momentum classes whose two Hermite contractions run on the

@@ -132,6 +132,7 @@ struct BlockArgs {
     int raw, nrep;
     const double* Dim;          // raw: imaginary part of dP, or null
     const double* Dsh;          // raw: shell-block maxima of |dP|
+    const double* qraw;         // raw: per pair the largest square root of its Schwarz values
     int nshell;
 };
 

@@ -659,7 +659,7 @@ __global__ void __launch_bounds__(64 * GW_WAVES) eri_block_wave_kernel(ClassArgs
         block_quartet(B, q, qd.x, qd.y);
         const ShellPair bra = A.pairs[qd.x];
         const ShellPair ket = A.pairs[qd.y];
-        if (B.raw && !raw_keeps(A, B, bra, ket)) continue;   // uniform across the wavefront
+        if (B.raw && !raw_keeps(A, B, qd.x, qd.y, bra, ket)) continue;   // uniform across the wavefront
         double acc[NCPL];
         for (int i = 0; i < NCPL; ++i) acc[i] = 0.0;
         for (int ip = 0; ip < bra.npp; ++ip) {
@@ -876,6 +876,36 @@ hipError_t launch_shell_block_max_raw(int nshell, const int* sh_bf0, const int* 
     if (n <= 0) return hipSuccess;
     hipLaunchKernelGGL(shell_block_max_raw_kernel, dim3((n + 255) / 256), dim3(256), 0, st, nshell, sh_bf0, sh_nbf, N,
                        absD, Dsh);
+    return hipGetLastError();
+}
+
+// qraw of the shell pairs (BlockArgs): over a pair's functions the largest of
+// sqS in the order that the test of a function quartet reads, infinity where one
+// is not a number (a negative Schwarz value has no root).
+__global__ void pair_qraw_kernel(int npairs, const ShellPair* __restrict__ pairs, const int* __restrict__ nbf, int N,
+                                 const double* __restrict__ sqS, double* __restrict__ qraw)
+{
+    const int e = blockIdx.x * blockDim.x + threadIdx.x;
+    if (e >= npairs) return;
+    const ShellPair sp = pairs[e];
+    double m = 0.0;
+    bool nan = false;
+    for (int x = 0; x < nbf[sp.sa]; ++x)
+        for (int y = 0; y < nbf[sp.sb]; ++y) {
+            const int i = sp.bfa + x, j = sp.bfb + y;
+            const double v = sqS[(size_t)max(i, j) * N + min(i, j)];
+            nan = nan || v != v;
+            m = fmax(m, v);
+        }
+    qraw[e] = nan ? HUGE_VAL : m;
+}
+
+hipError_t launch_pair_qraw(int npairs, const ShellPair* pairs, const int* sh_nbf, int N, const double* sqS,
+                            double* qraw, hipStream_t st)
+{
+    if (npairs <= 0) return hipSuccess;
+    hipLaunchKernelGGL(pair_qraw_kernel, dim3((npairs + 255) / 256), dim3(256), 0, st, npairs, pairs, sh_nbf, N, sqS,
+                       qraw);
     return hipGetLastError();
 }
 
