@@ -43,19 +43,19 @@ FP64_PEAK_TFLOPS = 78.6
 # counters read for a copy of known size (recorded with the command lines in
 # profiles/); a class absent here reports null.
 TRAFFIC = {
-    (0, 0, 0, 0): 1.952e+07, (1, 0, 0, 0): 3.593e+07, (1, 0, 1, 0): 4.307e+07, (1, 1, 0, 0): 1.612e+07,
-    (1, 1, 1, 0): 5.138e+07, (1, 1, 1, 1): 1.609e+07, (2, 0, 0, 0): 1.492e+07, (2, 0, 1, 0): 3.541e+07,
-    (2, 0, 1, 1): 2.083e+07, (2, 0, 2, 0): 9.272e+06, (2, 1, 0, 0): 1.078e+07, (2, 1, 1, 0): 1.505e+07,
-    (2, 1, 1, 1): 7.267e+06, (2, 1, 2, 0): 7.338e+06, (2, 1, 2, 1): 7.045e+06, (2, 2, 0, 0): 5.339e+06,
-    (2, 2, 1, 0): 7.265e+06, (2, 2, 1, 1): 5.863e+06, (2, 2, 2, 0): 4.766e+06, (2, 2, 2, 1): 3.505e+06,
-    (2, 2, 2, 2): 1.195e+06,
+    (0, 0, 0, 0): 1.946e+07, (1, 0, 0, 0): 3.597e+07, (1, 0, 1, 0): 4.306e+07, (1, 1, 0, 0): 1.615e+07,
+    (1, 1, 1, 0): 5.137e+07, (1, 1, 1, 1): 1.611e+07, (2, 0, 0, 0): 1.491e+07, (2, 0, 1, 0): 3.539e+07,
+    (2, 0, 1, 1): 2.092e+07, (2, 0, 2, 0): 9.275e+06, (2, 1, 0, 0): 1.074e+07, (2, 1, 1, 0): 1.509e+07,
+    (2, 1, 1, 1): 7.263e+06, (2, 1, 2, 0): 7.348e+06, (2, 1, 2, 1): 7.041e+06, (2, 2, 0, 0): 5.339e+06,
+    (2, 2, 1, 0): 7.265e+06, (2, 2, 1, 1): 5.840e+06, (2, 2, 2, 0): 4.766e+06, (2, 2, 2, 1): 8.672e+06,
+    (2, 2, 2, 2): 1.196e+06,
 }
 
 
 # The same for the dominant class kernel of the headline workload.
 TRAFFIC_HEADLINE = {
-    (0, 0, 0, 0): 5.743e+08, (1, 0, 0, 0): 4.618e+08, (1, 0, 1, 0): 2.574e+08, (1, 1, 0, 0): 1.647e+08,
-    (1, 1, 1, 0): 1.733e+08, (1, 1, 1, 1): 4.770e+07,
+    (0, 0, 0, 0): 5.639e+08, (1, 0, 0, 0): 4.609e+08, (1, 0, 1, 0): 2.583e+08, (1, 1, 0, 0): 1.631e+08,
+    (1, 1, 1, 0): 1.751e+08, (1, 1, 1, 1): 4.769e+07,
 }
 
 
