@@ -52,6 +52,7 @@ int current_device()
 
 void free_slots(int n, const StageSlot* s)
 {
+    if (n == 0) return;
     std::lock_guard<std::recursive_mutex> lk(device_alloc_mutex());
     for (int i = 0; i < n; ++i) {
         if (s[i].ev) (void)hipEventDestroy(s[i].ev);
@@ -61,6 +62,7 @@ void free_slots(int n, const StageSlot* s)
 
 void free_buffers(int n, const Buffer* b)
 {
+    if (n == 0) return;   // nor wait for another thread's capture
     std::lock_guard<std::recursive_mutex> lk(device_alloc_mutex());
     for (int i = 0; i < n; ++i) (void)hipFree(b[i].p);
 }
