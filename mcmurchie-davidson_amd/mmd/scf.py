@@ -149,10 +149,17 @@ class SCF(object):
                 energy_old = self.energy
                 self.buildFock()
                 self.P_old = self.P
-                if DIIS:
+            extrapolated = False
+            if DIIS and step > 0:
+                try:
                     F_diis = _re(self.updateDIIS(self.F, self.P))
                     self.FO = np.dot(self.X.T, np.dot(F_diis, self.X))
-            if not DIIS or step == 0:
+                    extrapolated = True
+                except np.linalg.LinAlgError:
+                    # errors that vanish to the last bit (two electrons, near
+                    # convergence) leave nothing to extrapolate with
+                    pass
+            if not extrapolated:
                 self.orthoFock()
 
             with _blas_threads(getattr(self, "_eigh_threads", None)):

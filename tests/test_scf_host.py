@@ -125,6 +125,25 @@ def test_diis_singular_subspace_raises(cpu_molecule):
         mol.updateDIIS(F, P)
 
 
+def test_rhf_goes_on_without_extrapolation(cpu_molecule, oracle, monkeypatch):
+    """Singular DIIS equations in the middle of an SCF: steps without
+    extrapolation to the same energy (1e-10 in ||dP||: 1e-9 Eh)."""
+    from mmd.scf import SCF
+    mol, om = cpu_molecule(WATER, "sto-3g")
+    calls = []
+
+    def singular(self, F, P):
+        calls.append(0)
+        if len(calls) > 3:
+            raise np.linalg.LinAlgError("Singular matrix")
+        return update(self, F, P)
+    update = SCF.updateDIIS
+    monkeypatch.setattr(SCF, "updateDIIS", singular)
+    mol.RHF(doPrint=False, conver=1e-10)
+    assert len(calls) > 3 and mol.is_converged
+    assert abs(mol.energy.real - oracle.rhf(om, conver=1e-10)["energy"].real) < 1e-9
+
+
 # -- SAD initial guess ----------------------------------------------------------
 
 @pytest.fixture
